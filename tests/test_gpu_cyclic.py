@@ -173,3 +173,17 @@ def test_triangle_orientations(provider, monkeypatch, wcoj):
         assert st["iterations"] == 1 and st["delta_sizes"] == [len(want), 0]
     ss, sd = datagen.sparse_ids(s), datagen.sparse_ids(d)
     _parity(provider, "sparse triangles", cp.triangles_plan(), [pack(ss, sd), None], [1])
+
+
+@pytest.mark.parametrize("degree", [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 300])
+def test_triangle_run_lengths(provider, monkeypatch, degree):
+    """The generic join at the edges of its row groups (16 lanes a row, four rows at a time, 64 rows a wave) and of
+    its LDS stage (runs of 128 values): runs of `degree` values against short and long ones, on row counts that are
+    no multiple of 64."""
+    _wcoj(monkeypatch, "1")
+    rng = np.random.default_rng(degree)
+    n = 2 * degree + 60
+    rows = [(u, v) for u in range(3) for v in rng.choice(n, degree, replace=False)]
+    rows += [(u, v) for u in range(3, n) for v in rng.choice(n, int(rng.integers(1, 9)), replace=False)]
+    s, d = np.array(rows, dtype=np.uint32).T
+    _parity(provider, f"triangles degree {degree}", cp.triangles_plan(), [pack(s, d), None], [1])
