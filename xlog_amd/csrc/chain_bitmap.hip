@@ -1143,6 +1143,34 @@ void chain_fixpoint(Ctx *ctx, const std::vector<ChainRule> &rules, uint32_t n_pr
         if (r.path.size() == 1 && !r.path[0].backward) seed_e = r.path[0].pred;
     }
     const bool seed_cand = n_idb == 1 && rows[seed_h] == 0 && n_exit == 1 && seed_e >= 0 && rows[seed_e] > 0;
+    // with one recursive rule H(X,Z) :- F(X,Y), H(Y,Z) beside it, the columns of H are independent: each block of
+    // them runs to its fixpoint on chip
+    if (seed_cand && rules.size() == 2) {
+        const ChainRule &rec = idb[rules[0].path[0].pred] || rules[0].path.size() == 2 ? rules[0] : rules[1];
+        if (rec.path.size() == 2 && !idb[rec.path[0].pred] && !rec.path[0].backward && rec.path[1].pred == seed_h &&
+            !rec.path[1].backward && closure_columns_fits(domain, rows[rec.path[0].pred], rows[seed_e])) {
+            const int f = rec.path[0].pred;
+            Buf<uint64_t> row_ptr(ctx, (uint64_t)domain + 1), R(ctx, (uint64_t)domain * words), rc(ctx, (uint64_t)domain + 1);
+            Buf<uint32_t> adj(ctx, rows[f] ? rows[f] : 1);
+            pairs_csr(ctx, keys[f], rows[f], domain, row_ptr.p, adj.p);
+            std::vector<uint64_t> layers;
+            const uint64_t n = closure_columns(ctx, keys[f], rows[f], row_ptr.p, adj.p, keys[seed_e], rows[seed_e],
+                                               domain, words, max_iter, R.p, rc.p, layers);
+            uint64_t total = rows[seed_e];
+            deltas.push_back(total);
+            for (uint64_t v : layers) {
+                deltas.push_back(v);
+                total += v;
+            }
+            const bool converged = n < max_iter;
+            if (converged) deltas.push_back(0);
+            *iterations = deltas.size() - 1;
+            XH_REQUIRE(converged, XLOG_HIP_ITERATION_LIMIT,
+                       "Recursive SCC iteration limit (" + std::to_string(max_iter) + ") exceeded");
+            out_n[seed_h] = bitmap_emit(ctx, R.p, domain, words, &out[seed_h], XLOG_HIP_KERNEL_CHAIN_EMIT, total, rc.p);
+            return;
+        }
+    }
     run.setup(seed_cand);
     // (a head read backward or as R minus D also needs its transposes and P seeded: the general seed)
     const bool seed_rows =

@@ -659,8 +659,9 @@ void pairs_csr(Ctx *ctx, const uint64_t *pairs, uint64_t m, uint32_t nv, uint64_
 // Set bits of an nv x words bitmap as sorted packed (x << 32) | z rows in a
 // new pool buffer *out; returns the row count.
 // known_total: the number of set bits when the caller knows it (no read-back), else UINT64_MAX
+// row_counts: each row's bits in nv + 1 entries when the caller has them (scanned in place), else null
 uint64_t bitmap_emit(Ctx *ctx, const uint64_t *bits, uint32_t nv, uint64_t words, uint64_t **out, int prof_kind,
-                     uint64_t known_total = UINT64_MAX);
+                     uint64_t known_total = UINT64_MAX, uint64_t *row_counts = nullptr);
 
 // Dense-domain fixpoint of a program whose rules are chains of binary
 // relations: rule r derives head(v0, vk) from path[0](v0, v1), ...,
@@ -678,6 +679,20 @@ void chain_fixpoint(Ctx *ctx, const std::vector<ChainRule> &rules, uint32_t n_pr
                     uint64_t *iterations, std::vector<uint64_t> &deltas);
 // Bytes of device memory chain_fixpoint keeps for its bitmaps.
 uint64_t chain_fixpoint_bytes(const std::vector<ChainRule> &rules, const std::vector<char> &idb, uint32_t domain);
+
+// The bits of H(X,Z) :- E(X,Z).  H(X,Z) :- F(X,Y), H(Y,Z)  over a dense domain
+// (closure_columns.hip): F as m sorted unique packed pairs and their CSR
+// (row_ptr, adj), E as n_seed sorted unique packed pairs (seed == edge when E
+// is F), the result as a domain x words bit matrix R (written whole) and the number
+// of bits in each of its rows.  layers
+// receives the new tuples of each iteration after the seed, up to the last
+// non-empty one or max_iter of them; returns their number.
+// closure_columns_fits: the domains and relation sizes it takes.
+constexpr uint64_t CLOSURE_COLUMNS_EDGES = 1ull << 21;
+bool closure_columns_fits(uint32_t domain, uint64_t edges, uint64_t seeds);
+uint64_t closure_columns(Ctx *ctx, const uint64_t *edge, uint64_t m, const uint64_t *row_ptr, const uint32_t *adj,
+                         const uint64_t *seed, uint64_t n_seed, uint32_t domain, uint64_t words, uint64_t max_iter,
+                         uint64_t *R, uint64_t *row_counts, std::vector<uint64_t> &layers);
 
 // Arrow IPC stream codec for relations of 1..4 UInt32 columns (arrow_ipc.cpp,
 // host code).  decode checks the stream and returns pointers to the column

@@ -353,16 +353,19 @@ void pairs_csr(Ctx *ctx, const uint64_t *pairs, uint64_t m, uint32_t nv, uint64_
 // (row counts, a scan, then one block per row writing at its offset; rows
 // of EMIT_STAGED_ROW tuples or more on average are staged in LDS).
 uint64_t bitmap_emit(Ctx *ctx, const uint64_t *bits, uint32_t nv, uint64_t words, uint64_t **out, int prof_kind,
-                     uint64_t known_total) {
+                     uint64_t known_total, uint64_t *row_counts) {
     *out = nullptr;
     if (nv == 0 || known_total == 0) return 0;
-    Buf<uint64_t> rc(ctx, (uint64_t)nv + 1);
-    hipLaunchKernelGGL(k_row_counts, dim3(nv), dim3(TB), 0, ctx->stream, bits, words, rc.p);
-    XH_CHECK_HIP(hipGetLastError());
-    scan_u64_inplace(ctx, rc.p, nv, rc.p + nv);
+    Buf<uint64_t> own(ctx, row_counts ? 0 : (uint64_t)nv + 1);
+    uint64_t *rc = row_counts ? row_counts : own.p;
+    if (!row_counts) {
+        hipLaunchKernelGGL(k_row_counts, dim3(nv), dim3(TB), 0, ctx->stream, bits, words, rc);
+        XH_CHECK_HIP(hipGetLastError());
+    }
+    scan_u64_inplace(ctx, rc, nv, rc + nv);
     uint64_t total = known_total;
     if (total == UINT64_MAX) {
-        ctx->read_scalars(rc.p + nv, 1);
+        ctx->read_scalars(rc + nv, 1);
         total = ctx->host_scalars[0];
     }
     if (total == 0) return 0;
@@ -372,9 +375,9 @@ uint64_t bitmap_emit(Ctx *ctx, const uint64_t *bits, uint32_t nv, uint64_t words
     uint64_t staged_row = EMIT_STAGED_ROW;
     if (const char *e = getenv("XLOG_HIP_EMIT_STAGED_ROW")) staged_row = strtoull(e, nullptr, 10);
     if (total >= staged_row * nv)
-        hipLaunchKernelGGL(k_emit_rows, dim3(nv), dim3(EMIT_TB), 0, ctx->stream, bits, words, rc.p, *out, total);
+        hipLaunchKernelGGL(k_emit_rows, dim3(nv), dim3(EMIT_TB), 0, ctx->stream, bits, words, rc, *out, total);
     else
-        hipLaunchKernelGGL(k_emit_rows_direct, dim3(nv), dim3(TB), 0, ctx->stream, bits, words, rc.p, *out, total);
+        hipLaunchKernelGGL(k_emit_rows_direct, dim3(nv), dim3(TB), 0, ctx->stream, bits, words, rc, *out, total);
     XH_CHECK_HIP(hipGetLastError());
     return total;
 }
