@@ -1,0 +1,48 @@
+"""GPU parity of the one-workgroup sort (up to 16,384 keys) against numpy: its wave, round and size edges, keys whose
+bins are short (hashed, dense ids) and long (hubs, few values: the digit passes in LDS), and the stable sort by one
+column that a join's build side takes."""
+import numpy as np
+import pytest
+
+from xlog_amd import pack
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [1, 2, 3, 63, 64, 65, 1023, 1024, 1025, 4097, 16383, 16384, 16385]
+
+
+def _keys(kind, n, rng):
+    if kind == "hashed":
+        return rng.integers(0, 1 << 64, n, dtype=np.uint64)
+    if kind == "dense":
+        return pack(rng.integers(0, 1000, n), rng.integers(0, 700, n))
+    if kind == "hub":
+        return pack(np.where(rng.random(n) < 0.6, 7, rng.integers(0, 1 << 32, n)), rng.integers(0, 3000, n))
+    if kind == "few":
+        return rng.choice(np.array([0, 1, (1 << 64) - 1, 1 << 63], dtype=np.uint64), n)
+    return np.full(n, 0xFFFFFFFF00000000, dtype=np.uint64)  # equal
+
+
+@pytest.mark.parametrize("kind", ["hashed", "dense", "hub", "few", "equal"])
+def test_sort_and_dedup(provider, kind):
+    for n in SIZES:
+        k = _keys(kind, n, np.random.default_rng(n))
+        R = provider.create_buffer_from_packed(k)
+        assert np.array_equal(provider.download_packed(provider.sort(R, [0, 1])), np.sort(k)), n
+        d = provider.dedup_full_row(R)
+        assert np.array_equal(provider.download_packed(d), np.unique(k)), n
+        assert d.is_canonical()
+        assert np.array_equal(provider.download_packed(R), k), n  # the input is left as it is
+
+
+@pytest.mark.parametrize("kind", ["hashed", "dense", "hub", "few", "equal"])
+@pytest.mark.parametrize("n", [1, 65, 1025, 16384])
+def test_stable_by_column(provider, kind, n):
+    """The rows of a run of equal join keys come in input order."""
+    k = _keys(kind, n, np.random.default_rng(n))
+    col = (k >> np.uint64(32)).astype(np.uint32)
+    some = np.unique(col)[:8]
+    out = provider.hash_join_v2(provider.create_buffer_from_u32_columns([some]),
+                                provider.create_buffer_from_u32_columns([col, np.arange(n, dtype=np.uint32)]), [0], [0])
+    want = np.concatenate([np.nonzero(col == v)[0] for v in some])
+    assert np.array_equal(provider.download_column(out, 2), want.astype(np.uint32))

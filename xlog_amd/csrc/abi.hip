@@ -433,6 +433,13 @@ static uint64_t unique_keys(Ctx *ctx, const uint64_t *sorted, uint64_t n, uint64
 // known_digits: the digits the keys may vary in (0: unknown, the histograms decide)
 void sort_unique_keys_async(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t **out, uint64_t *d_count,
                             uint32_t known_digits) {
+    if (n && n <= BLOCK_SORT_KEYS) {
+        Owned o(ctx, alloc_keys(ctx, n));
+        if (block_sort_unique(ctx, keys, n, o.p, d_count)) {
+            *out = o.release();
+            return;
+        }
+    }
     if (n >= 2 && n < (1ull << 30)) {
         Owned ga(ctx, alloc_keys(ctx, n)), gb(ctx, alloc_keys(ctx, n));
         uint64_t *a = ga.p, *b = gb.p;

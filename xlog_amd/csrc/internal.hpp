@@ -308,6 +308,12 @@ struct SortUnique {
     bool done = false;
     uint64_t count = 0;
 };
+// Keys-only sorts of at most BLOCK_SORT_KEYS keys run in one workgroup (one
+// launch, no read-back).  block_sort_unique: the sorted unique keys of such an
+// input to out (n entries) and their number to *d_count (device); false (and
+// nothing done) for a larger or empty one.
+constexpr uint64_t BLOCK_SORT_KEYS = 1ull << 14;
+bool block_sort_unique(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *out, uint64_t *d_count);
 // XLOG_HIP_SORT_TICKETS=1 (read at each sort): the radix pass and the
 // short-run unique order their tiles by an atomic start ticket instead of the
 // workgroup index, so that their look-back does not rest on workgroups

@@ -180,6 +180,224 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int lane) {
     return v;
 }
 
+// A sort of at most BLOCK_SORT_KEYS keys: one workgroup, one launch, the keys
+// in LDS.  Launches and their gaps bound a sort of this size (5,003 random
+// pairs by digit passes: a histogram, an offset and eight one-tile passes of 9
+// us each, 0.090 ms in all; here 0.010; a dedup with its read-back 0.112 ->
+// 0.026 ms, 16,384 pairs 0.136 -> 0.039).  Whole keys are binned by the top 12 of
+// the bits that vary (the high word's varying bits above the low word's, so
+// that ids of a small domain fill the bins) with LDS atomics, and each key is
+// ranked in its bin by the whole key; equal keys are indistinguishable, so the
+// bins' order by arrival does not show.  Bins that are long on average
+// (BLOCK_SORT_BIN keys: hub ids) and sorts by a part of the key, which have to
+// be stable, take digit passes in LDS instead, over the digits that vary.
+enum { BS_SORT, BS_UNIQUE, BS_DIGITS };
+constexpr int BS_TB = 1024, BS_ITEMS = 16, BS_BINS = 4096;
+constexpr uint32_t BLOCK_SORT_BIN = 64;
+static_assert(BS_TB * BS_ITEMS == BLOCK_SORT_KEYS, "keys of one workgroup");
+template <int MODE>
+__global__ __launch_bounds__(BS_TB) void k_block_sort(const uint64_t *in, uint32_t n, uint64_t *out, uint64_t window,
+                                                      uint64_t *d_count) {
+    constexpr int WAVES = BS_TB / WAVE;
+    __shared__ uint64_t s_key[BS_TB * BS_ITEMS];
+    __shared__ uint32_t s_bin[BS_BINS];  // bins; the digit passes' [WAVES][256] counts; the unique's counts
+    __shared__ uint32_t s_part[WAVES], s_part2[WAVES];
+    static_assert(WAVES * 256 == BS_BINS && BS_ITEMS * WAVES <= BS_BINS, "shared arrays");
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid >> 6;
+    const uint32_t rounds = (n + BS_TB - 1) / BS_TB;
+    auto block_or = [&](uint32_t v, uint32_t *part) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v |= (uint32_t)__shfl_xor((int)v, o, WAVE);
+        if (lane == 0) part[wave] = v;
+    };
+    // exclusive prefix of one value per thread
+    auto block_scan = [&](uint32_t v) {
+        const uint32_t x = wave_incl_scan(v, lane);
+        if (lane == WAVE - 1) s_part[wave] = x;
+        __syncthreads();
+        uint32_t pre = 0;
+        for (int w = 0; w < wave; ++w) pre += s_part[w];
+        return pre + x - v;
+    };
+    // the wave's keys are consecutive (wave * rounds * 64 + r * 64 + lane), as the stable passes need them
+    const uint32_t base = (uint32_t)wave * rounds * WAVE + lane;
+    uint64_t k[BS_ITEMS];
+    const uint64_t k0 = in[0];
+    uint64_t vary = 0;
+#pragma unroll
+    for (int r = 0; r < BS_ITEMS; ++r) {
+        const uint32_t i = base + r * WAVE;
+        const bool live = (uint32_t)r < rounds && i < n;
+        k[r] = live ? in[i] : k0;
+        vary |= k[r] ^ k0;
+    }
+    block_or((uint32_t)vary, s_part);
+    block_or((uint32_t)(vary >> 32), s_part2);
+#pragma unroll
+    for (int q = 0; q < BS_BINS / BS_TB; ++q) s_bin[q * BS_TB + tid] = 0;
+    __syncthreads();
+    uint32_t vlo = 0, vhi = 0;
+    for (int w = 0; w < WAVES; ++w) {
+        vlo |= s_part[w];
+        vhi |= s_part2[w];
+    }
+    vary = (((uint64_t)vhi << 32) | vlo) & window;
+    bool sorted = false;
+    if (MODE != BS_DIGITS && vary) {
+        const int nlo = vlo ? 32 - __clz((int)vlo) : 0, nhi = vhi ? 32 - __clz((int)vhi) : 0;
+        const int shift = nlo + nhi > 12 ? nlo + nhi - 12 : 0;
+        const uint64_t mlo = (1ull << nlo) - 1, mhi = (1ull << nhi) - 1;
+        auto bin_of = [&](uint64_t x) { return (uint32_t)(((((x >> 32) & mhi) << nlo) | (x & mlo)) >> shift); };
+        uint32_t slot[BS_ITEMS];
+#pragma unroll
+        for (int r = 0; r < BS_ITEMS; ++r) {
+            const uint32_t i = base + r * WAVE;
+            slot[r] = (uint32_t)r < rounds && i < n ? atomicAdd(&s_bin[bin_of(k[r])], 1u) : 0u;
+        }
+        __syncthreads();
+        uint32_t c[BS_BINS / BS_TB], tot = 0, sq = 0;
+#pragma unroll
+        for (int q = 0; q < BS_BINS / BS_TB; ++q) {
+            c[q] = s_bin[tid * (BS_BINS / BS_TB) + q];
+            tot += c[q];
+            sq += c[q] * c[q];  // (at most 2^28 over all bins)
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sq += (uint32_t)__shfl_xor((int)sq, o, WAVE);
+        if (lane == 0) s_part2[wave] = sq;
+        uint32_t pre = block_scan(tot);  // (its barrier also publishes s_part2)
+        uint32_t sum = 0;
+        for (int w = 0; w < WAVES; ++w) sum += s_part2[w];
+        __syncthreads();
+        sorted = sum <= BLOCK_SORT_BIN * n;  // block-uniform
+        if (sorted) {
+#pragma unroll
+            for (int q = 0; q < BS_BINS / BS_TB; ++q) {
+                s_bin[tid * (BS_BINS / BS_TB) + q] = pre;
+                pre += c[q];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < BS_ITEMS; ++r) {
+                const uint32_t i = base + r * WAVE;
+                if ((uint32_t)r < rounds && i < n) s_key[s_bin[bin_of(k[r])] + slot[r]] = k[r];
+            }
+            __syncthreads();
+            uint32_t to[BS_ITEMS];
+#pragma unroll
+            for (int r = 0; r < BS_ITEMS; ++r) {
+                const uint32_t i = base + r * WAVE;
+                to[r] = 0;
+                if ((uint32_t)r < rounds && i < n) {
+                    k[r] = s_key[i];
+                    const uint32_t b = bin_of(k[r]);
+                    const uint32_t lo = s_bin[b], hi = b + 1 < BS_BINS ? s_bin[b + 1] : n;
+                    uint32_t rank = lo;
+                    for (uint32_t j = lo; j < hi; ++j) {
+                        const uint64_t x = s_key[j];
+                        rank += (x < k[r] || (x == k[r] && j < i)) ? 1u : 0u;
+                    }
+                    to[r] = rank;
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < BS_ITEMS; ++r) {
+                const uint32_t i = base + r * WAVE;
+                if ((uint32_t)r < rounds && i < n) s_key[to[r]] = k[r];
+            }
+            __syncthreads();
+        }
+    }
+    if (!sorted) {
+        for (int dgt = 0; dgt < 8; ++dgt) {
+            if (!((vary >> (8 * dgt)) & 255u)) continue;  // block-uniform
+            for (int q = 0; q < BS_BINS / BS_TB; ++q) s_bin[q * BS_TB + tid] = 0;
+            __syncthreads();
+            uint32_t *wcnt = s_bin + wave * 256;
+            uint32_t rank[BS_ITEMS];
+#pragma unroll
+            for (int r = 0; r < BS_ITEMS; ++r) {
+                rank[r] = 0;
+                if ((uint32_t)r >= rounds) continue;  // block-uniform
+                const uint32_t i = base + r * WAVE;
+                const uint32_t dg = (uint32_t)(k[r] >> (8 * dgt)) & 255u;
+                uint64_t peers = __ballot(i < n);
+#pragma unroll
+                for (int b = 0; b < 8; ++b) {
+                    const uint64_t m = __ballot((dg >> b) & 1u);
+                    peers &= ((dg >> b) & 1u) ? m : ~m;
+                }
+                const uint32_t below = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
+                // every peer reads the running count before the group's first lane bumps it (one wave's LDS
+                // operations complete in order)
+                const uint32_t old = wcnt[dg];
+                if (i < n && below == 0) wcnt[dg] = old + (uint32_t)__popcll(peers);
+                rank[r] = old + below;
+            }
+            __syncthreads();
+            uint32_t cnt = 0;
+            if (tid < 256)
+                for (int w = 0; w < WAVES; ++w) {
+                    const uint32_t c = s_bin[w * 256 + tid];
+                    s_bin[w * 256 + tid] = cnt;
+                    cnt += c;
+                }
+            const uint32_t start = block_scan(tid < 256 ? cnt : 0u);
+            if (tid < 256)
+                for (int w = 0; w < WAVES; ++w) s_bin[w * 256 + tid] += start;
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < BS_ITEMS; ++r) {
+                const uint32_t i = base + r * WAVE;
+                if ((uint32_t)r < rounds && i < n) s_key[wcnt[(uint32_t)(k[r] >> (8 * dgt)) & 255u] + rank[r]] = k[r];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < BS_ITEMS; ++r) {
+                const uint32_t i = base + r * WAVE;
+                if ((uint32_t)r < rounds && i < n) k[r] = s_key[i];
+            }
+        }
+        if (!vary) {  // nothing to order
+#pragma unroll
+            for (int r = 0; r < BS_ITEMS; ++r) {
+                const uint32_t i = base + r * WAVE;
+                if ((uint32_t)r < rounds && i < n) s_key[i] = k[r];
+            }
+        }
+        __syncthreads();
+    }
+    if (MODE != BS_UNIQUE) {
+        for (uint32_t i = tid; i < n; i += BS_TB) out[i] = s_key[i];
+        return;
+    }
+    // the keys that differ from the one before, in order: counts per (wave, round), their prefix, the write
+    uint64_t bal[BS_ITEMS];
+    uint32_t mine = 0;
+#pragma unroll
+    for (int r = 0; r < BS_ITEMS; ++r) {
+        const uint32_t i = base + r * WAVE;
+        k[r] = (uint32_t)r < rounds && i < n ? s_key[i] : 0ull;
+        const bool keep = (uint32_t)r < rounds && i < n && (i == 0 || s_key[i - 1] != k[r]);
+        bal[r] = __ballot(keep);
+        mine += (uint32_t)__popcll(bal[r]);
+    }
+    if (lane == 0) s_part2[wave] = mine;
+    __syncthreads();
+    uint32_t pos = 0, total = 0;
+    for (int w = 0; w < WAVES; ++w) {
+        if (w < wave) pos += s_part2[w];
+        total += s_part2[w];
+    }
+#pragma unroll
+    for (int r = 0; r < BS_ITEMS; ++r) {
+        if ((bal[r] >> lane) & 1ull) out[pos + (uint32_t)__popcll(bal[r] & ((1ull << lane) - 1ull))] = k[r];
+        pos += (uint32_t)__popcll(bal[r]);
+    }
+    if (tid == 0) *d_count = total;
+}
+
 // Tile order of the digit passes.  Consecutive tiles write adjacent pieces of
 // every digit run, so their partial cache lines merge only when they run under
 // one L2.  Workgroups are dispatched in index order, round-robin over the 8
@@ -773,6 +991,19 @@ int radix_sort_dev(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n_bo
     return passes;
 }
 
+// A tile order or wait asked for by name (XLOG_HIP_SORT_TICKETS, _PERSIST,
+// _SPIN) asks for the digit passes, whatever the size.
+static bool sort_block() {
+    return !getenv("XLOG_HIP_SORT_TICKETS") && !getenv("XLOG_HIP_SORT_PERSIST") && !getenv("XLOG_HIP_SORT_SPIN");
+}
+bool block_sort_unique(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *out, uint64_t *d_count) {
+    if (n == 0 || n > BLOCK_SORT_KEYS || !sort_block()) return false;
+    Prof prof(ctx, XLOG_HIP_KERNEL_SORT_PASS, 16.0 * (double)n);
+    hipLaunchKernelGGL(k_block_sort<BS_UNIQUE>, dim3(1), dim3(BS_TB), 0, ctx->stream, keys, (uint32_t)n, out, ~0ull,
+                       d_count);
+    XH_CHECK_HIP(hipGetLastError());
+    return true;
+}
 int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **vals, uint32_t **vals_alt,
                    uint64_t n, int digit_lo, int digit_hi, const uint64_t *src, uint32_t known_digits,
                    SortUnique *uq, bool *whole) {
@@ -785,6 +1016,18 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **va
     XH_REQUIRE(n < (1ull << 30), XLOG_HIP_CAPACITY_OVERFLOW,
                "radix sort: a single sort call is limited to 2^30 - 1 keys");
     const bool has_val = vals && *vals;
+    if (!has_val && n <= BLOCK_SORT_KEYS && sort_block()) {
+        const uint64_t *from = src ? src : *keys;
+        Prof prof(ctx, XLOG_HIP_KERNEL_SORT_PASS, 16.0 * (double)n);
+        if (digit_lo == 0 && digit_hi == 8)
+            hipLaunchKernelGGL(k_block_sort<BS_SORT>, dim3(1), dim3(BS_TB), 0, ctx->stream, from, (uint32_t)n, *keys,
+                               ~0ull, nullptr);
+        else
+            hipLaunchKernelGGL(k_block_sort<BS_DIGITS>, dim3(1), dim3(BS_TB), 0, ctx->stream, from, (uint32_t)n, *keys,
+                               (~0ull >> (64 - 8 * digit_hi)) & ~((1ull << (8 * digit_lo)) - 1ull), nullptr);
+        XH_CHECK_HIP(hipGetLastError());
+        return 1;
+    }
     const uint64_t tile_keys = has_val ? (uint64_t)SORT_BLOCK_V * SORT_ITEMS_V : (uint64_t)SORT_BLOCK_K * SORT_ITEMS_K;
     const uint64_t tiles = (n + tile_keys - 1) / tile_keys;
     SortState &st = sort_state(ctx, tiles);
