@@ -105,10 +105,34 @@ Pool::~Pool() {
     for (auto &kv : live_) (void)hipFree(kv.first);
 }
 
-void Ctx::read_scalars(const void *dev, size_t count_u64) {
-    XH_REQUIRE(count_u64 <= HOST_STAGE_U64, XLOG_HIP_INVALID_ARG, "read_scalars: more than the pinned staging holds");
-    XH_CHECK_HIP(hipMemcpyAsync(host_scalars, dev, count_u64 * sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
-    sync();
+namespace {
+__global__ __launch_bounds__(256) void k_read_back(const uint64_t *__restrict__ src, uint32_t n, uint64_t *dst,
+                                                   uint64_t *seq, uint64_t v) {
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+    __threadfence_system();  // the words reach the host before the number does
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(seq, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+}  // namespace
+void Ctx::post_read(const void *dev, size_t count_u64) {
+    XH_REQUIRE(count_u64 <= HOST_STAGE_U64, XLOG_HIP_INVALID_ARG, "read-back: more than the pinned staging holds");
+    hipLaunchKernelGGL(k_read_back, dim3(1), dim3(count_u64 > 64 ? 256 : 64), 0, stream,
+                       static_cast<const uint64_t *>(dev), (uint32_t)count_u64, host_scalars, host_seq, ++read_seq);
+    XH_CHECK_HIP(hipGetLastError());
+}
+void Ctx::wait_read() {
+    ++host_waits;
+    for (uint64_t spins = 1; __atomic_load_n(host_seq, __ATOMIC_ACQUIRE) != read_seq; ++spins) {
+        __builtin_ia32_pause();
+        if (spins % 4096) continue;
+        // (now and then: a device error, or a stream that is done and has not stored the number)
+        const hipError_t e = hipStreamQuery(stream);
+        if (e == hipErrorNotReady) continue;
+        XH_CHECK_HIP(e);
+        XH_CHECK_HIP(hipStreamSynchronize(stream));
+        XH_REQUIRE(__atomic_load_n(host_seq, __ATOMIC_ACQUIRE) == read_seq, XLOG_HIP_DEVICE_ERROR,
+                   "read-back did not arrive");
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1126,13 +1150,11 @@ static xlog_hip_rel *op_join_keys(Ctx *ctx, const xlog_hip_rel *l, const xlog_hi
 
 static bool column_sorted(Ctx *ctx, const xlog_hip_rel *rel, uint32_t col) {
     if (rel->rows < 2) return true;
-    Buf<uint32_t> flag(ctx, 1);
-    fill_u32(ctx, flag.p, 0u, 1);
+    Buf<uint32_t> flag(ctx, 2);
+    fill_u32(ctx, flag.p, 0u, 2);
     LAUNCH_1D(k_col_unsorted, rel->rows, view_of(rel), (int)col, rel->rows, flag.p);
-    uint32_t h = 0;
-    XH_CHECK_HIP(hipMemcpyAsync(&h, flag.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-    ctx->sync();
-    return h == 0;
+    ctx->read_scalars(flag.p, 1);
+    return ctx->host_scalars[0] == 0;
 }
 
 // Sort-merge inner join (reference sort_merge_join_v2_inner_u32_1key,
@@ -1514,9 +1536,7 @@ static xlog_hip_rel *op_join_project_dedup(Ctx *ctx, const xlog_hip_rel *l, cons
         side.payload = J.payload.p;
         probe_count_only(ctx, side);
         probe_scan_async(ctx, side);
-        XH_CHECK_HIP(hipMemcpyAsync(ctx->host_scalars, side.toff.p + side.tiles, sizeof(uint64_t),
-                                    hipMemcpyDeviceToHost, ctx->stream));
-        XH_CHECK_HIP(hipEventRecord(ctx->ev_read, ctx->stream));
+        ctx->post_read(side.toff.p + side.tiles, 1);
     }
     ProbeJob job;
     job.probe = lkeys;
@@ -1532,7 +1552,7 @@ static xlog_hip_rel *op_join_project_dedup(Ctx *ctx, const xlog_hip_rel *l, cons
     Buf<unsigned long long> mx(ctx, 1);
     uint64_t m2 = 0;
     if (nm) {
-        ctx->wait_event(ctx->ev_read);
+        ctx->wait_read();
         m2 = ctx->host_scalars[0];
         probe_finish(side, nm, m2);
         gseg = Buf<uint64_t>(ctx, 2 * nh);
@@ -1704,15 +1724,17 @@ xlog_hip_status xlog_hip_ctx_create(int device, xlog_hip_ctx **out) {
         c.num_cus = prop.multiProcessorCount;
         XH_CHECK_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
         c.pool = new Pool(device);
-        XH_CHECK_HIP(hipHostMalloc((void **)&c.host_scalars, Ctx::HOST_STAGE_U64 * sizeof(uint64_t),
-                                   hipHostMallocDefault));
+        // (coherent: a kernel's stores are seen by the host while it waits; the word after the staging is host_seq)
+        XH_CHECK_HIP(hipHostMalloc((void **)&c.host_scalars, (Ctx::HOST_STAGE_U64 + 8) * sizeof(uint64_t),
+                                   hipHostMallocCoherent));
+        c.host_seq = c.host_scalars + Ctx::HOST_STAGE_U64;
+        *c.host_seq = 0;
         scan_noalloc_init(device);  // the allocation-free scan's scratch on this device
         c.tickets = static_cast<unsigned long long *>(c.alloc(16 * sizeof(unsigned long long)));
         fill_u64(&c, reinterpret_cast<uint64_t *>(c.tickets), 0ull, 16);
         XH_CHECK_HIP(hipEventCreate(&c.ev_a));
         XH_CHECK_HIP(hipEventCreate(&c.ev_b));
         XH_CHECK_HIP(hipEventCreateWithFlags(&c.ev_sync, hipEventDisableTiming));
-        XH_CHECK_HIP(hipEventCreateWithFlags(&c.ev_read, hipEventDisableTiming));
         c.sync();
         *out = h.release();
     });
@@ -1732,7 +1754,6 @@ void xlog_hip_ctx_destroy(xlog_hip_ctx *ctx) {
     if (c.ev_a) (void)hipEventDestroy(c.ev_a);
     if (c.ev_b) (void)hipEventDestroy(c.ev_b);
     if (c.ev_sync) (void)hipEventDestroy(c.ev_sync);
-    if (c.ev_read) (void)hipEventDestroy(c.ev_read);
     for (auto &r : c.prof_pending) {
         (void)hipEventDestroy(r.a);
         (void)hipEventDestroy(r.b);

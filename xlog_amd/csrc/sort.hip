@@ -1124,11 +1124,10 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **va
     // waits instead, since its histograms may choose the high-word route.
     uint32_t h_hist[8 * 256];
     static_assert(sizeof(h_hist) <= Ctx::HOST_STAGE_U64 * sizeof(uint64_t), "histograms exceed the staging");
-    XH_CHECK_HIP(hipMemcpyAsync(ctx->host_scalars, hist, sizeof(h_hist), hipMemcpyDeviceToHost, ctx->stream));
-    XH_CHECK_HIP(hipEventRecord(ctx->ev_read, ctx->stream));
+    ctx->post_read(hist, sizeof(h_hist) / 8);
     int first = digit_lo;
     if (digit_hi - digit_lo >= 2 && !hybrid_candidate && !word_candidate) launch_pass(first++);
-    ctx->wait_event(ctx->ev_read);
+    ctx->wait_read();
     memcpy(h_hist, ctx->host_scalars, sizeof(h_hist));
     auto trivial = [&](int dgt) {
         for (int b = 0; b < 256; ++b)
@@ -1138,9 +1137,7 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **va
     // the low word's histograms (their counters are still zero) from the same multiset of keys, and back
     auto low_word_histograms = [&](const uint64_t *from) {
         histograms(from, 0, 4);
-        XH_CHECK_HIP(hipMemcpyAsync(ctx->host_scalars, hist, sizeof(h_hist), hipMemcpyDeviceToHost, ctx->stream));
-        XH_CHECK_HIP(hipEventRecord(ctx->ev_read, ctx->stream));
-        ctx->wait_event(ctx->ev_read);
+        ctx->read_scalars(hist, sizeof(h_hist) / 8);
         memcpy(h_hist, ctx->host_scalars, sizeof(h_hist));
     };
     int gshift = 0;
