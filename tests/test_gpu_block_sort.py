@@ -1,4 +1,4 @@
-"""GPU parity of the one-workgroup sort (up to 16,384 keys) against numpy: its wave, round and size edges, keys whose
+"""GPU parity of the one-workgroup sort (up to 16,384 keys) and the bucket sort (up to 2^20) against numpy: its wave, round and size edges, keys whose
 bins are short (hashed, dense ids) and long (hubs, few values: the digit passes in LDS), and the stable sort by one
 column that a join's build side takes."""
 import numpy as np
@@ -46,3 +46,37 @@ def test_stable_by_column(provider, kind, n):
                                 provider.create_buffer_from_u32_columns([col, np.arange(n, dtype=np.uint32)]), [0], [0])
     want = np.concatenate([np.nonzero(col == v)[0] for v in some])
     assert np.array_equal(provider.download_column(out, 2), want.astype(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["hashed", "dense", "hub", "few", "equal"])
+@pytest.mark.parametrize("n", [16385, 32768, 32769, 100003, (1 << 20) - 1, 1 << 20, (1 << 20) + 1])
+def test_bucket_sort(provider, kind, n):
+    """The bucket sort at its size edges and where the number of buckets changes; a value with more repeats than a
+    bucket holds (few, equal) falls back to the digit passes."""
+    k = _keys(kind, n, np.random.default_rng(n))
+    R = provider.create_buffer_from_packed(k)
+    assert np.array_equal(provider.download_packed(provider.sort(R, [0, 1])), np.sort(k))
+    assert np.array_equal(provider.download_packed(provider.dedup_full_row(R)), np.unique(k))
+    assert np.array_equal(provider.download_packed(R), k)
+
+
+@pytest.mark.parametrize("order", ["ascending", "descending", "runs"])
+def test_bucket_sort_ordered_input(provider, order):
+    """Inputs whose order the sample's stretches follow."""
+    n = 200001
+    k = np.sort(np.random.default_rng(1).integers(0, 1 << 64, n, dtype=np.uint64))
+    k = {"ascending": k, "descending": k[::-1], "runs": np.roll(np.repeat(k[:: 7], 7)[:n], 3)}[order].copy()
+    R = provider.create_buffer_from_packed(k)
+    assert np.array_equal(provider.download_packed(provider.dedup_full_row(R)), np.unique(k))
+
+
+def test_fixpoint_with_repeated_facts(provider):
+    """A relation whose buckets do not fit (one fact repeated 60,000 times) inside a program."""
+    import oracle
+    from xlog_amd import datagen, tc_plan
+
+    s, d = datagen.random_digraph(3000, 4000, 5)
+    e = np.concatenate([pack(s, d), np.full(60000, pack(s[:1], d[:1])[0], dtype=np.uint64)])
+    outs, st = provider.fixpoint(tc_plan(), [provider.create_buffer_from_packed(e), None])
+    ref = oracle.bfs_tc(3000, s, d)
+    assert np.array_equal(provider.download_packed(outs[1]), ref["relation"]) and st["iterations"] == ref["iterations"]

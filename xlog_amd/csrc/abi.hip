@@ -488,9 +488,26 @@ void sort_unique_keys_async(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t
     select_unique(ctx, s, n, o.p, d_count);
     *out = o.release();
 }
+// The same by buckets: *d_count is ~0, and *out incomplete, when a bucket is too long for the route
+bool bucket_unique_keys_async(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t **out, uint64_t *d_count) {
+    if (!bucket_sort_takes(n)) return false;
+    Owned o(ctx, alloc_keys(ctx, n));
+    Buf<uint64_t> st;
+    bucket_sort(ctx, keys, n, o.p, d_count, st);
+    *out = o.release();
+    return true;
+}
 // The same with the count read back (returned).
 static uint64_t sort_unique_keys(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t **out) {
     Buf<uint64_t> cnt(ctx, 1);
+    if (bucket_unique_keys_async(ctx, keys, n, out, cnt.p)) {
+        Owned o(ctx, *out);
+        const uint64_t c = read_count(ctx, cnt.p);
+        if (c != ~0ull) {
+            o.release();
+            return c;
+        }
+    }
     sort_unique_keys_async(ctx, keys, n, out, cnt.p);
     return read_count(ctx, cnt.p);
 }

@@ -2210,11 +2210,21 @@ static DRel canon_drel_async(Ctx *ctx, const xlog_hip_rel *r, uint64_t *d_count,
         return d;
     }
     uint64_t *u;
-    sort_unique_keys_async(ctx, r->w[0], r->rows, &u, d_count, known_digits);
+    // (by buckets: the caller finds ~0 in *d_count when that did not fit, and calls canon_drel_again)
+    if (!bucket_unique_keys_async(ctx, r->w[0], r->rows, &u, d_count))
+        sort_unique_keys_async(ctx, r->w[0], r->rows, &u, d_count, known_digits);
     d.n = r->rows;
     d.k = u;
     d.owned = true;
     return d;
+}
+
+// The same by digit passes, for a relation whose buckets did not fit.
+static void canon_drel_again(Ctx *ctx, const xlog_hip_rel *r, uint64_t *d_count, uint32_t known_digits, DRel &d) {
+    ctx->free(d.k);
+    d.owned = false;
+    sort_unique_keys_async(ctx, r->w[0], r->rows, &d.k, d_count, known_digits);
+    d.owned = true;
 }
 
 // Device bytes an operation may still take: the free device memory, within
@@ -2338,10 +2348,17 @@ static void run_fixpoint_impl(Ctx *ctx, const int32_t *plan, uint32_t n_preds, c
             const int bits = maxid ? 32 - __builtin_clz(maxid) : 0;
             const uint32_t nd = (uint32_t)(bits + 7) / 8;  // bytes per column
             const uint32_t digits = nd ? (((1u << nd) - 1u) | (((1u << nd) - 1u) << 4)) : 1u;
+            auto digits_of = [&](uint32_t p) { return rels[p] && rels[p]->rows >= (1ull << 22) ? 0u : digits; };
             for (uint32_t p = 0; p < n_preds; ++p)
-                canon.d[p] = canon_drel_async(ctx, rels[p], sc.p + 1 + p,
-                                              rels[p] && rels[p]->rows >= (1ull << 22) ? 0u : digits);
+                canon.d[p] = canon_drel_async(ctx, rels[p], sc.p + 1 + p, digits_of(p));
             ctx->read_scalars(sc.p + 1, (uint64_t)n_preds);
+            bool again = false;
+            for (uint32_t p = 0; p < n_preds; ++p)
+                if (canon.d[p].owned && ctx->host_scalars[p] == ~0ull) {
+                    canon_drel_again(ctx, rels[p], sc.p + 1 + p, digits_of(p), canon.d[p]);
+                    again = true;
+                }
+            if (again) ctx->read_scalars(sc.p + 1, (uint64_t)n_preds);
             for (uint32_t p = 0; p < n_preds; ++p)
                 if (canon.d[p].owned) canon.d[p].n = ctx->host_scalars[p];
         }

@@ -326,6 +326,15 @@ struct SortUnique {
 // nothing done) for a larger or empty one.
 constexpr uint64_t BLOCK_SORT_KEYS = 1ull << 14;
 bool block_sort_unique(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *out, uint64_t *d_count);
+// Sorts of the whole key of up to BUCKET_SORT_KEYS keys (above the block
+// sort's) from in to out (n entries each, not shared).  With d_count the unique
+// keys, their number to *d_count (device).  A bucket too long for LDS leaves
+// out incomplete, *d_count = ~0 and the low half of state's first word
+// non-zero: the caller then sorts otherwise.
+// bucket_sort_takes: the sizes it is for (no: another sort was asked for).
+constexpr uint64_t BUCKET_SORT_KEYS = 1ull << 20;
+bool bucket_sort_takes(uint64_t n);
+void bucket_sort(Ctx *ctx, const uint64_t *in, uint64_t n, uint64_t *out, uint64_t *d_count, Buf<uint64_t> &state);
 // XLOG_HIP_SORT_TICKETS=1 (read at each sort): the radix pass and the
 // short-run unique order their tiles by an atomic start ticket instead of the
 // workgroup index, so that their look-back does not rest on workgroups

@@ -28,6 +28,7 @@
 #include "internal.hpp"
 #include "short_runs.hpp"
 
+#include <algorithm>
 #include <atomic>
 
 namespace xh {
@@ -191,20 +192,25 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int lane) {
 // bins' order by arrival does not show.  Bins that are long on average
 // (BLOCK_SORT_BIN keys: hub ids) and sorts by a part of the key, which have to
 // be stable, take digit passes in LDS instead, over the digits that vary.
-enum { BS_SORT, BS_UNIQUE, BS_DIGITS };
-constexpr int BS_TB = 1024, BS_ITEMS = 16, BS_BINS = 4096;
+constexpr int BS_TB = 1024, BS_ITEMS = 16;
 constexpr uint32_t BLOCK_SORT_BIN = 64;
 static_assert(BS_TB * BS_ITEMS == BLOCK_SORT_KEYS, "keys of one workgroup");
-template <int MODE>
-__global__ __launch_bounds__(BS_TB) void k_block_sort(const uint64_t *in, uint32_t n, uint64_t *out, uint64_t window,
-                                                      uint64_t *d_count) {
-    constexpr int WAVES = BS_TB / WAVE;
-    __shared__ uint64_t s_key[BS_TB * BS_ITEMS];
-    __shared__ uint32_t s_bin[BS_BINS];  // bins; the digit passes' [WAVES][256] counts; the unique's counts
-    __shared__ uint32_t s_part[WAVES], s_part2[WAVES];
-    static_assert(WAVES * 256 == BS_BINS && BS_ITEMS * WAVES <= BS_BINS, "shared arrays");
+template <int TB, int ITEMS>
+struct BsSmem {
+    static constexpr int WAVES = TB / WAVE, BINS = WAVES * 256;  // (bins, or the digit passes' [WAVES][256] counts)
+    uint64_t key[TB * ITEMS];
+    uint32_t bin[BINS];
+    uint32_t part[WAVES], part2[WAVES];
+};
+// The workgroup's n <= TB * ITEMS keys in[0 .. n) into sm.key, sorted by the
+// key's bits of `window` (stable: by digit passes only).  k is scratch.
+template <int TB, int ITEMS>
+__device__ __forceinline__ void block_sort(const uint64_t *in, uint32_t n, uint64_t window, bool stable,
+                                           BsSmem<TB, ITEMS> &sm, uint64_t (&k)[ITEMS]) {
+    constexpr int WAVES = TB / WAVE, BINS = WAVES * 256, BIN_BITS = __builtin_ctz(BINS), PER = BINS / TB;
+    static_assert(BINS == 1 << BIN_BITS && TB >= 256, "a power of two of bins; a thread per digit");
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid >> 6;
-    const uint32_t rounds = (n + BS_TB - 1) / BS_TB;
+    const uint32_t rounds = (n + TB - 1) / TB;
     auto block_or = [&](uint32_t v, uint32_t *part) {
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v |= (uint32_t)__shfl_xor((int)v, o, WAVE);
@@ -213,88 +219,87 @@ __global__ __launch_bounds__(BS_TB) void k_block_sort(const uint64_t *in, uint32
     // exclusive prefix of one value per thread
     auto block_scan = [&](uint32_t v) {
         const uint32_t x = wave_incl_scan(v, lane);
-        if (lane == WAVE - 1) s_part[wave] = x;
+        if (lane == WAVE - 1) sm.part[wave] = x;
         __syncthreads();
         uint32_t pre = 0;
-        for (int w = 0; w < wave; ++w) pre += s_part[w];
+        for (int w = 0; w < wave; ++w) pre += sm.part[w];
         return pre + x - v;
     };
     // the wave's keys are consecutive (wave * rounds * 64 + r * 64 + lane), as the stable passes need them
     const uint32_t base = (uint32_t)wave * rounds * WAVE + lane;
-    uint64_t k[BS_ITEMS];
     const uint64_t k0 = in[0];
     uint64_t vary = 0;
 #pragma unroll
-    for (int r = 0; r < BS_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const uint32_t i = base + r * WAVE;
         const bool live = (uint32_t)r < rounds && i < n;
         k[r] = live ? in[i] : k0;
         vary |= k[r] ^ k0;
     }
-    block_or((uint32_t)vary, s_part);
-    block_or((uint32_t)(vary >> 32), s_part2);
+    block_or((uint32_t)vary, sm.part);
+    block_or((uint32_t)(vary >> 32), sm.part2);
 #pragma unroll
-    for (int q = 0; q < BS_BINS / BS_TB; ++q) s_bin[q * BS_TB + tid] = 0;
+    for (int q = 0; q < PER; ++q) sm.bin[q * TB + tid] = 0;
     __syncthreads();
     uint32_t vlo = 0, vhi = 0;
     for (int w = 0; w < WAVES; ++w) {
-        vlo |= s_part[w];
-        vhi |= s_part2[w];
+        vlo |= sm.part[w];
+        vhi |= sm.part2[w];
     }
     vary = (((uint64_t)vhi << 32) | vlo) & window;
     bool sorted = false;
-    if (MODE != BS_DIGITS && vary) {
+    if (!stable && vary) {
         const int nlo = vlo ? 32 - __clz((int)vlo) : 0, nhi = vhi ? 32 - __clz((int)vhi) : 0;
-        const int shift = nlo + nhi > 12 ? nlo + nhi - 12 : 0;
+        const int shift = nlo + nhi > BIN_BITS ? nlo + nhi - BIN_BITS : 0;
         const uint64_t mlo = (1ull << nlo) - 1, mhi = (1ull << nhi) - 1;
         auto bin_of = [&](uint64_t x) { return (uint32_t)(((((x >> 32) & mhi) << nlo) | (x & mlo)) >> shift); };
-        uint32_t slot[BS_ITEMS];
+        uint32_t slot[ITEMS];
 #pragma unroll
-        for (int r = 0; r < BS_ITEMS; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const uint32_t i = base + r * WAVE;
-            slot[r] = (uint32_t)r < rounds && i < n ? atomicAdd(&s_bin[bin_of(k[r])], 1u) : 0u;
+            slot[r] = (uint32_t)r < rounds && i < n ? atomicAdd(&sm.bin[bin_of(k[r])], 1u) : 0u;
         }
         __syncthreads();
-        uint32_t c[BS_BINS / BS_TB], tot = 0, sq = 0;
+        uint32_t c[PER], tot = 0, sq = 0;
 #pragma unroll
-        for (int q = 0; q < BS_BINS / BS_TB; ++q) {
-            c[q] = s_bin[tid * (BS_BINS / BS_TB) + q];
+        for (int q = 0; q < PER; ++q) {
+            c[q] = sm.bin[tid * (PER) + q];
             tot += c[q];
             sq += c[q] * c[q];  // (at most 2^28 over all bins)
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) sq += (uint32_t)__shfl_xor((int)sq, o, WAVE);
-        if (lane == 0) s_part2[wave] = sq;
-        uint32_t pre = block_scan(tot);  // (its barrier also publishes s_part2)
+        if (lane == 0) sm.part2[wave] = sq;
+        uint32_t pre = block_scan(tot);  // (its barrier also publishes sm.part2)
         uint32_t sum = 0;
-        for (int w = 0; w < WAVES; ++w) sum += s_part2[w];
+        for (int w = 0; w < WAVES; ++w) sum += sm.part2[w];
         __syncthreads();
         sorted = sum <= BLOCK_SORT_BIN * n;  // block-uniform
         if (sorted) {
 #pragma unroll
-            for (int q = 0; q < BS_BINS / BS_TB; ++q) {
-                s_bin[tid * (BS_BINS / BS_TB) + q] = pre;
+            for (int q = 0; q < PER; ++q) {
+                sm.bin[tid * (PER) + q] = pre;
                 pre += c[q];
             }
             __syncthreads();
 #pragma unroll
-            for (int r = 0; r < BS_ITEMS; ++r) {
+            for (int r = 0; r < ITEMS; ++r) {
                 const uint32_t i = base + r * WAVE;
-                if ((uint32_t)r < rounds && i < n) s_key[s_bin[bin_of(k[r])] + slot[r]] = k[r];
+                if ((uint32_t)r < rounds && i < n) sm.key[sm.bin[bin_of(k[r])] + slot[r]] = k[r];
             }
             __syncthreads();
-            uint32_t to[BS_ITEMS];
+            uint32_t to[ITEMS];
 #pragma unroll
-            for (int r = 0; r < BS_ITEMS; ++r) {
+            for (int r = 0; r < ITEMS; ++r) {
                 const uint32_t i = base + r * WAVE;
                 to[r] = 0;
                 if ((uint32_t)r < rounds && i < n) {
-                    k[r] = s_key[i];
+                    k[r] = sm.key[i];
                     const uint32_t b = bin_of(k[r]);
-                    const uint32_t lo = s_bin[b], hi = b + 1 < BS_BINS ? s_bin[b + 1] : n;
+                    const uint32_t lo = sm.bin[b], hi = b + 1 < BINS ? sm.bin[b + 1] : n;
                     uint32_t rank = lo;
                     for (uint32_t j = lo; j < hi; ++j) {
-                        const uint64_t x = s_key[j];
+                        const uint64_t x = sm.key[j];
                         rank += (x < k[r] || (x == k[r] && j < i)) ? 1u : 0u;
                     }
                     to[r] = rank;
@@ -302,9 +307,9 @@ __global__ __launch_bounds__(BS_TB) void k_block_sort(const uint64_t *in, uint32
             }
             __syncthreads();
 #pragma unroll
-            for (int r = 0; r < BS_ITEMS; ++r) {
+            for (int r = 0; r < ITEMS; ++r) {
                 const uint32_t i = base + r * WAVE;
-                if ((uint32_t)r < rounds && i < n) s_key[to[r]] = k[r];
+                if ((uint32_t)r < rounds && i < n) sm.key[to[r]] = k[r];
             }
             __syncthreads();
         }
@@ -312,12 +317,12 @@ __global__ __launch_bounds__(BS_TB) void k_block_sort(const uint64_t *in, uint32
     if (!sorted) {
         for (int dgt = 0; dgt < 8; ++dgt) {
             if (!((vary >> (8 * dgt)) & 255u)) continue;  // block-uniform
-            for (int q = 0; q < BS_BINS / BS_TB; ++q) s_bin[q * BS_TB + tid] = 0;
+            for (int q = 0; q < PER; ++q) sm.bin[q * TB + tid] = 0;
             __syncthreads();
-            uint32_t *wcnt = s_bin + wave * 256;
-            uint32_t rank[BS_ITEMS];
+            uint32_t *wcnt = sm.bin + wave * 256;
+            uint32_t rank[ITEMS];
 #pragma unroll
-            for (int r = 0; r < BS_ITEMS; ++r) {
+            for (int r = 0; r < ITEMS; ++r) {
                 rank[r] = 0;
                 if ((uint32_t)r >= rounds) continue;  // block-uniform
                 const uint32_t i = base + r * WAVE;
@@ -339,63 +344,223 @@ __global__ __launch_bounds__(BS_TB) void k_block_sort(const uint64_t *in, uint32
             uint32_t cnt = 0;
             if (tid < 256)
                 for (int w = 0; w < WAVES; ++w) {
-                    const uint32_t c = s_bin[w * 256 + tid];
-                    s_bin[w * 256 + tid] = cnt;
+                    const uint32_t c = sm.bin[w * 256 + tid];
+                    sm.bin[w * 256 + tid] = cnt;
                     cnt += c;
                 }
             const uint32_t start = block_scan(tid < 256 ? cnt : 0u);
             if (tid < 256)
-                for (int w = 0; w < WAVES; ++w) s_bin[w * 256 + tid] += start;
+                for (int w = 0; w < WAVES; ++w) sm.bin[w * 256 + tid] += start;
             __syncthreads();
 #pragma unroll
-            for (int r = 0; r < BS_ITEMS; ++r) {
+            for (int r = 0; r < ITEMS; ++r) {
                 const uint32_t i = base + r * WAVE;
-                if ((uint32_t)r < rounds && i < n) s_key[wcnt[(uint32_t)(k[r] >> (8 * dgt)) & 255u] + rank[r]] = k[r];
+                if ((uint32_t)r < rounds && i < n) sm.key[wcnt[(uint32_t)(k[r] >> (8 * dgt)) & 255u] + rank[r]] = k[r];
             }
             __syncthreads();
 #pragma unroll
-            for (int r = 0; r < BS_ITEMS; ++r) {
+            for (int r = 0; r < ITEMS; ++r) {
                 const uint32_t i = base + r * WAVE;
-                if ((uint32_t)r < rounds && i < n) k[r] = s_key[i];
+                if ((uint32_t)r < rounds && i < n) k[r] = sm.key[i];
             }
         }
         if (!vary) {  // nothing to order
 #pragma unroll
-            for (int r = 0; r < BS_ITEMS; ++r) {
+            for (int r = 0; r < ITEMS; ++r) {
                 const uint32_t i = base + r * WAVE;
-                if ((uint32_t)r < rounds && i < n) s_key[i] = k[r];
+                if ((uint32_t)r < rounds && i < n) sm.key[i] = k[r];
             }
         }
         __syncthreads();
     }
-    if (MODE != BS_UNIQUE) {
-        for (uint32_t i = tid; i < n; i += BS_TB) out[i] = s_key[i];
-        return;
-    }
-    // the keys that differ from the one before, in order: counts per (wave, round), their prefix, the write
-    uint64_t bal[BS_ITEMS];
+}
+// Of the sorted keys in sm.key, the ones that differ from the one before: the
+// wave's (its consecutive keys, k) as ballots per round, the number before the
+// wave's first in pos; returns the workgroup's number.
+template <int TB, int ITEMS>
+__device__ __forceinline__ uint32_t block_unique(uint32_t n, BsSmem<TB, ITEMS> &sm, uint64_t (&k)[ITEMS],
+                                                 uint64_t (&bal)[ITEMS], uint32_t *pos) {
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid >> 6;
+    const uint32_t rounds = (n + TB - 1) / TB, base = (uint32_t)wave * rounds * WAVE + lane;
     uint32_t mine = 0;
 #pragma unroll
-    for (int r = 0; r < BS_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const uint32_t i = base + r * WAVE;
-        k[r] = (uint32_t)r < rounds && i < n ? s_key[i] : 0ull;
-        const bool keep = (uint32_t)r < rounds && i < n && (i == 0 || s_key[i - 1] != k[r]);
+        k[r] = (uint32_t)r < rounds && i < n ? sm.key[i] : 0ull;
+        const bool keep = (uint32_t)r < rounds && i < n && (i == 0 || sm.key[i - 1] != k[r]);
         bal[r] = __ballot(keep);
         mine += (uint32_t)__popcll(bal[r]);
     }
-    if (lane == 0) s_part2[wave] = mine;
+    if (lane == 0) sm.part2[wave] = mine;
     __syncthreads();
-    uint32_t pos = 0, total = 0;
-    for (int w = 0; w < WAVES; ++w) {
-        if (w < wave) pos += s_part2[w];
-        total += s_part2[w];
+    uint32_t total = 0;
+    *pos = 0;
+    for (int w = 0; w < (TB / WAVE); ++w) {
+        if (w < wave) *pos += sm.part2[w];
+        total += sm.part2[w];
+    }
+    return total;
+}
+template <int ITEMS>
+__device__ __forceinline__ void block_write(const uint64_t (&k)[ITEMS], const uint64_t (&bal)[ITEMS], uint64_t *out) {
+    const int lane = threadIdx.x & (WAVE - 1);
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        if ((bal[r] >> lane) & 1ull) out[__popcll(bal[r] & ((1ull << lane) - 1ull))] = k[r];
+        out += __popcll(bal[r]);
+    }
+}
+enum { BS_SORT, BS_UNIQUE, BS_DIGITS };
+template <int MODE>
+__global__ __launch_bounds__(BS_TB) void k_block_sort(const uint64_t *in, uint32_t n, uint64_t *out, uint64_t window,
+                                                      uint64_t *d_count) {
+    __shared__ BsSmem<BS_TB, BS_ITEMS> sm;
+    uint64_t k[BS_ITEMS];
+    block_sort<BS_TB, BS_ITEMS>(in, n, window, MODE == BS_DIGITS, sm, k);
+    if (MODE != BS_UNIQUE) {
+        for (uint32_t i = threadIdx.x; i < n; i += BS_TB) out[i] = sm.key[i];
+        return;
+    }
+    uint64_t bal[BS_ITEMS];
+    uint32_t pos;
+    const uint32_t total = block_unique<BS_TB, BS_ITEMS>(n, sm, k, bal, &pos);
+    block_write<BS_ITEMS>(k, bal, out + pos);
+    if (threadIdx.x == 0) *d_count = total;
+}
+
+// Sorts of BLOCK_SORT_KEYS .. BUCKET_SORT_KEYS whole keys (a sample sort): one
+// workgroup sorts a sample of the keys and takes the buckets' bounds from it,
+// one pass moves the keys into their buckets' fixed regions (about 1,024 keys
+// in room for 4,096), and one workgroup per bucket sorts it in LDS and writes
+// it (or its unique keys, gathered by a fourth launch), against a histogram and
+// up to eight passes of 9 to 20 us that leave most CUs idle at these sizes (a
+// dedup of 10^5 hashed pairs 145 -> 42 us, of 10^6 196 -> 89, of 10^6 pairs of
+// ids below 1,000 121 -> 84; the digit passes of 4 * 10^6 pairs are faster).  Bounds from a sample follow any distribution (hub ids included); only
+// one value's repeats, or a sample far off, can fill a bucket, which sets
+// `over`: the caller then takes the digit passes.  The buckets are filled in
+// arrival order (whole keys: it does not show).
+constexpr int BK_TB = 512, BK_ITEMS = 8, BK_KEYS = BK_TB * BK_ITEMS, BK_MAX_BITS = 10;
+constexpr uint32_t BK_SAMPLE = 8 << BK_MAX_BITS;  // eight keys per bucket: the fullest holds about 2.5 times the average
+struct BucketState {
+    uint32_t over, pad;
+    uint32_t cursor[1 << BK_MAX_BITS], uniq[1 << BK_MAX_BITS];  // keys, unique keys of each bucket
+    uint64_t bound[1 << BK_MAX_BITS];  // bucket b holds the keys x with bound[b - 1] <= x < bound[b]
+};
+__global__ __launch_bounds__(BS_TB) void k_bucket_sample(const uint64_t *__restrict__ in, uint64_t n, BucketState *st,
+                                                         int bits, uint64_t *__restrict__ sample) {
+    __shared__ BsSmem<BS_TB, BK_SAMPLE / BS_TB> sm;
+    const uint32_t nb = 1u << bits;
+    for (uint32_t i = threadIdx.x; i < nb; i += BS_TB) st->cursor[i] = 0;
+    if (threadIdx.x == 0) st->over = 0;
+    const uint32_t ns = 8u << bits;
+    const uint64_t step = n / ns;  // (over 512 keys a bucket)
+    for (uint32_t i = threadIdx.x; i < ns; i += BS_TB)  // one key of each stretch, at a place of its own
+        sample[i] = in[i * step + (((i * 0x9E3779B1u) >> 8) % (uint32_t)step)];
+    __syncthreads();
+    uint64_t k[BK_SAMPLE / BS_TB];
+    block_sort<BS_TB, BK_SAMPLE / BS_TB>(sample, ns, ~0ull, false, sm, k);
+    for (uint32_t i = threadIdx.x; i < nb; i += BS_TB)
+        st->bound[i] = i + 1 < nb ? sm.key[(i + 1) * 8] : ~0ull;
+}
+constexpr int BC_TB = 1024, BC_ITEMS = 8;  // a tile of 8,192 keys
+__global__ __launch_bounds__(BC_TB) void k_bucket_scatter(const uint64_t *__restrict__ in, uint64_t n, BucketState *st,
+                                                          int bits, uint64_t *__restrict__ out) {
+    __shared__ uint64_t s_bound[1 << BK_MAX_BITS];
+    __shared__ uint32_t s_cnt[1 << BK_MAX_BITS];
+    const int tid = threadIdx.x, nb = 1 << bits;
+    const uint64_t base = (uint64_t)blockIdx.x * BC_TB * BC_ITEMS + tid;
+    uint64_t k[BC_ITEMS];
+#pragma unroll
+    for (int r = 0; r < BC_ITEMS; ++r) k[r] = base + r * BC_TB < n ? in[base + r * BC_TB] : 0ull;
+    for (int i = tid; i < nb; i += BC_TB) {
+        s_cnt[i] = 0;
+        s_bound[i] = st->bound[i];
+    }
+    __syncthreads();
+    // the number of bounds <= the key (the last bound is no bound: every search ends below it)
+    uint32_t b[BC_ITEMS], rank[BC_ITEMS];
+#pragma unroll
+    for (int r = 0; r < BC_ITEMS; ++r) b[r] = 0;
+    for (int step = nb >> 1; step > 0; step >>= 1) {
+#pragma unroll
+        for (int r = 0; r < BC_ITEMS; ++r) b[r] += s_bound[b[r] + step - 1] <= k[r] ? step : 0;
     }
 #pragma unroll
-    for (int r = 0; r < BS_ITEMS; ++r) {
-        if ((bal[r] >> lane) & 1ull) out[pos + (uint32_t)__popcll(bal[r] & ((1ull << lane) - 1ull))] = k[r];
-        pos += (uint32_t)__popcll(bal[r]);
+    for (int r = 0; r < BC_ITEMS; ++r) rank[r] = base + r * BC_TB < n ? atomicAdd(&s_cnt[b[r]], 1u) : 0u;
+    __syncthreads();
+    for (int i = tid; i < nb; i += BC_TB)
+        if (s_cnt[i]) {
+            const uint32_t c = s_cnt[i], at = atomicAdd(&st->cursor[i], c);
+            if (at + c > (uint32_t)BK_KEYS) st->over = 1;
+            s_cnt[i] = at;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < BC_ITEMS; ++r) {
+        const uint32_t at = s_cnt[b[r]] + rank[r];
+        if (base + r * BC_TB < n && at < (uint32_t)BK_KEYS) out[(uint64_t)b[r] * BK_KEYS + at] = k[r];
     }
-    if (tid == 0) *d_count = total;
+}
+__device__ __forceinline__ uint32_t bucket_block_total(uint32_t v, uint32_t *part) {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o, WAVE);
+    __syncthreads();
+    if ((tid & (WAVE - 1)) == 0) part[tid >> 6] = v;
+    __syncthreads();
+    v = 0;
+    for (int w = 0; w < BK_TB / WAVE; ++w) v += part[w];
+    return v;
+}
+// All keys: each workgroup adds up the buckets before its own and writes to out.
+// Unique keys: their number is known only here, so they stay in the bucket's
+// region and k_bucket_gather moves them to out (waiting for the counts of the
+// buckets before, in this launch, took 23 us at 10^6 keys; the gather takes 5).
+template <bool UNIQUE>
+__global__ __launch_bounds__(BK_TB) void k_bucket_sort(uint64_t *regions, BucketState *st, uint64_t *__restrict__ out) {
+    __shared__ BsSmem<BK_TB, BK_ITEMS> sm;
+    const int tid = threadIdx.x;
+    if (st->over) return;
+    const uint32_t t = blockIdx.x, n = st->cursor[t];
+    uint64_t *region = regions + (uint64_t)t * BK_KEYS;
+    uint64_t k[BK_ITEMS];
+    if (n) block_sort<BK_TB, BK_ITEMS>(region, n, ~0ull, false, sm, k);  // block-uniform
+    if (!UNIQUE) {
+        uint32_t before = 0;
+        for (uint32_t i = tid; i < t; i += BK_TB) before += st->cursor[i];
+        before = bucket_block_total(before, sm.part);
+        for (uint32_t i = tid; i < n; i += BK_TB) out[before + i] = sm.key[i];
+        return;
+    }
+    uint32_t total = 0;
+    if (n) {
+        uint64_t bal[BK_ITEMS];
+        uint32_t pos;
+        total = block_unique<BK_TB, BK_ITEMS>(n, sm, k, bal, &pos);
+        block_write<BK_ITEMS>(k, bal, region + pos);
+    }
+    if (tid == 0) st->uniq[t] = total;
+}
+__global__ __launch_bounds__(BK_TB) void k_bucket_gather(const uint64_t *__restrict__ regions,
+                                                         const BucketState *__restrict__ st, uint64_t *__restrict__ out,
+                                                         uint64_t *d_count) {
+    __shared__ uint32_t s_part[BK_TB / WAVE];
+    const uint32_t tid = threadIdx.x, t = blockIdx.x;
+    if (st->over) {
+        if (t == 0 && tid == 0) *d_count = ~0ull;
+        return;
+    }
+    const uint32_t n = st->uniq[t];
+    uint64_t k[BK_ITEMS];
+#pragma unroll
+    for (int r = 0; r < BK_ITEMS; ++r) k[r] = r * BK_TB + tid < n ? regions[(uint64_t)t * BK_KEYS + r * BK_TB + tid] : 0ull;
+    uint32_t before = 0;
+    for (uint32_t i = tid; i < t; i += BK_TB) before += st->uniq[i];
+    before = bucket_block_total(before, s_part);
+#pragma unroll
+    for (int r = 0; r < BK_ITEMS; ++r)
+        if (r * BK_TB + tid < n) out[before + r * BK_TB + tid] = k[r];
+    if (tid == 0 && t + 1 == gridDim.x) *d_count = before + n;
 }
 
 // Tile order of the digit passes.  Consecutive tiles write adjacent pieces of
@@ -996,6 +1161,29 @@ int radix_sort_dev(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n_bo
 static bool sort_block() {
     return !getenv("XLOG_HIP_SORT_TICKETS") && !getenv("XLOG_HIP_SORT_PERSIST") && !getenv("XLOG_HIP_SORT_SPIN");
 }
+bool bucket_sort_takes(uint64_t n) { return n > BLOCK_SORT_KEYS && n <= BUCKET_SORT_KEYS && sort_block(); }
+void bucket_sort(Ctx *ctx, const uint64_t *in, uint64_t n, uint64_t *out, uint64_t *d_count, Buf<uint64_t> &state) {
+    int bits = 1;
+    while ((n >> bits) > 1024) ++bits;
+    XH_REQUIRE(n > BLOCK_SORT_KEYS && n <= BUCKET_SORT_KEYS && bits <= BK_MAX_BITS, XLOG_HIP_INVALID_ARG,
+               "bucket sort: number of keys");
+    Buf<uint64_t> regions(ctx, (uint64_t)BK_KEYS << bits);
+    state = Buf<uint64_t>(ctx, sizeof(BucketState) / 8);
+    BucketState *st = reinterpret_cast<BucketState *>(state.p);
+    // (the sample's keys pass through the regions, which the scatter fills afterwards)
+    hipLaunchKernelGGL(k_bucket_sample, dim3(1), dim3(BS_TB), 0, ctx->stream, in, n, st, bits, regions.p);
+    hipLaunchKernelGGL(k_bucket_scatter, dim3((unsigned)((n + BC_TB * BC_ITEMS - 1) / (BC_TB * BC_ITEMS))), dim3(BC_TB), 0,
+                       ctx->stream, in, n, st, bits, regions.p);
+    Prof prof(ctx, XLOG_HIP_KERNEL_SORT_SEGMENTS, 16.0 * (double)n);
+    if (d_count) {
+        hipLaunchKernelGGL(k_bucket_sort<true>, dim3(1u << bits), dim3(BK_TB), 0, ctx->stream, regions.p, st, out);
+        hipLaunchKernelGGL(k_bucket_gather, dim3(1u << bits), dim3(BK_TB), 0, ctx->stream, regions.p, st, out, d_count);
+    } else {
+        hipLaunchKernelGGL(k_bucket_sort<false>, dim3(1u << bits), dim3(BK_TB), 0, ctx->stream, regions.p, st, out);
+    }
+    XH_CHECK_HIP(hipGetLastError());
+}
+
 bool block_sort_unique(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *out, uint64_t *d_count) {
     if (n == 0 || n > BLOCK_SORT_KEYS || !sort_block()) return false;
     Prof prof(ctx, XLOG_HIP_KERNEL_SORT_PASS, 16.0 * (double)n);
@@ -1027,6 +1215,15 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **va
                                (~0ull >> (64 - 8 * digit_hi)) & ~((1ull << (8 * digit_lo)) - 1ull), nullptr);
         XH_CHECK_HIP(hipGetLastError());
         return 1;
+    }
+    if (!has_val && digit_lo == 0 && digit_hi == 8 && !known_digits && !uq && bucket_sort_takes(n)) {
+        Buf<uint64_t> st;
+        bucket_sort(ctx, src ? src : *keys, n, *keys_alt, nullptr, st);
+        ctx->read_scalars(st.p, 1);
+        if (!(uint32_t)ctx->host_scalars[0]) {  // BucketState::over
+            std::swap(*keys, *keys_alt);
+            return 2;
+        }
     }
     const uint64_t tile_keys = has_val ? (uint64_t)SORT_BLOCK_V * SORT_ITEMS_V : (uint64_t)SORT_BLOCK_K * SORT_ITEMS_K;
     const uint64_t tiles = (n + tile_keys - 1) / tile_keys;
