@@ -194,8 +194,9 @@ struct Ctx {
         wait_event(ev_sync);
     }
     // D2H of a few u64 scalars to host_scalars (waits for them)
-    void read_scalars(const void *dev, size_t count_u64) {
-        post_read(dev, count_u64);
+    // (also, when given: one more word, at host_scalars[count_u64])
+    void read_scalars(const void *dev, size_t count_u64, const uint64_t *also = nullptr) {
+        post_read(dev, count_u64, also);
         wait_read();
     }
     // The two halves of a read-back: a kernel on the stream stores the words
@@ -204,7 +205,7 @@ struct Ctx {
     // launch and no packets around it, 6 us less per read-back (a dedup of
     // 5,003 pairs with its one read-back 31 -> 25 us).
     // Later launches may be queued between the halves; one read-back at a time.
-    void post_read(const void *dev, size_t count_u64);
+    void post_read(const void *dev, size_t count_u64, const uint64_t *also = nullptr);
     void wait_read();
     uint64_t *host_seq = nullptr;  // pinned, beside host_scalars
     uint64_t read_seq = 0;
@@ -490,6 +491,9 @@ struct RunIndex {
     Buf<unsigned long long> table;  // per slot: (key << 32) | run length (0 = empty), run start
     uint64_t nruns = 0;
     uint64_t table_mask = 0;
+    // the slot of a key is the key itself (keys below table_mask + 1): for keys packed from a few bits, whose runs
+    // then land in their slots in order and are found in one access.  Only the probe of a ProbeJob reads such a table.
+    bool direct = false;
 };
 void build_run_index(Ctx *ctx, const uint64_t *sorted_keys, uint64_t n, RunIndex &ix);
 // The same in two steps around one read-back: the runs of sorted_keys[0, n)
@@ -506,6 +510,7 @@ void build_run_index_finish(Ctx *ctx, RunScratch &rs, uint64_t nruns, uint64_t n
 // device row count: *d_nruns runs, at most runs_bound, over *d_n sorted keys):
 // ix.table holds ix.table_mask + 1 >= 2 * runs_bound slots and is cleared and
 // filled here, with no read-back; a raised stop leaves it cleared.
+// (ix.direct: table_mask + 1 slots above every key instead.)
 void run_index_insert_dev(Ctx *ctx, const uint32_t *run_key, const uint64_t *run_start, const uint64_t *d_nruns,
                           uint64_t runs_bound, const uint64_t *d_n, RunIndex &ix, const uint32_t *stop);
 // Merge-path lookup of the sort-merge join: for every row of l (sorted by the
@@ -549,6 +554,9 @@ struct ProbeJob {
     Buf<uint32_t> rec_cnt;
     Buf<uint64_t> toff;  // exclusive prefix of per-tile output counts; toff[tiles] = total
     uint64_t tiles = 0, total = 0;
+    // optional device word read back together with the total
+    const uint64_t *also = nullptr;
+    uint64_t also_value = 0;
     int items = 16;      // probe rows per thread (set by probe_prepare); a tile is 256 * items rows
 };
 uint64_t probe_prepare(Ctx *ctx, ProbeJob &job);

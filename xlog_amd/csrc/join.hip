@@ -102,6 +102,21 @@ __global__ void k_insert_dev(const uint32_t *__restrict__ run_key, const uint64_
     }
 }
 
+// k_insert_dev for a table whose slots are the keys (RunIndex::direct): the
+// runs come in key order, so their slots are written in order, with no atomic.
+__global__ void k_insert_direct(const uint32_t *__restrict__ run_key, const uint64_t *__restrict__ run_start,
+                                const uint64_t *d_nruns, uint64_t runs_bound, const uint64_t *d_n,
+                                unsigned long long *table, uint64_t mask) {
+    const uint64_t nruns = *d_nruns < runs_bound ? *d_nruns : runs_bound, n = *d_n;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < nruns; r += stride) {
+        const uint32_t key = run_key[r];
+        const uint64_t st = run_start[r], en = r + 1 < nruns ? run_start[r + 1] : n;
+        if (key > mask) continue;  // (only in the words of a sort that did not fit)
+        *reinterpret_cast<u64x2 *>(table + 2 * (uint64_t)key) = u64x2{((unsigned long long)key << 32) | (en - st), st};
+    }
+}
+
 __global__ void k_set_u64(uint64_t *p, uint64_t v) { *p = v; }
 __global__ void k_max_run_len(const uint64_t *__restrict__ run_start, uint64_t nruns, unsigned long long *mx) {
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -170,6 +185,8 @@ struct ProbeArgs {
     unsigned long long *fcount;
     uint64_t fcap;
     uint32_t fwords;
+    // RunIndex::direct
+    uint32_t direct;
 };
 // set in a row's start when its outputs come from gsrc
 constexpr uint64_t GROUP_BIT = 1ull << 63;
@@ -204,7 +221,8 @@ __device__ __forceinline__ void lookup_batch(const ProbeArgs &a, const uint64_t 
             const uint32_t key = a.pcol ? (uint32_t)rows[r] : (uint32_t)(rows[r] >> 32);
             const uint64_t idx = wbase + (uint64_t)r * WAVE + lane;
             const bool valid = idx < a.n;
-            slot[q] = valid ? load_slot(a.table, hash_slot(key, a.bits)) : u64x2{0ull, 0ull};
+            const bool in = valid && (!a.direct || key <= a.mask);
+            slot[q] = in ? load_slot(a.table, a.direct ? (uint64_t)key : hash_slot(key, a.bits)) : u64x2{0ull, 0ull};
             g[q] = (a.gsel && valid) ? a.gsel[idx] : -1;
         }
 #pragma unroll
@@ -710,7 +728,57 @@ __global__ __launch_bounds__(JB) void k_wcoj_triangle(const uint64_t *__restrict
     }
 }
 
+// A set of u32 keys for semi and anti joins, which need no runs: 8-byte slots
+// (1 << 32) | key, 0 empty, linear probing.
+__device__ __forceinline__ uint32_t key_of_row(uint64_t row, int pcol) { return pcol ? (uint32_t)row : (uint32_t)(row >> 32); }
+__global__ void k_key_set_insert(const uint64_t *__restrict__ rows, uint64_t n, int pcol, unsigned long long *set,
+                                 uint64_t mask, int bits) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        const unsigned long long v = (1ull << 32) | key_of_row(rows[i], pcol);
+        for (uint64_t h = hash_slot((uint32_t)v, bits);; h = (h + 1) & mask) {
+            // (a key already there, a hub's above all, needs no atomic)
+            unsigned long long s = __hip_atomic_load(&set[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (s == 0ull) s = atomicCAS(&set[h], 0ull, v);
+            if (s == 0ull || s == v) break;
+        }
+    }
+}
+__global__ void k_key_set_flags(const uint64_t *__restrict__ rows, uint64_t n, int pcol,
+                                const unsigned long long *__restrict__ set, uint64_t mask, int bits, int want,
+                                uint8_t *__restrict__ flags) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        const unsigned long long v = (1ull << 32) | key_of_row(rows[i], pcol);
+        bool hit = false;
+        for (uint64_t h = hash_slot((uint32_t)v, bits);; h = (h + 1) & mask) {
+            const unsigned long long s = set[h];
+            hit = s == v;
+            if (hit || s == 0ull) break;
+        }
+        flags[i] = (uint8_t)(hit == (want != 0));
+    }
+}
+
 }  // namespace
+
+void key_set_build(Ctx *ctx, const uint64_t *rows, uint64_t n, int pcol, Buf<unsigned long long> &set) {
+    uint64_t slots = 1024;
+    while (slots < 2 * n) slots <<= 1;
+    set = Buf<unsigned long long>(ctx, slots);
+    fill_u64(ctx, reinterpret_cast<uint64_t *>(set.p), 0ull, slots);
+    if (!n) return;
+    hipLaunchKernelGGL(k_key_set_insert, dim3(grid_for(n, 256, 16384)), dim3(256), 0, ctx->stream, rows, n, pcol, set.p,
+                       slots - 1, __builtin_ctzll(slots));
+    XH_CHECK_HIP(hipGetLastError());
+}
+void key_set_flags(Ctx *ctx, const uint64_t *rows, uint64_t n, int pcol, const Buf<unsigned long long> &set, int want,
+                   uint8_t *flags) {
+    if (!n) return;
+    hipLaunchKernelGGL(k_key_set_flags, dim3(grid_for(n, 256, 16384)), dim3(256), 0, ctx->stream, rows, n, pcol, set.p,
+                       set.n - 1, __builtin_ctzll(set.n), want, flags);
+    XH_CHECK_HIP(hipGetLastError());
+}
 
 // Runs of the high word of sorted keys [0, n), n = *d_n when d_n is set
 // (then n_bound sizes the buffers): key and start per run, the run count to
@@ -751,6 +819,15 @@ void build_run_index_finish(Ctx *ctx, RunScratch &rs, uint64_t nruns, uint64_t n
 void run_index_insert_dev(Ctx *ctx, const uint32_t *run_key, const uint64_t *run_start, const uint64_t *d_nruns,
                           uint64_t runs_bound, const uint64_t *d_n, RunIndex &ix, const uint32_t *stop) {
     const uint64_t slots = ix.table_mask + 1;
+    if (ix.direct) {
+        XH_REQUIRE(!stop, XLOG_HIP_INVALID_ARG, "run index: a direct table in a queued iteration");
+        fill_u64(ctx, reinterpret_cast<uint64_t *>(ix.table.p), 0ull, 2 * slots);
+        if (!runs_bound) return;
+        hipLaunchKernelGGL(k_insert_direct, dim3(grid_for(runs_bound, 256, 16384)), dim3(256), 0, ctx->stream, run_key,
+                           run_start, d_nruns, runs_bound, d_n, ix.table.p, ix.table_mask);
+        XH_CHECK_HIP(hipGetLastError());
+        return;
+    }
     XH_REQUIRE(slots >= 2 * runs_bound, XLOG_HIP_INVALID_ARG, "run index: table smaller than twice its runs");
     fill_u64(ctx, reinterpret_cast<uint64_t *>(ix.table.p), 0ull, 2 * slots);
     if (!runs_bound) return;
@@ -774,8 +851,10 @@ static int table_bits(const RunIndex &ix) {
 
 static ProbeArgs probe_args(const ProbeJob &job) {
     const RunIndex &ix = *job.ix;
-    return ProbeArgs{job.probe, job.n, job.pcol, ix.table.p, ix.table_mask, table_bits(ix), job.payload, job.gsel,
-                     job.gseg, job.gsrc, job.pre_start, job.pre_cnt, nullptr, nullptr};
+    ProbeArgs a{job.probe, job.n, job.pcol, ix.table.p, ix.table_mask, table_bits(ix), job.payload, job.gsel,
+                job.gseg, job.gsrc, job.pre_start, job.pre_cnt, nullptr, nullptr};
+    a.direct = ix.direct ? 1u : 0u;
+    return a;
 }
 
 uint64_t probe_prepare(Ctx *ctx, ProbeJob &job) {
@@ -802,8 +881,9 @@ uint64_t probe_prepare(Ctx *ctx, ProbeJob &job) {
         XH_CHECK_HIP(hipGetLastError());
     }
     scan_u64_inplace(ctx, job.toff.p, job.tiles, job.toff.p + job.tiles);
-    ctx->read_scalars(job.toff.p + job.tiles, 1);
+    ctx->read_scalars(job.toff.p + job.tiles, 1, job.also);
     job.total = ctx->host_scalars[0];
+    if (job.also && (job.also_value = ctx->host_scalars[1])) return job.total;  // the caller discards the job
     XH_REQUIRE(job.total < SCAN64_EXACT, XLOG_HIP_CAPACITY_OVERFLOW,
                "join probe: " + std::to_string(job.total) + " output rows");
     if (a.rec_cnt) {

@@ -451,7 +451,7 @@ __global__ __launch_bounds__(BS_TB) void k_bucket_sample(const uint64_t *__restr
     __shared__ BsSmem<BS_TB, BK_SAMPLE / BS_TB> sm;
     const uint32_t nb = 1u << bits;
     for (uint32_t i = threadIdx.x; i < nb; i += BS_TB) st->cursor[i] = 0;
-    if (threadIdx.x == 0) st->over = 0;
+    if (threadIdx.x == 0) st->over = st->pad = 0;
     const uint32_t ns = 8u << bits;
     const uint64_t step = n / ns;  // (over 512 keys a bucket)
     for (uint32_t i = threadIdx.x; i < ns; i += BS_TB)  // one key of each stretch, at a place of its own
