@@ -809,7 +809,7 @@ struct ChainRun {
                     Buf<uint64_t> alt(ctx, m);
                     swap_words(ctx, keys[p], m, c.pairs_t.p);
                     uint64_t *a = c.pairs_t.p, *b = alt.p;
-                    radix_sort_u64(ctx, &a, &b, nullptr, nullptr, m);
+                    radix_sort_u64(ctx, &a, &b, m);
                     if (a != c.pairs_t.p) std::swap(c.pairs_t.p, alt.p);
                     pairs = c.pairs_t.p;
                 }

@@ -293,17 +293,16 @@ void rel_free(xlog_hip_rel *r);
 // stream-ordered on ctx->stream.
 // ---------------------------------------------------------------------------
 
-// LSD radix sort of u64 keys with an optional u32 payload, stable, over the
-// 8-bit digits [digit_lo, digit_hi) (0..8 = the whole key; 4..8 = the high
-// word only).  On return *keys (and *vals) point at whichever of the two
-// buffers holds the result; the other is scratch.  The pass of the lowest
+// LSD radix sort of u64 keys, stable, over the 8-bit digits [digit_lo, digit_hi) (0..8 = the whole key; 4..8 = the high
+// word only).  On return *keys points at whichever of the two buffers holds
+// the result; the other is scratch.  The pass of the lowest
 // digit always runs (it is queued before the histograms are read back); every
 // higher digit that is constant over the input is skipped.  A keys-only sort
 // of the whole key over at least 2^22 keys instead waits for the histograms,
 // and when they predict that the high word leaves runs of a few keys, runs
 // the high word's passes and one sort_short_runs pass (the low word's passes
 // only if some run exceeds 256 keys).  Returns the number of passes executed.
-// With `src` (keys only) the first pass reads src and both buffers are
+// With `src` the first pass reads src and both buffers are
 // scratch, so an input that must not be modified is never copied first.
 // With known_digits (a bitmask of digits that may vary, e.g. from the value
 // domain) the passes are exactly those digits of [digit_lo, digit_hi) and the
@@ -344,8 +343,7 @@ bool sort_tickets();
 // With `whole` (a keys-only sort of the high word, digits 4..7, of at least
 // 2^22 keys) the sort may order the keys by the whole key instead, through the
 // segment route; *whole tells whether it did.
-int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **vals, uint32_t **vals_alt,
-                   uint64_t n, int digit_lo = 0, int digit_hi = 8, const uint64_t *src = nullptr,
+int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, int digit_lo = 0, int digit_hi = 8, const uint64_t *src = nullptr,
                    uint32_t known_digits = 0, SortUnique *uq = nullptr, bool *whole = nullptr);
 // A keys-only sort of a queued iteration: the key count on the device
 // (*d_n <= n_bound, the bound the launches are sized for), exactly the digit

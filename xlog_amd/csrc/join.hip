@@ -1340,8 +1340,7 @@ void sort_segments_long(Ctx *ctx, uint64_t *data, const uint64_t *seg, uint64_t 
         uint64_t *a = data + st;
         uint64_t *b = static_cast<uint64_t *>(ctx->alloc(len * sizeof(uint64_t)));
         uint64_t *k0 = a, *k1 = b;
-        uint32_t *v0 = nullptr, *v1 = nullptr;
-        radix_sort_u64(ctx, &k0, &k1, &v0, &v1, len, 0, 4);
+        radix_sort_u64(ctx, &k0, &k1, len, 0, 4);
         if (k0 != a) XH_CHECK_HIP(hipMemcpyAsync(a, k0, len * 8, hipMemcpyDeviceToDevice, ctx->stream));
         ctx->free(b);
     }

@@ -21,8 +21,7 @@
 //      word's digits take passes; k_sort_short_runs then orders every run of
 //      equal high word by its low word in one more pass (4 + 1 passes over
 //      uniform keys instead of 8).
-// Each pass reads and writes every key exactly once (16 B per key, plus the
-// optional u32 payload).  Tiles go to the XCDs in chunks of consecutive
+// Each pass reads and writes every key exactly once (16 B per key).  Tiles go to the XCDs in chunks of consecutive
 // tiles, so that neighbouring tiles share an L2, and a tile only ever waits
 // for tiles of earlier-dispatched blocks.
 #include "internal.hpp"
@@ -37,19 +36,12 @@ namespace {
 
 // Tile shapes: BLOCK threads (>= 256; threads 0..255 own one digit each in
 // the counting phase) x ITEMS keys per thread.  512x16 (8192 keys, 74 KB LDS,
-// 2 blocks per CU); key + payload sorts need LDS for the payload too, hence
-// a smaller tile.
+// 2 blocks per CU).
 #ifndef XH_SORT_BLOCK_K
 #define XH_SORT_BLOCK_K 512
 #endif
 #ifndef XH_SORT_ITEMS_K
 #define XH_SORT_ITEMS_K 16
-#endif
-#ifndef XH_SORT_BLOCK_V
-#define XH_SORT_BLOCK_V 256
-#endif
-#ifndef XH_SORT_ITEMS_V
-#define XH_SORT_ITEMS_V 16
 #endif
 #ifndef XH_SORT_LOOKBACK
 #define XH_SORT_LOOKBACK 4
@@ -57,9 +49,7 @@ namespace {
 constexpr int SORT_LOOKBACK = XH_SORT_LOOKBACK;
 
 constexpr int SORT_BLOCK_K = XH_SORT_BLOCK_K, SORT_ITEMS_K = XH_SORT_ITEMS_K;
-constexpr int SORT_BLOCK_V = XH_SORT_BLOCK_V, SORT_ITEMS_V = XH_SORT_ITEMS_V;
-static_assert(SORT_BLOCK_K >= 256 && SORT_BLOCK_K % 256 == 0 && SORT_BLOCK_V >= 256 && SORT_BLOCK_V % 256 == 0,
-              "digit phase needs 256 threads");
+static_assert(SORT_BLOCK_K >= 256 && SORT_BLOCK_K % 256 == 0, "digit phase needs 256 threads");
 constexpr uint32_t ST_AGG = 1u << 30;
 constexpr uint32_t ST_INC = 2u << 30;
 constexpr uint32_t ST_VAL = (1u << 30) - 1;
@@ -606,10 +596,9 @@ __device__ uint32_t tile_digit_count(const uint64_t *__restrict__ kin, uint64_t 
 // whose predecessor's block has not started (out-of-order dispatch, or fewer
 // co-resident blocks than a chunk group) only costs the waiting tile a read
 // of that predecessor, and under in-order dispatch the bound is never reached.
-template <bool HAS_VAL, int BLOCK, int ITEMS>
+template <int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) void k_onesweep(
-    const uint64_t *__restrict__ kin, uint64_t *__restrict__ kout, const uint32_t *__restrict__ vin,
-    uint32_t *__restrict__ vout, uint64_t n, uint32_t tiles, int shift, const uint32_t *__restrict__ digit_off,
+    const uint64_t *__restrict__ kin, uint64_t *__restrict__ kout, uint64_t n, uint32_t tiles, int shift, const uint32_t *__restrict__ digit_off,
     uint32_t *status, uint32_t *status_next, uint32_t chunk, unsigned long long *ticket,
     unsigned long long ticket_base, const uint64_t *d_n, const uint32_t *stop, uint32_t spin_limit) {
     __shared__ uint32_t s_wcnt[(BLOCK / WAVE)][256];
@@ -617,7 +606,6 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(
     __shared__ uint32_t s_gbase[256];
     __shared__ uint32_t s_wsum[(BLOCK / WAVE)];
     __shared__ uint64_t s_keys[(BLOCK * ITEMS)];
-    __shared__ uint32_t s_vals[HAS_VAL ? (BLOCK * ITEMS) : 1];
 
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid >> 6;
     const uint32_t lane_u = (uint32_t)lane;
@@ -666,14 +654,12 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(
         };
 
         uint64_t k[ITEMS];
-        uint32_t v[ITEMS];
         uint32_t rank[ITEMS];
 #pragma unroll
         for (int r = 0; r < ITEMS; ++r) {
             const uint64_t idx = wbase + (uint64_t)r * WAVE + lane;
             const bool valid = (uint32_t)lane < round_valid(r);
             k[r] = valid ? kin[idx] : 0ull;
-            if (HAS_VAL) v[r] = valid ? vin[idx] : 0u;
         }
         // Stable rank of each key among the wave's keys of equal digit, two
         // rounds at a time so that the two ballot chains interleave.  A lane's
@@ -764,7 +750,6 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(
                 const uint32_t dd = (uint32_t)(k[r] >> shift) & 255u;
                 const uint32_t pos = s_wcnt[wave][dd] + rank[r];
                 s_keys[pos] = k[r];
-                if (HAS_VAL) s_vals[pos] = v[r];
             }
         }
         if (digit_thread) {
@@ -825,7 +810,6 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(
             const uint64_t o = (uint64_t)s_gbase[dd] + i;
             if (o < n) {  // always true for a consistent histogram; keeps a bad one in bounds
                 kout[o] = key;
-                if (HAS_VAL) vout[o] = s_vals[i];
             }
         }
     }
@@ -966,13 +950,13 @@ static SortState &sort_state(Ctx *ctx, uint64_t tiles) {
 
 // Blocks of one digit pass kernel that the device holds at once (occupancy
 // queried once per process): the tile order needs 8 * chunk of them.
-template <bool HAS_VAL, int BLOCK, int ITEMS>
+template <int BLOCK, int ITEMS>
 static uint32_t pass_capacity(Ctx *ctx) {
     static std::atomic<int> per_cu{0};  // contexts on other threads may ask at the same time
     int b = per_cu.load(std::memory_order_relaxed);
     if (b == 0) {
         XH_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &b, reinterpret_cast<const void *>(&k_onesweep<HAS_VAL, BLOCK, ITEMS>), BLOCK, 0));
+            &b, reinterpret_cast<const void *>(&k_onesweep<BLOCK, ITEMS>), BLOCK, 0));
         if (b <= 0) b = 1;
         per_cu.store(b, std::memory_order_relaxed);
     }
@@ -1115,7 +1099,7 @@ int radix_sort_dev(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n_bo
     SortState &st = sort_state(ctx, tiles);
     uint32_t *hist = st.hist, *off = st.hist + 8 * 256;
     // persistent passes: at most the blocks the device holds, tickets from a counter zeroed per pass
-    const uint32_t cap = pass_capacity<false, SORT_BLOCK_K, SORT_ITEMS_K>(ctx);
+    const uint32_t cap = pass_capacity<SORT_BLOCK_K, SORT_ITEMS_K>(ctx);
     const unsigned grid = (unsigned)std::min<uint64_t>(tiles, cap);
     unsigned long long *tk = ctx->tickets + PERSIST_TICKET_SLOT + 1;
     fill_u32(ctx, hist, 0u, 8 * 256);
@@ -1143,8 +1127,8 @@ int radix_sort_dev(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n_bo
         const int nxt = 1 - cur;
         Prof prof(ctx, XLOG_HIP_KERNEL_SORT_PASS, 0.0);
         add_work_rows(ctx, prof.work(16.0), d_n, n_bound, 1, nullptr, 0, 0, nullptr, stop);
-        hipLaunchKernelGGL((k_onesweep<false, SORT_BLOCK_K, SORT_ITEMS_K>), dim3(grid), dim3(SORT_BLOCK_K), 0,
-                           ctx->stream, *keys, *keys_alt, nullptr, nullptr, n_bound, (uint32_t)tiles, 8 * dgt,
+        hipLaunchKernelGGL((k_onesweep<SORT_BLOCK_K, SORT_ITEMS_K>), dim3(grid), dim3(SORT_BLOCK_K), 0,
+                           ctx->stream, *keys, *keys_alt, n_bound, (uint32_t)tiles, 8 * dgt,
                            off + dgt * 256, st.status[cur], st.status[nxt], 1u, tk, 0ull, d_n, stop, sort_spin_limit());
         XH_CHECK_HIP(hipGetLastError());
         std::swap(*keys, *keys_alt);
@@ -1192,19 +1176,16 @@ bool block_sort_unique(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *out
     XH_CHECK_HIP(hipGetLastError());
     return true;
 }
-int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **vals, uint32_t **vals_alt,
-                   uint64_t n, int digit_lo, int digit_hi, const uint64_t *src, uint32_t known_digits,
+int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, int digit_lo, int digit_hi, const uint64_t *src, uint32_t known_digits,
                    SortUnique *uq, bool *whole) {
     if (whole) *whole = false;
     if (n < 2 || digit_lo >= digit_hi) {
         if (src && n) XH_CHECK_HIP(hipMemcpyAsync(*keys, src, n * 8, hipMemcpyDeviceToDevice, ctx->stream));
         return 0;
     }
-    XH_REQUIRE(!(src && vals && *vals), XLOG_HIP_INVALID_ARG, "radix sort: a separate source is keys-only");
     XH_REQUIRE(n < (1ull << 30), XLOG_HIP_CAPACITY_OVERFLOW,
                "radix sort: a single sort call is limited to 2^30 - 1 keys");
-    const bool has_val = vals && *vals;
-    if (!has_val && n <= BLOCK_SORT_KEYS && sort_block()) {
+    if (n <= BLOCK_SORT_KEYS && sort_block()) {
         const uint64_t *from = src ? src : *keys;
         Prof prof(ctx, XLOG_HIP_KERNEL_SORT_PASS, 16.0 * (double)n);
         if (digit_lo == 0 && digit_hi == 8)
@@ -1216,7 +1197,7 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **va
         XH_CHECK_HIP(hipGetLastError());
         return 1;
     }
-    if (!has_val && digit_lo == 0 && digit_hi == 8 && !known_digits && !uq && bucket_sort_takes(n)) {
+    if (digit_lo == 0 && digit_hi == 8 && !known_digits && !uq && bucket_sort_takes(n)) {
         Buf<uint64_t> st;
         bucket_sort(ctx, src ? src : *keys, n, *keys_alt, nullptr, st);
         ctx->read_scalars(st.p, 1);
@@ -1225,12 +1206,11 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **va
             return 2;
         }
     }
-    const uint64_t tile_keys = has_val ? (uint64_t)SORT_BLOCK_V * SORT_ITEMS_V : (uint64_t)SORT_BLOCK_K * SORT_ITEMS_K;
+    const uint64_t tile_keys = (uint64_t)SORT_BLOCK_K * SORT_ITEMS_K;
     const uint64_t tiles = (n + tile_keys - 1) / tile_keys;
     SortState &st = sort_state(ctx, tiles);
     uint32_t *hist = st.hist, *off = st.hist + 8 * 256;
-    const uint32_t cap = has_val ? pass_capacity<true, SORT_BLOCK_V, SORT_ITEMS_V>(ctx)
-                                 : pass_capacity<false, SORT_BLOCK_K, SORT_ITEMS_K>(ctx);
+    const uint32_t cap = pass_capacity<SORT_BLOCK_K, SORT_ITEMS_K>(ctx);
     // chunks of 8 consecutive tiles (4 and 16 measured alike, 1 and 2 slower),
     // at most 1/16 of the blocks the device holds, and smaller when a sort
     // has few tiles so that it still spreads over the XCDs
@@ -1244,9 +1224,9 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **va
     // the low word's only when a pass over a low digit is needed.
     // (a sort given known_digits takes exactly those passes, so it needs every digit's histogram)
     const bool hybrid_candidate =
-        !has_val && !known_digits && digit_lo == 0 && digit_hi == 8 && n >= HYBRID_MIN_KEYS && sort_hybrid();
+        !known_digits && digit_lo == 0 && digit_hi == 8 && n >= HYBRID_MIN_KEYS && sort_hybrid();
     // a sort of the high word that may order the keys by the whole key instead (the segment route)
-    const bool word_candidate = whole && !has_val && !known_digits && digit_lo == 4 && digit_hi == 8 &&
+    const bool word_candidate = whole && !known_digits && digit_lo == 4 && digit_hi == 8 &&
                                 n >= HYBRID_MIN_KEYS && sort_hybrid();
     auto histograms = [&](const uint64_t *from, int dlo, int dhi) {
         Prof prof(ctx, XLOG_HIP_KERNEL_SORT_HIST, 8.0 * (double)n);  // reads every key once
@@ -1271,7 +1251,7 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **va
             fill_u32(ctx, st.status[cur], 0u, st.dirty[cur] * 256);
             st.dirty[cur] = 0;
         }
-        Prof prof(ctx, XLOG_HIP_KERNEL_SORT_PASS, (has_val ? 24.0 : 16.0) * (double)n);
+        Prof prof(ctx, XLOG_HIP_KERNEL_SORT_PASS, 16.0 * (double)n);
         unsigned long long *tk = pass_tickets() ? ctx->tickets + 2 : nullptr;
         unsigned long long tb = tk ? ctx->take_tickets(2, grid) : 0ull;
         // tickets go to tiles in plain order (chunk 1: chunk_tile is then the identity), which measured
@@ -1289,21 +1269,14 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint32_t **va
             fill_u64(ctx, reinterpret_cast<uint64_t *>(ctx->tickets + 12), n, 1);
             pgrid = (unsigned)std::min<uint64_t>(tiles, cap);
         }
-        if (has_val)
-            hipLaunchKernelGGL((k_onesweep<true, SORT_BLOCK_V, SORT_ITEMS_V>), dim3(pgrid), dim3(SORT_BLOCK_V), 0,
-                               ctx->stream, *keys, *keys_alt, *vals, *vals_alt, n, (uint32_t)tiles, 8 * dgt,
-                               off + dgt * 256, st.status[cur], st.status[nxt], pchunk, tk, tb, pn, nullptr,
-                               sort_spin_limit());
-        else
-            hipLaunchKernelGGL((k_onesweep<false, SORT_BLOCK_K, SORT_ITEMS_K>), dim3(pgrid), dim3(SORT_BLOCK_K), 0,
-                               ctx->stream, (passes == 0 && src) ? src : *keys, *keys_alt, nullptr, nullptr, n,
+        hipLaunchKernelGGL((k_onesweep<SORT_BLOCK_K, SORT_ITEMS_K>), dim3(pgrid), dim3(SORT_BLOCK_K), 0,
+                               ctx->stream, (passes == 0 && src) ? src : *keys, *keys_alt, n,
                                (uint32_t)tiles, 8 * dgt, off + dgt * 256, st.status[cur], st.status[nxt], pchunk,
                                tk, tb, pn, nullptr, sort_spin_limit());
         XH_CHECK_HIP(hipGetLastError());
         st.dirty[cur] = tiles;
         if (st.dirty[nxt] <= tiles) st.dirty[nxt] = 0;
         std::swap(*keys, *keys_alt);
-        if (has_val) std::swap(*vals, *vals_alt);
         cur = nxt;
         ++passes;
     };
