@@ -859,12 +859,16 @@ static xlog_hip_rel *op_union_many(Ctx *ctx, const xlog_hip_rel *const *ins, uin
         total += ins[i]->rows;
     }
     if (arity <= 2 && n == 2 && (ins[0]->flags & ins[1]->flags & REL_CANONICAL)) {
-        uint64_t *m = static_cast<uint64_t *>(ctx->alloc((total ? total : 1) * sizeof(uint64_t)));
-        merge_sorted(ctx, ins[0]->w[0], ins[0]->rows, ins[1]->w[0], ins[1]->rows, m);
-        uint64_t *u;
-        uint64_t cnt = unique_keys(ctx, m, total, &u);
-        ctx->free(m);
-        return rel_adopt(ctx, arity, cnt, u, nullptr, REL_CANONICAL);
+        // Sets that share nothing (an iteration's new rows and the relation they were checked against) are united
+        // by the merge alone; the unique pass queued after it ends at once unless the merge found a shared key.
+        Owned m(ctx, alloc_keys(ctx, total)), u(ctx, alloc_keys(ctx, total));
+        if (total == 0) return rel_adopt(ctx, arity, 0, m.release(), nullptr, REL_CANONICAL);
+        Buf<uint64_t> res(ctx, 2);
+        merge_unique_sorted(ctx, ins[0]->w[0], ins[0]->rows, ins[1]->w[0], ins[1]->rows, m.p, u.p, res.p);
+        ctx->read_scalars(res.p, 2);
+        const bool apart = ctx->host_scalars[0] == 0;
+        const uint64_t cnt = apart ? total : ctx->host_scalars[1];
+        return rel_adopt(ctx, arity, cnt, apart ? m.release() : u.release(), nullptr, REL_CANONICAL);
     }
     xlog_hip_rel *cat = rel_new(ctx, arity, total);
     cat->rows = total;
@@ -886,7 +890,8 @@ static xlog_hip_rel *op_diff(Ctx *ctx, const xlog_hip_rel *a, const xlog_hip_rel
     canonical_keys(ctx, b, cb);
     uint64_t *o = static_cast<uint64_t *>(ctx->alloc((ca.n ? ca.n : 1) * sizeof(uint64_t)));
     Buf<uint64_t> cnt(ctx, 1);
-    select_unique_diff(ctx, ca.k, ca.n, cb.k, cb.n, o, cnt.p);
+    if (diff_by_merge_takes(ca.n, cb.n)) diff_by_merge(ctx, ca.k, ca.n, cb.k, cb.n, o, cnt.p);
+    else select_unique_diff(ctx, ca.k, ca.n, cb.k, cb.n, o, cnt.p);
     uint64_t n = read_count(ctx, cnt.p);
     return rel_adopt(ctx, a->arity, n, o, nullptr, REL_CANONICAL);
 }

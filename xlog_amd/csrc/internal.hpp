@@ -480,7 +480,20 @@ void merge_sorted(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *b, u
 // stop flag and a skip word: nothing is written when *stop is raised or
 // *skip is zero.
 void merge_sorted_dev(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *d_na, const uint64_t *b, uint64_t nb,
-                      const uint64_t *d_nb, uint64_t *out, const uint64_t *skip, const uint32_t *stop);
+                      const uint64_t *d_nb, uint64_t *out, const uint64_t *skip, const uint32_t *stop,
+                      unsigned long long *equal = nullptr);
+// The union of two sorted sets: their merge in out, and d_res[0] (device) the
+// number of keys they share.  When that is not zero the merge repeats those
+// keys, and uniq holds the d_res[1] unique ones (na + nb entries each);
+// otherwise the merge is the union and nothing is written to uniq.
+void merge_unique_sorted(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb, uint64_t *out,
+                         uint64_t *uniq, uint64_t *d_res);
+// The keys of the sorted set k that are not in the sorted set b, in order, by
+// the merge path of the two (select_unique_diff searches windows of b instead);
+// diff_by_merge_takes: the sizes for which that is faster.
+bool diff_by_merge_takes(uint64_t n, uint64_t nb);
+void diff_by_merge(Ctx *ctx, const uint64_t *k, uint64_t n, const uint64_t *b, uint64_t nb, uint64_t *out,
+                   uint64_t *d_count);
 
 // Sorted-run index over the high word of sorted packed keys (join build):
 // an open-addressing hash table of 16-byte slots mapping key -> (run start,

@@ -120,7 +120,8 @@ __global__ __launch_bounds__(SelShape<Sel>::block) void k_select(const uint64_t 
                                                       uint64_t *__restrict__ d_count, uint64_t *status,
                                                       uint64_t epoch_tag, unsigned long long *ticket,
                                                       unsigned long long ticket_base, uint64_t ntiles,
-                                                      const uint64_t *d_n, const uint32_t *stop) {
+                                                      const uint64_t *d_n, const uint32_t *stop,
+                                                      const uint64_t *only_if) {
     __shared__ uint64_t s_tile;
     __shared__ uint64_t s_prefix;
     constexpr int SEL_WAVES = SelShape<Sel>::waves;
@@ -143,6 +144,10 @@ __global__ __launch_bounds__(SelShape<Sel>::block) void k_select(const uint64_t 
         const uint64_t used = n ? (n + SEL_TILE - 1) / SEL_TILE : 1;
         ntiles = used < ntiles ? used : ntiles;
         if (blockIdx.x >= ntiles) return;  // more blocks than tiles: these take no ticket
+    }
+    if (only_if && *only_if == 0) {  // not wanted: one block takes all the launch's tickets, as the next one expects
+        if (blockIdx.x == 0 && tid == 0) atomicAdd(ticket, (unsigned long long)gridDim.x);
+        return;
     }
     for (;;) {
     if (tid == 0) s_tile = atomicAdd(ticket, 1ull) - ticket_base;
@@ -899,9 +904,9 @@ __global__ void k_merge_partition(const uint64_t *__restrict__ a, uint64_t na, c
 __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict__ a, uint64_t na,
                                                      const uint64_t *__restrict__ b, uint64_t nb,
                                                      const uint64_t *__restrict__ split, uint64_t *__restrict__ out,
-                                                     MergeDev dv) {
+                                                     MergeDev dv, unsigned long long *equal) {
     __shared__ uint64_t s[MRG_TILE];
-    __shared__ uint64_t s_split[2];
+    __shared__ uint64_t s_split[2], s_prev;
     const int tid = threadIdx.x;
     if (dv.off()) return;
     dv.counts(na, nb);
@@ -925,6 +930,7 @@ __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict_
     }
     const uint32_t la = (uint32_t)(a1 - a0), len = (uint32_t)(d1 - d0), lb = len - la;
     const uint64_t b0 = d0 - a0;
+    if (equal && tid == 0) s_prev = a0 ? a[a0 - 1] : 0ull;
     batched_copy<MRG_BLOCK, MRG_ITEMS>(
         len, tid, [&](uint32_t i) { return i < la ? a[a0 + i] : b[b0 + (i - la)]; },
         [&](uint32_t i, uint64_t v) { s[i] = v; });
@@ -932,7 +938,7 @@ __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict_
     const uint64_t *sa = s, *sb = s + la;
     uint32_t td = tid * MRG_ITEMS;
     uint64_t r[MRG_ITEMS];
-    uint32_t cnt = 0;
+    uint32_t cnt = 0, eq = 0;
     if (td < len) {
         uint32_t ia = (uint32_t)merge_path(sa, la, sb, lb, td);
         uint32_t ib = td - ia;
@@ -941,11 +947,14 @@ __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict_
             if (td + j < len) {
                 bool take_a = ib >= lb || (ia < la && sa[ia] <= sb[ib]);
                 r[j] = take_a ? sa[ia] : sb[ib];
+                // a key of b equal to one of a comes right after it
+                if (!take_a && (ia ? sa[ia - 1] == r[j] : (a0 && s_prev == r[j]))) ++eq;
                 ia += take_a; ib += !take_a;
                 ++cnt;
             }
         }
     }
+    if (equal && eq) atomicAdd(equal, (unsigned long long)eq);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < MRG_ITEMS; ++j)
@@ -954,6 +963,52 @@ __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict_
     for (uint32_t i = tid; i < len; i += MRG_BLOCK) out[d0 + i] = s[i];
     if (!persist) return;
     __syncthreads();  // s is reused by the next tile
+    }
+}
+
+// flags[i] = b[i] is not among a, over the merge-path tiles of a and b (both
+// sorted and unique): a tile's a keys and b keys are staged in LDS and each b
+// key is searched there, so every key of a is read once, streaming, whatever
+// window it falls in.  2^22 keys against 2^24 took 0.117 ms by windows (0.179
+// against 2^25, 0.37 against 2^27; 2^16 against 2^20 0.159), by merge 0.076
+// (0.112, 0.26; 0.031), reads of both arrays and all; from 64 keys of b per key
+// the windows, which read less of it, are level.
+__global__ __launch_bounds__(MRG_BLOCK) void k_merge_absent(const uint64_t *__restrict__ a, uint64_t na,
+                                                            const uint64_t *__restrict__ b, uint64_t nb,
+                                                            const uint64_t *__restrict__ split,
+                                                            uint8_t *__restrict__ flags) {
+    __shared__ uint64_t s[MRG_TILE];
+    __shared__ uint64_t s_split[2], s_prev;
+    const int tid = threadIdx.x;
+    const uint64_t total = na + nb, d0 = (uint64_t)blockIdx.x * MRG_TILE;
+    const uint64_t d1 = (d0 + MRG_TILE < total) ? d0 + MRG_TILE : total;
+    if (tid < 2) s_split[tid] = split[blockIdx.x + tid];
+    __syncthreads();
+    const uint64_t a0 = s_split[0];
+    uint64_t a1 = s_split[1];
+    {  // (as in k_merge)
+        const uint64_t lo1 = d1 > nb && d1 - nb > a0 ? d1 - nb : a0;
+        const uint64_t hi1 = a0 + (d1 - d0) < na ? a0 + (d1 - d0) : na;
+        a1 = a1 < lo1 ? lo1 : (a1 > hi1 ? hi1 : a1);
+    }
+    const uint32_t la = (uint32_t)(a1 - a0), len = (uint32_t)(d1 - d0), lb = len - la;
+    const uint64_t b0 = d0 - a0;
+    if (lb == 0) return;  // block-uniform
+    if (tid == 0) s_prev = a0 ? a[a0 - 1] : 0ull;
+    batched_copy<MRG_BLOCK, MRG_ITEMS>(
+        len, tid, [&](uint32_t i) { return i < la ? a[a0 + i] : b[b0 + (i - la)]; },
+        [&](uint32_t i, uint64_t v) { s[i] = v; });
+    __syncthreads();
+    for (uint32_t i = tid; i < lb; i += MRG_BLOCK) {
+        const uint64_t k = s[la + i];
+        uint32_t lo = 0, hi = la;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (s[mid] < k) lo = mid + 1; else hi = mid;
+        }
+        // (the equal key of a comes before k in the merge: in this tile, or the last one of the tiles before)
+        const bool found = (lo < la && s[lo] == k) || (lo == 0 && a0 && s_prev == k);
+        flags[b0 + i] = !found;
     }
 }
 
@@ -1381,7 +1436,8 @@ static uint64_t *select_status(Ctx *ctx, uint64_t tiles, uint64_t *epoch_tag) {
 // iteration; a raised flag makes the launch do nothing (*d_count unwritten).
 template <class Sel>
 static void run_select(Ctx *ctx, const uint64_t *in, uint64_t n, const Sel &sel, uint64_t *d_count,
-                       const uint64_t *d_n = nullptr, const uint32_t *stop = nullptr) {
+                       const uint64_t *d_n = nullptr, const uint32_t *stop = nullptr,
+                       const uint64_t *only_if = nullptr) {
     if (n == 0) {
         fill_u64(ctx, d_count, 0ull, 1);
         return;
@@ -1406,7 +1462,7 @@ static void run_select(Ctx *ctx, const uint64_t *in, uint64_t n, const Sel &sel,
     if (d_n) add_work_rows(ctx, prof.work(8.0), d_n, n, 1, nullptr, 0, 0, nullptr, stop);
     const size_t dyn = Sel::kWindow ? (size_t)WIN_CAP * sizeof(uint64_t) : 0;
     hipLaunchKernelGGL(k_select<Sel>, dim3(grid), dim3(SelShape<Sel>::block), dyn, ctx->stream, in, n, sel, d_count,
-                       status, tag, tk, tb, tiles, d_n, stop);
+                       status, tag, tk, tb, tiles, d_n, stop, only_if);
     XH_CHECK_HIP(hipGetLastError());
 }
 
@@ -1691,7 +1747,8 @@ void merge_sorted(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *b, u
     merge_sorted_dev(ctx, a, na, nullptr, b, nb, nullptr, out, nullptr, nullptr);
 }
 void merge_sorted_dev(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *d_na, const uint64_t *b, uint64_t nb,
-                      const uint64_t *d_nb, uint64_t *out, const uint64_t *skip, const uint32_t *stop) {
+                      const uint64_t *d_nb, uint64_t *out, const uint64_t *skip, const uint32_t *stop,
+                      unsigned long long *equal) {
     uint64_t total = na + nb;
     if (!total) return;
     uint64_t tiles = (total + MRG_TILE - 1) / MRG_TILE;
@@ -1715,8 +1772,28 @@ void merge_sorted_dev(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *
         return v ? (uint32_t)v : 32u;
     }();
     hipLaunchKernelGGL(k_merge, dim3(dev ? persistent_grid(ctx, tiles, merge_per_cu) : (unsigned)tiles), dim3(MRG_BLOCK), 0,
-                       ctx->stream, a, na, b, nb, split.p, out, dv);
+                       ctx->stream, a, na, b, nb, split.p, out, dv, equal);
     XH_CHECK_HIP(hipGetLastError());
+}
+void merge_unique_sorted(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb, uint64_t *out,
+                         uint64_t *uniq, uint64_t *d_res) {
+    fill_u64(ctx, d_res, 0ull, 2);
+    merge_sorted_dev(ctx, a, na, nullptr, b, nb, nullptr, out, nullptr, nullptr,
+                     reinterpret_cast<unsigned long long *>(d_res));
+    run_select(ctx, out, na + nb, SelUnique{out, uniq}, d_res + 1, nullptr, nullptr, d_res);
+}
+bool diff_by_merge_takes(uint64_t n, uint64_t nb) { return n >= (1ull << 12) && nb >= n / 2 && nb / 32 <= n; }
+void diff_by_merge(Ctx *ctx, const uint64_t *k, uint64_t n, const uint64_t *b, uint64_t nb, uint64_t *out,
+                   uint64_t *d_count) {
+    const uint64_t tiles = (n + nb + MRG_TILE - 1) / MRG_TILE;
+    XH_REQUIRE(tiles < (1ull << 31), XLOG_HIP_CAPACITY_OVERFLOW, "diff: input too large");
+    Buf<uint64_t> split(ctx, tiles + 1);
+    Buf<uint8_t> flags(ctx, n);
+    hipLaunchKernelGGL(k_merge_partition, dim3((unsigned)((tiles + 1 + 255) / 256)), dim3(256), 0, ctx->stream, b, nb, k, n,
+                       tiles, split.p, MergeDev{});
+    hipLaunchKernelGGL(k_merge_absent, dim3((unsigned)tiles), dim3(MRG_BLOCK), 0, ctx->stream, b, nb, k, n, split.p, flags.p);
+    XH_CHECK_HIP(hipGetLastError());
+    select_flags(ctx, k, flags.p, n, out, d_count);
 }
 
 void pack_columns(Ctx *ctx, const uint32_t *c0, const uint32_t *c1, uint64_t n, uint64_t *out) {
