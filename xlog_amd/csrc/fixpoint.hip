@@ -1622,6 +1622,33 @@ struct Driver {
                     "Recursive SCC iteration limit (" + std::to_string(max_iter) + ") exceeded"};
     }
 
+    // The closure of one relation, H(X,Z) :- E(X,Z) beside H(X,Z) :- H(X,Y), E(Y,Z) or E(X,Y), H(Y,Z), with H empty
+    // at the start: a walk from every source instead of run_hash's loop (closure_rows.hip).  false, with nothing
+    // done, for other plans, where its scratch is too large for the device and when it gave up.
+    bool run_rows(uint64_t max_iter, std::vector<uint64_t> &deltas, const std::vector<ChainRule> &chains,
+                  uint64_t *iterations) {
+        if (chains.size() != 2) return false;
+        const ChainRule &exit = chains[chains[0].path.size() == 1 ? 0 : 1], &rec = chains[&exit == &chains[0] ? 1 : 0];
+        if (exit.path.size() != 1 || rec.path.size() != 2 || exit.head != rec.head) return false;
+        const int h = exit.head, e = exit.path[0].pred;
+        const ChainAtom &a = rec.path[0], &b = rec.path[1];
+        if (idb[e] || full[h].n || exit.path[0].backward || a.backward || b.backward ||
+            !((a.pred == h && b.pred == e) || (a.pred == e && b.pred == h)) || !closure_rows_takes(ctx, full[e].n))
+            return false;
+        DRel f;
+        std::vector<uint64_t> layers;
+        f.k = closure_rows(ctx, full[e].k, full[e].n, index_of(full[e], 0).ix, max_iter, &f.n, layers);
+        if (!f.k) return false;
+        deltas = layers;
+        deltas.push_back(0);
+        *iterations = layers.size();
+        f.owned = true;
+        f.version = version_counter++;
+        release(full[h]);
+        full[h] = f;
+        return true;
+    }
+
     // The loop of run() over device hash sets, for path-shaped rules of at
     // most three atoms (chains[ri]: rule ri as a path from its first head
     // variable to its second).  The full relation of every IDB predicate also
@@ -2445,7 +2472,11 @@ static void run_fixpoint_impl(Ctx *ctx, const int32_t *plan, uint32_t n_preds, c
         }
         if (stats) stats->route = use_hash ? XLOG_HIP_ROUTE_HASH : XLOG_HIP_ROUTE_JOIN;  // also on failure
         try {
-            iterations = use_hash ? drv.run_hash(max_iter, deltas, paths) : drv.run(max_iter, deltas);
+            // (a call that asks for the hash route, or sets its sizes, gets its loop)
+            const bool rows = use_hash && route == XLOG_HIP_ROUTE_AUTO && !env_u64("XLOG_HIP_HASH_SLOTS", 0) &&
+                              !env_u64("XLOG_HIP_HASH_APPENDS", 0) && !env_u64("XLOG_HIP_HASH_QUEUE", 0);
+            if (!rows || !drv.run_rows(max_iter, deltas, paths, &iterations))
+                iterations = use_hash ? drv.run_hash(max_iter, deltas, paths) : drv.run(max_iter, deltas);
         } catch (const Error &) {
             reached = drv.cur_iter;
             throw;
