@@ -28,9 +28,9 @@ namespace xh {
 
 namespace {
 
-constexpr int CR_EDGES = 12;  // rows of E whose sources one wave walks together: about 8 sources at 1.5 rows each
-constexpr int CR_ROWS = 16;
-constexpr uint32_t CR_CAP1 = 448, CR_CAP2 = 1792, CR_CAP3 = 7168;  // pairs: 7/8 of the tiers' sets
+constexpr int CR_EDGES = 24;  // rows of E whose sources one wave walks together: about 16 sources at 1.5 rows each
+constexpr int CR_ROWS = 32;
+constexpr uint32_t CR_CAP1 = 896, CR_CAP2 = 1792, CR_CAP3 = 7168;  // pairs: 7/8 of the tiers' sets
 constexpr int CR_LAYERS = 4096;                                    // layers of the largest tier
 constexpr int CR_BINS = 32;                                        // copies of the layer counters
 constexpr uint64_t CR_EMPTY = ~0ull;                               // no pair is: its row is below CR_ROWS
@@ -76,27 +76,25 @@ __global__ __launch_bounds__(256) void k_cr_records(CrArgs a) {
 
 template <int SLOTS, int FR, int LV>
 struct CrLds {
-    unsigned long long set[SLOTS];  // row << 32 | target; compacted in place at the end
-    uint32_t fr[2][FR];             // up to four edges each: first edge << 6 | (edges - 1) << 4 | row
-    uint32_t nf[2], total, fail, packed, item;
+    // row << 32 | target; at the end the targets alone, a segment per row
+    alignas(16) unsigned long long set[SLOTS];
+    uint32_t fr[2][FR];  // the edges to follow: edge << 5 | row
+    uint32_t nf[2], total, fail, item;
     uint32_t row_n[CR_ROWS], src[CR_ROWS];
+    uint32_t row_at[CR_ROWS + 1], row_out[CR_ROWS];  // a row's segment (of whole quads) and place in the result
     uint32_t lev[LV];
 };
 
+// a run's edges to follow (all or, when they do not fit, none)
 template <int FR, class L>
 __device__ __forceinline__ void cr_push(L &l, int f, uint32_t row, uint32_t start, uint32_t len) {
-    const uint32_t np = (len + 3) / 4;
-    if (np > (uint32_t)FR) {
+    uint32_t p = FR;
+    if (len <= (uint32_t)FR) p = atomicAdd(&l.nf[f], len);
+    if (p + len > (uint32_t)FR) {
         l.fail = 1;
         return;
     }
-    const uint32_t p = atomicAdd(&l.nf[f], np);
-    if (p + np > (uint32_t)FR) {
-        l.fail = 1;
-        return;
-    }
-    for (uint32_t q = 0; q < np; ++q)
-        l.fr[f][p + q] = ((start + 4 * q) << 6) | ((min(len - 4 * q, 4u) - 1) << 4) | row;
+    for (uint32_t q = 0; q < len; ++q) l.fr[f][p + q] = ((start + q) << 5) | row;
 }
 
 // an empty walk (the caller pushes its first edges after the barrier)
@@ -105,7 +103,7 @@ __device__ __forceinline__ void cr_reset(L &l) {
     __syncthreads();
     for (int i = threadIdx.x; i < SLOTS; i += T) l.set[i] = CR_EMPTY;
     if (threadIdx.x < CR_ROWS) l.row_n[threadIdx.x] = 0;
-    if (threadIdx.x == 0) l.nf[0] = l.nf[1] = l.total = l.fail = l.packed = 0;
+    if (threadIdx.x == 0) l.nf[0] = l.nf[1] = l.total = l.fail = 0;
     __syncthreads();
 }
 
@@ -128,18 +126,15 @@ __device__ int cr_walk(L &l, const CrArgs &a, uint32_t cap) {
         prev = total;
         if (nf == 0) return lv;
         if (lv == LV) return -1;
-        for (uint32_t i = t; i < nf; i += T) {
-            const uint32_t f = l.fr[cur][i], start = f >> 6, n = ((f >> 4) & 3) + 1, row = f & 15;
-            uint64_t r[4];
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) r[u] = u < n ? a.rec[start + u] : 0ull;
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                if (u >= n) continue;
-                const uint32_t to = (uint32_t)(r[u] >> 32);
+        for (uint32_t base = 0; base < nf; base += T) {
+            bool novel = false;
+            if (base + t < nf) {
+                const uint32_t f = l.fr[cur][base + t], row = f & (CR_ROWS - 1);
+                const uint64_t r = a.rec[f >> 5];
+                const uint32_t to = (uint32_t)(r >> 32);
                 const unsigned long long key = ((unsigned long long)row << 32) | to;
                 uint32_t h = ((to ^ (row << 20)) * 0x9E3779B1u) >> (32 - __builtin_ctz(SLOTS));
-                bool novel = false, found = false;
+                bool found = false;
                 for (int p = 0; p < SLOTS && !found; ++p) {  // ends: a full table is a walk that does not fit
                     unsigned long long c = l.set[h];
                     if (c == CR_EMPTY) {
@@ -150,113 +145,121 @@ __device__ int cr_walk(L &l, const CrArgs &a, uint32_t cap) {
                     h = (h + 1) & (SLOTS - 1);
                 }
                 if (!found) l.fail = 1;
-                if (!novel) continue;
-                atomicAdd(&l.total, 1u);
-                atomicAdd(&l.row_n[row], 1u);
-                uint32_t len = (uint32_t)r[u] & 255u, first = (uint32_t)(r[u] >> 8) & 0xFFFFFFu;
-                if (len == 255u) len = cr_run(a, to, &first);
-                if (len) cr_push<FR>(l, cur ^ 1, row, first, len);
+                uint32_t len = (uint32_t)r & 255u, first = (uint32_t)(r >> 8) & 0xFFFFFFu;
+                if (novel && len) {
+                    if (len == 255u) len = cr_run(a, to, &first);
+                    cr_push<FR>(l, cur ^ 1, row, first, len);
+                }
             }
+            const uint32_t c = (uint32_t)__popcll(__ballot(novel));
+            if ((t & (WAVE - 1)) == 0 && c) atomicAdd(&l.total, c);
         }
         cur ^= 1;
     }
 }
 
-// The walk's pairs in order to out[0, n).
+// The walk's pairs in order to out[0, total): the targets row by row (the rows
+// ascend), and in a row each counts the smaller ones, four per LDS read.
 template <int T, int SLOTS, class L>
-__device__ void cr_write(L &l, uint32_t n, uint64_t *__restrict__ out) {
+__device__ void cr_write(L &l, uint64_t *__restrict__ out) {
     constexpr int R = SLOTS / T;
-    const int t = threadIdx.x, lane = t & (WAVE - 1);
+    const int t = threadIdx.x;
     unsigned long long k[R];
+    uint32_t at[R];
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < R; ++q) k[q] = l.set[q * T + t];
-    __syncthreads();
 #pragma unroll
-    for (int q = 0; q < R; ++q) {
-        const bool v = k[q] != CR_EMPTY;
-        const uint64_t m = __ballot(v);
-        uint32_t base = 0;
-        if (lane == 0 && m) base = atomicAdd(&l.packed, (uint32_t)__popcll(m));
-        base = __shfl(base, 0, WAVE);
-        if (v) l.set[base + __popcll(m & ((1ull << lane) - 1ull))] = k[q];
+    for (int q = 0; q < R; ++q) at[q] = k[q] != CR_EMPTY ? atomicAdd(&l.row_n[k[q] >> 32], 1u) : 0u;
+    __syncthreads();
+    if (t < WAVE) {
+        const uint32_t c = t < CR_ROWS ? l.row_n[t] : 0u, c4 = (c + 3) & ~3u;
+        uint32_t quads = c4, rows = c;
+#pragma unroll
+        for (int o = 1; o < CR_ROWS; o <<= 1) {
+            const uint32_t u = __shfl_up(quads, o, WAVE), v = __shfl_up(rows, o, WAVE);
+            if (t >= o) {
+                quads += u;
+                rows += v;
+            }
+        }
+        if (t < CR_ROWS) {
+            l.row_at[t + 1] = quads;
+            l.row_out[t] = rows - c;
+        }
+        if (t == 0) l.row_at[0] = 0;
     }
     __syncthreads();
+    uint32_t *seg = reinterpret_cast<uint32_t *>(l.set);
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+        if (k[q] != CR_EMPTY) seg[l.row_at[k[q] >> 32] + at[q]] = (uint32_t)k[q];
+    if (t < CR_ROWS)  // (all ones is smaller than no target)
+        for (uint32_t i = l.row_at[t] + l.row_n[t]; i < l.row_at[t + 1]; ++i) seg[i] = ~0u;
+    __syncthreads();
+    const uint32_t n = l.row_at[CR_ROWS];
     for (uint32_t i = t; i < n; i += T) {
-        const unsigned long long key = l.set[i];
+        int r = 0;  // the last row that begins at or before i and is not empty
+#pragma unroll
+        for (int s = CR_ROWS / 2; s > 0; s >>= 1)
+            if (l.row_at[r + s] <= i) r += s;
+        const uint32_t lo = l.row_at[r];
+        if (i - lo >= l.row_n[r]) continue;
+        const uint32_t to = seg[i], hi = l.row_at[r + 1];
         uint32_t rank = 0;
-#pragma unroll 8
-        for (uint32_t j = 0; j < n; ++j) rank += l.set[j] < key ? 1u : 0u;
-        out[rank] = ((uint64_t)l.src[key >> 32] << 32) | (uint32_t)key;
+#pragma unroll 4
+        for (uint32_t j = lo; j < hi; j += 4) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(seg + j);
+            rank += (v.x < to ? 1u : 0u) + (v.y < to ? 1u : 0u) + (v.z < to ? 1u : 0u) + (v.w < to ? 1u : 0u);
+        }
+        out[l.row_out[r] + rank] = ((uint64_t)l.src[r] << 32) | to;
     }
 }
 
-constexpr int CR_SLOTS1 = 512, CR_FR1 = 256, CR_LV1 = 64;
+constexpr int CR_SLOTS1 = 1024, CR_FR1 = 256, CR_LV1 = 128;
 __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
     __shared__ CrLds<CR_SLOTS1, CR_FR1, CR_LV1> l;
-    __shared__ uint32_t hist[CR_LV1];
     const int lane = threadIdx.x;
-    hist[lane] = 0;
-    const uint64_t nb = (a.m + CR_EDGES - 1) / CR_EDGES;
-    for (uint64_t b = blockIdx.x; b < nb; b += gridDim.x) {
-        const uint64_t e = b * CR_EDGES + lane;
-        const bool mine = lane < CR_EDGES && e < a.m;
-        const uint32_t src = mine ? (uint32_t)(a.edge[e] >> 32) : 0u;
-        const bool head = mine && (e == 0 || (uint32_t)(a.edge[e - 1] >> 32) != src);
-        if (__hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-        const uint64_t heads = __ballot(head);
-        const int rows = __popcll(heads);
-        const uint32_t row = __popcll(heads & ((1ull << lane) - 1ull));
-        uint32_t start = 0, len = 0;
-        if (head) len = cr_run(a, src, &start);
-        cr_reset<WAVE, CR_SLOTS1>(l);
-        if (head) {
-            l.src[row] = src;
-            cr_push<CR_FR1>(l, 0, row, start, len);
-        }
-        const int nl = cr_walk<WAVE, CR_SLOTS1, CR_FR1, CR_LV1>(l, a, CR_CAP1);
-        __syncthreads();
-        if (nl >= 0) {
-            uint32_t before = 0;
-            for (uint32_t r = 0; head && r < row; ++r) before += l.row_n[r];
-            if (mine) {
-                a.cnt[e] = head ? l.row_n[row] : 0u;
-                a.pos[e] = (uint32_t)(b * CR_CAP1) + before;
-            }
-            if (lane < nl) hist[lane] += l.lev[lane];
-            cr_write<WAVE, CR_SLOTS1>(l, l.total, a.scratch + b * CR_CAP1);
-            continue;
-        }
-        // together they do not fit: one source at a time, and those that do not fit alone are listed
-        if (mine && !head) a.cnt[e] = 0;
-        uint32_t used = 0;
-        for (int r = 0; r < rows; ++r) {
-            cr_reset<WAVE, CR_SLOTS1>(l);
-            const bool it = head && row == (uint32_t)r;
-            if (it) cr_push<CR_FR1>(l, 0, row, start, len);
-            const int n1 = cr_walk<WAVE, CR_SLOTS1, CR_FR1, CR_LV1>(l, a, CR_CAP1 - used);
-            __syncthreads();
-            if (n1 < 0) {
-                if (it) {
-                    const uint32_t i = atomicAdd(&a.ctl[1], 1u);
-                    if (i < a.list_cap[0])
-                        a.list[0][i] = (uint32_t)e;
-                    else
-                        a.ctl[0] = 1u;
-                }
-                continue;
-            }
-            const uint32_t n = l.total;
-            if (it) {
-                a.cnt[e] = n;
-                a.pos[e] = (uint32_t)(b * CR_CAP1) + used;
-            }
-            if (lane < n1) hist[lane] += l.lev[lane];
-            cr_write<WAVE, CR_SLOTS1>(l, n, a.scratch + b * CR_CAP1 + used);
-            used += n;
-        }
+    const uint64_t b = blockIdx.x, e = b * CR_EDGES + lane;
+    // the sources that begin in the batch's edges, the last one's run as far as the lanes see it
+    const bool mine = lane < CR_EDGES && e < a.m;
+    const uint32_t src = e < a.m ? (uint32_t)(a.edge[e] >> 32) : 0u;
+    const bool head = mine && (e == 0 || (uint32_t)(a.edge[e - 1] >> 32) != src);
+    if (__hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+    const uint64_t heads = __ballot(head);
+    const int row = __popcll(heads & ((2ull << min(lane, CR_EDGES - 1)) - 1ull)) - 1;  // -1: an earlier batch's
+    const uint32_t last_src = __shfl(src, CR_EDGES - 1, WAVE);
+    const bool walks = row >= 0 && e < a.m && (lane < CR_EDGES || src == last_src);
+    cr_reset<WAVE, CR_SLOTS1>(l);
+    if (head) l.src[row] = src;
+    if (walks) cr_push<CR_FR1>(l, 0, row, (uint32_t)e, 1);
+    if (walks && lane == WAVE - 1) {  // what lies past the lanes
+        uint32_t start = 0;
+        const uint32_t len = cr_run(a, src, &start);
+        cr_push<CR_FR1>(l, 0, row, (uint32_t)e + 1, len - ((uint32_t)e + 1 - start));
     }
-    if (hist[lane]) atomicAdd(&a.layers[lane * CR_BINS + blockIdx.x % CR_BINS], (unsigned long long)hist[lane]);
+    const int nl = cr_walk<WAVE, CR_SLOTS1, CR_FR1, CR_LV1>(l, a, CR_CAP1);
+    __syncthreads();
+    if (nl >= 0) {
+        for (int q = lane; q < nl; q += WAVE)
+            if (l.lev[q]) atomicAdd(&a.layers[q * CR_BINS + b % CR_BINS], (unsigned long long)l.lev[q]);
+        cr_write<WAVE, CR_SLOTS1>(l, a.scratch + b * CR_CAP1);
+        if (mine) {
+            a.cnt[e] = head ? l.row_n[row] : 0u;
+            a.pos[e] = (uint32_t)(b * CR_CAP1) + (head ? l.row_out[row] : 0u);
+        }
+        return;
+    }
+    // together they do not fit: each goes on the list
+    if (mine && !head) a.cnt[e] = 0;
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(&a.ctl[1], (uint32_t)__popcll(heads));
+    at = __shfl(at, 0, WAVE) + (uint32_t)row;
+    if (!head) return;
+    if (at < a.list_cap[0])
+        a.list[0][at] = (uint32_t)e;
+    else
+        a.ctl[0] = 1u;
 }
 
 // the listed sources, one at a time; those that do not fit go to the next
@@ -305,7 +308,7 @@ __global__ __launch_bounds__(T) void k_cr_walk_one(CrArgs a, uint32_t cap) {
         if (p == ~0u) continue;
         for (int q = threadIdx.x; q < nl; q += T)
             if (l.lev[q]) atomicAdd(&a.layers[q * CR_BINS + blockIdx.x % CR_BINS], (unsigned long long)l.lev[q]);
-        cr_write<T, SLOTS>(l, total, a.scratch + a.region + p);
+        cr_write<T, SLOTS>(l, a.scratch + a.region + p);
     }
 }
 
@@ -349,7 +352,7 @@ __global__ __launch_bounds__(256) void k_cr_gather(const uint64_t *__restrict__ 
 
 // device bytes closure_rows takes besides the result
 static uint64_t closure_rows_bytes(uint64_t m) {
-    return ((m + CR_EDGES - 1) / CR_EDGES * CR_CAP1 + 16 * m + 65536) * 8 + 17 * m + (1ull << 21);
+    return ((m + CR_EDGES - 1) / CR_EDGES * CR_CAP1 + 16 * m + 65536) * 8 + 21 * m + (1ull << 21);
 }
 
 bool closure_rows_takes(Ctx *ctx, uint64_t m) {
@@ -362,7 +365,7 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, const RunInde
                "closure rows: relation too large");
     const uint64_t nb = (m + CR_EDGES - 1) / CR_EDGES;
     const uint64_t region = nb * CR_CAP1, region_n = 16 * m + 65536;  // both below 2^32
-    const uint64_t cap2 = m / 32 + 64, cap3 = m / 512 + 64;
+    const uint64_t cap2 = m, cap3 = m / 512 + 64;
     Buf<uint64_t> rec(ctx, m), scratch(ctx, region + region_n), result(ctx, 2 + CR_LAYERS);
     Buf<uint32_t> off(ctx, m + 1), pos(ctx, m), list(ctx, cap2 + cap3);
     Buf<uint64_t> z(ctx, (uint64_t)CR_LAYERS * CR_BINS + 3);  // zeroed: layers, ctl, the scan's total
@@ -391,11 +394,11 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, const RunInde
     hipLaunchKernelGGL(k_cr_records, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, ctx->stream, a);
     {
         Prof prof(ctx, XLOG_HIP_KERNEL_HASH_INSERT, 16.0 * (double)m);  // the edges and their records, read once
-        hipLaunchKernelGGL(k_cr_walk, dim3((unsigned)std::min<uint64_t>(nb, 24 * cus)), dim3(WAVE), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_cr_walk, dim3((unsigned)nb), dim3(WAVE), 0, ctx->stream, a);
         XH_CHECK_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL((k_cr_walk_one<128, 2048, 512, 512, 1>), dim3((unsigned)std::min<uint64_t>(cap2, 6 * cus)),
-                       dim3(128), 0, ctx->stream, a, CR_CAP2);
+    hipLaunchKernelGGL((k_cr_walk_one<WAVE, 2048, 512, 512, 1>), dim3((unsigned)std::min<uint64_t>(cap2, 7 * cus)),
+                       dim3(WAVE), 0, ctx->stream, a, CR_CAP2);
     hipLaunchKernelGGL((k_cr_walk_one<512, 8192, 2048, CR_LAYERS, 2>), dim3((unsigned)std::min<uint64_t>(cap3, cus)),
                        dim3(512), 0, ctx->stream, a, CR_CAP3);
     XH_CHECK_HIP(hipGetLastError());
