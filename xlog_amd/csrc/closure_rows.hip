@@ -67,6 +67,7 @@ __device__ __forceinline__ uint32_t cr_run(const CrArgs &a, uint32_t key, uint32
 
 __global__ __launch_bounds__(256) void k_cr_records(CrArgs a) {
     const uint64_t e = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e == 0) a.cnt[a.m] = 0;  // the scan's last
     if (e >= a.m) return;
     const uint32_t to = (uint32_t)a.edge[e];
     uint32_t start = 0;
@@ -352,17 +353,27 @@ __global__ __launch_bounds__(256) void k_cr_gather(const uint64_t *__restrict__ 
 
 // device bytes closure_rows takes besides the result
 static uint64_t closure_rows_bytes(uint64_t m) {
-    return ((m + CR_EDGES - 1) / CR_EDGES * CR_CAP1 + 16 * m + 65536) * 8 + 21 * m + (1ull << 21);
+    return ((m + CR_EDGES - 1) / CR_EDGES * CR_CAP1 + 16 * m + 65536) * 8 + 97 * m + (1ull << 21);
 }
 
 bool closure_rows_takes(Ctx *ctx, uint64_t m) {
     return m >= 1 && m <= (1ull << 24) && closure_rows_bytes(m) <= device_room(ctx) / 4;
 }
 
-uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, const RunIndex &ix, uint64_t max_iter, uint64_t *n,
+uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_iter, uint64_t *n,
                        std::vector<uint64_t> &layers) {
-    XH_REQUIRE(m >= 1 && m <= (1ull << 24) && !ix.direct && ix.table_mask, XLOG_HIP_INVALID_ARG,
-               "closure rows: relation too large");
+    XH_REQUIRE(m >= 1 && m <= (1ull << 24), XLOG_HIP_INVALID_ARG, "closure rows: relation too large");
+    // the runs of E and their table, sized for m runs: no read-back
+    RunIndex ix;
+    RunScratch rs;
+    Buf<uint64_t> runs(ctx, 2);
+    fill_u64(ctx, runs.p + 1, m, 1);
+    build_run_index_async(ctx, edge, m, nullptr, rs, runs.p);
+    uint64_t slots = 1024;
+    while (slots < 2 * m) slots <<= 1;
+    ix.table = Buf<unsigned long long>(ctx, 2 * slots);
+    ix.table_mask = slots - 1;
+    run_index_insert_dev(ctx, rs.run_key.p, rs.run_start.p, runs.p, m, runs.p + 1, ix, nullptr);
     const uint64_t nb = (m + CR_EDGES - 1) / CR_EDGES;
     const uint64_t region = nb * CR_CAP1, region_n = 16 * m + 65536;  // both below 2^32
     const uint64_t cap2 = m, cap3 = m / 512 + 64;
@@ -370,7 +381,6 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, const RunInde
     Buf<uint32_t> off(ctx, m + 1), pos(ctx, m), list(ctx, cap2 + cap3);
     Buf<uint64_t> z(ctx, (uint64_t)CR_LAYERS * CR_BINS + 3);  // zeroed: layers, ctl, the scan's total
     fill_u64(ctx, z.p, 0ull, z.n);
-    fill_u32(ctx, off.p + m, 0u, 1);
     CrArgs a;
     a.edge = edge;
     a.m = m;

@@ -1637,7 +1637,7 @@ struct Driver {
             return false;
         DRel f;
         std::vector<uint64_t> layers;
-        f.k = closure_rows(ctx, full[e].k, full[e].n, index_of(full[e], 0).ix, max_iter, &f.n, layers);
+        f.k = closure_rows(ctx, full[e].k, full[e].n, max_iter, &f.n, layers);
         if (!f.k) return false;
         deltas = layers;
         deltas.push_back(0);

@@ -741,14 +741,13 @@ uint64_t closure_columns(Ctx *ctx, const uint64_t *edge, uint64_t m, const uint6
                          uint64_t *R, uint64_t *row_counts, std::vector<uint64_t> &layers);
 
 // The tuples of H(X,Z) :- E(X,Z).  H(X,Z) :- H(X,Y), E(Y,Z)  over any ids
-// (closure_rows.hip): E as m sorted unique packed pairs, ix its run index over
-// the first column.  Returns n sorted packed pairs (a pool block of the
-// caller's) and the new tuples of each iteration, E's own first, up to the
-// last non-empty one; nullptr (nothing done) when sources reach too much for
-// it or the iterations pass max_iter.  closure_rows_takes: the sizes it takes,
-// within the device's room.
+// (closure_rows.hip): E as m sorted unique packed pairs.  Returns n sorted
+// packed pairs (a pool block of the caller's) and the new tuples of each
+// iteration, E's own first, up to the last non-empty one; nullptr (nothing
+// done) when sources reach too much for it or the iterations pass max_iter.
+// closure_rows_takes: the sizes it takes, within the device's room.
 bool closure_rows_takes(Ctx *ctx, uint64_t m);
-uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, const RunIndex &ix, uint64_t max_iter, uint64_t *n,
+uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_iter, uint64_t *n,
                        std::vector<uint64_t> &layers);
 
 // Arrow IPC stream codec for relations of 1..4 UInt32 columns (arrow_ipc.cpp,
