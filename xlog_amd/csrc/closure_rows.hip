@@ -10,15 +10,20 @@
 // that grows with H is probed in memory and nothing of it is sorted there,
 // which is where the hash-set loop spends its time (2^20 vertices, 943,718
 // edges, 9.4 * 10^6 pairs, ids over 32 bits: 80 insert launches, two rehashes
-// and 8 passes of a sort, 4.24 ms).
+// and 8 passes of a sort, 4.24 ms whole; this takes 1.09 ms, 0.65 of them the
+// walks and 0.15 those of the listed sources).
 //
-// What bounds it is latency: a layer is one dependent read of E's records (8
-// bytes: target, and where the target's own run starts and how long it is) and
-// a few LDS accesses.  Hence one wave per workgroup, with a set small enough
-// for 24 of them on a CU.  Sources that reach more are listed and walked
-// by larger workgroups with larger sets; when they are many, or one of them
-// outgrows the largest set, the call gives up early and the caller goes on with
-// its loop over hash sets.
+// What bounds it is latency and the instructions of passes that few lanes take
+// part in: a layer is one dependent read of E's records (8 bytes: target, and
+// where the target's own run starts and how long it is) and a few LDS
+// accesses, for as many edges as the batch's sources have in that layer.  So a
+// lane takes one edge (four edges a lane, the batch half as large: 1.76 ms),
+// one wave is a workgroup with a set of 1,024 pairs, 15 of them on a CU, and a
+// batch is the largest that seldom outgrows it (32 edges: more sources listed,
+// the call 1.18 ms; 16: 1.17; 14 with sets of 512: 1.74).  The sources of a
+// batch that does not fit are listed and walked one by one with larger sets;
+// when they are many, or one of them outgrows the largest set, the attempt
+// ends early and the caller goes on with its loop over hash sets.
 #include "internal.hpp"
 #include "host.hpp"
 
