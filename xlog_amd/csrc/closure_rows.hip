@@ -36,6 +36,10 @@ namespace {
 constexpr int CR_EDGES = 24;  // rows of E whose sources one wave walks together: about 16 sources at 1.5 rows each
 constexpr int CR_ROWS = 32;
 constexpr uint32_t CR_CAP1 = 896, CR_CAP2 = 1792, CR_CAP3 = 7168;  // pairs: 7/8 of the tiers' sets
+// Sources listed up to batch b: at most CR_LISTED + b, one batch in 16 or so.  At 0.9 edges a vertex 1 % of the
+// batches are listed; at 0.95 a fifth would be, and the tiers after the first are then no faster than the hash loop
+// (2^20 vertices and as many edges: 18 ms in the second tier before it gave up, of a call of 83 ms without it).
+constexpr uint32_t CR_LISTED = 512;
 constexpr int CR_LAYERS = 4096;                                    // layers of the largest tier
 constexpr int CR_BINS = 32;                                        // copies of the layer counters
 constexpr uint64_t CR_EMPTY = ~0ull;                               // no pair is: its row is below CR_ROWS
@@ -50,6 +54,7 @@ struct CrArgs {
     uint64_t *scratch;
     uint32_t *cnt, *pos;  // per edge that begins a source: pairs, their place in scratch (cnt 0 at the others)
     unsigned long long *layers;  // [CR_LAYERS][CR_BINS]
+    unsigned long long *next;    // [CR_BINS] edges that follow an edge, over all edges
     uint32_t *ctl;               // give up, sources listed for tier 2, for tier 3, pairs of both in scratch
     uint32_t *list[2];
     uint32_t list_cap[2];
@@ -72,12 +77,18 @@ __device__ __forceinline__ uint32_t cr_run(const CrArgs &a, uint32_t key, uint32
 
 __global__ __launch_bounds__(256) void k_cr_records(CrArgs a) {
     const uint64_t e = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    uint32_t len = 0;
     if (e == 0) a.cnt[a.m] = 0;  // the scan's last
-    if (e >= a.m) return;
-    const uint32_t to = (uint32_t)a.edge[e];
-    uint32_t start = 0;
-    const uint32_t len = cr_run(a, to, &start);
-    a.rec[e] = ((uint64_t)to << 32) | ((uint64_t)start << 8) | min(len, 255u);
+    if (e < a.m) {
+        const uint32_t to = (uint32_t)a.edge[e];
+        uint32_t start = 0;
+        len = cr_run(a, to, &start);
+        a.rec[e] = ((uint64_t)to << 32) | ((uint64_t)start << 8) | min(len, 255u);
+    }
+    unsigned long long sum = len;
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, WAVE);
+    if ((threadIdx.x & (WAVE - 1)) == 0 && sum) atomicAdd(a.next + (blockIdx.x % CR_BINS), sum);
 }
 
 template <int SLOTS, int FR, int LV>
@@ -232,6 +243,16 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
     const uint32_t src = e < a.m ? (uint32_t)(a.edge[e] >> 32) : 0u;
     const bool head = mine && (e == 0 || (uint32_t)(a.edge[e - 1] >> 32) != src);
     if (__hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+    // The edges that follow an edge, on average: near one a walk hardly ends, above it most sources reach most of
+    // the graph.  From 15/16 the attempt ends here (at 0.95 the walks would take as long as the hash loop, and
+    // finding it out by the lists took 0.6 ms of 7.3 at 2^20 vertices, 0.36 of 1.8 at 20,000).
+    unsigned long long next = lane < CR_BINS ? a.next[lane] : 0ull;
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) next += __shfl_xor(next, o, WAVE);
+    if (16 * next >= 15 * a.m) {
+        if (b == 0 && lane == 0) a.ctl[0] = 1u;
+        return;
+    }
     const uint64_t heads = __ballot(head);
     const int row = __popcll(heads & ((2ull << min(lane, CR_EDGES - 1)) - 1ull)) - 1;  // -1: an earlier batch's
     const uint32_t last_src = __shfl(src, CR_EDGES - 1, WAVE);
@@ -262,7 +283,8 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
     if (lane == 0) at = atomicAdd(&a.ctl[1], (uint32_t)__popcll(heads));
     at = __shfl(at, 0, WAVE) + (uint32_t)row;
     if (!head) return;
-    if (at < a.list_cap[0])
+    // batches begin about in order, so a graph whose sources reach too much ends the attempt in its first batches
+    if (at < CR_LISTED + (uint32_t)b)
         a.list[0][at] = (uint32_t)e;
     else
         a.ctl[0] = 1u;
@@ -273,6 +295,7 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
 template <int T, int SLOTS, int FR, int LV, int TIER>
 __global__ __launch_bounds__(T) void k_cr_walk_one(CrArgs a, uint32_t cap) {
     __shared__ CrLds<SLOTS, FR, LV> l;
+    if (a.ctl[0]) return;  // by an earlier launch
     const uint32_t n = min(a.ctl[TIER], a.list_cap[TIER - 1]);
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
         cr_reset<T, SLOTS>(l);
@@ -358,7 +381,7 @@ __global__ __launch_bounds__(256) void k_cr_gather(const uint64_t *__restrict__ 
 
 // device bytes closure_rows takes besides the result
 static uint64_t closure_rows_bytes(uint64_t m) {
-    return ((m + CR_EDGES - 1) / CR_EDGES * CR_CAP1 + 16 * m + 65536) * 8 + 97 * m + (1ull << 21);
+    return ((m + CR_EDGES - 1) / CR_EDGES * CR_CAP1 + 16 * m + (1ull << 20)) * 8 + 93 * m + (1ull << 21);
 }
 
 bool closure_rows_takes(Ctx *ctx, uint64_t m) {
@@ -380,11 +403,11 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_
     ix.table_mask = slots - 1;
     run_index_insert_dev(ctx, rs.run_key.p, rs.run_start.p, runs.p, m, runs.p + 1, ix, nullptr);
     const uint64_t nb = (m + CR_EDGES - 1) / CR_EDGES;
-    const uint64_t region = nb * CR_CAP1, region_n = 16 * m + 65536;  // both below 2^32
-    const uint64_t cap2 = m, cap3 = m / 512 + 64;
+    const uint64_t region = nb * CR_CAP1, region_n = 16 * m + (1ull << 20);  // both below 2^32
+    const uint64_t cap2 = CR_LISTED + nb, cap3 = m / 4096 + 64;
     Buf<uint64_t> rec(ctx, m), scratch(ctx, region + region_n), result(ctx, 2 + CR_LAYERS);
     Buf<uint32_t> off(ctx, m + 1), pos(ctx, m), list(ctx, cap2 + cap3);
-    Buf<uint64_t> z(ctx, (uint64_t)CR_LAYERS * CR_BINS + 3);  // zeroed: layers, ctl, the scan's total
+    Buf<uint64_t> z(ctx, (uint64_t)(CR_LAYERS + 1) * CR_BINS + 3);  // zeroed: layers, next, ctl, the scan's total
     fill_u64(ctx, z.p, 0ull, z.n);
     CrArgs a;
     a.edge = edge;
@@ -397,14 +420,15 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_
     a.cnt = off.p;
     a.pos = pos.p;
     a.layers = reinterpret_cast<unsigned long long *>(z.p);
-    a.ctl = reinterpret_cast<uint32_t *>(z.p + (uint64_t)CR_LAYERS * CR_BINS);
+    a.next = a.layers + (uint64_t)CR_LAYERS * CR_BINS;
+    a.ctl = reinterpret_cast<uint32_t *>(a.next + CR_BINS);
     a.list[0] = list.p;
     a.list[1] = list.p + cap2;
     a.list_cap[0] = (uint32_t)cap2;
     a.list_cap[1] = (uint32_t)cap3;
     a.region = (uint32_t)region;
     a.region_n = (uint32_t)region_n;
-    unsigned long long *total = reinterpret_cast<unsigned long long *>(z.p + (uint64_t)CR_LAYERS * CR_BINS + 2);
+    unsigned long long *total = a.next + CR_BINS + 2;
     const unsigned cus = (unsigned)ctx->num_cus;
     hipLaunchKernelGGL(k_cr_records, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, ctx->stream, a);
     {
