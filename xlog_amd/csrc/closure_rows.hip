@@ -10,7 +10,7 @@
 // that grows with H is probed in memory and nothing of it is sorted there,
 // which is where the hash-set loop spends its time (2^20 vertices, 943,718
 // edges, 9.4 * 10^6 pairs, ids over 32 bits: 80 insert launches, two rehashes
-// and 8 passes of a sort, 4.24 ms whole; this takes 1.09 ms, 0.65 of them the
+// and 8 passes of a sort, 4.24 ms whole; this takes 1.10 ms, 0.65 of them the
 // walks and 0.15 those of the listed sources).
 //
 // What bounds it is latency and the instructions of passes that few lanes take
@@ -88,7 +88,21 @@ __global__ __launch_bounds__(256) void k_cr_records(CrArgs a) {
     unsigned long long sum = len;
 #pragma unroll
     for (int o = WAVE / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, WAVE);
-    if ((threadIdx.x & (WAVE - 1)) == 0 && sum) atomicAdd(a.next + (blockIdx.x % CR_BINS), sum);
+    __shared__ unsigned long long s_sum[4];
+    if ((threadIdx.x & (WAVE - 1)) == 0) s_sum[threadIdx.x / WAVE] = sum;
+    __syncthreads();
+    sum = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+    if (threadIdx.x == 0 && sum) atomicAdd(a.next + (blockIdx.x % CR_BINS), sum);
+}
+
+// The edges that follow an edge, on average: near one a walk hardly ends, above it most sources reach most of the
+// graph.  From 15/16 the attempt ends here (at 0.95 the walks would take as long as the hash loop, and finding it
+// out by the lists took 0.6 ms of 7.3 at 2^20 vertices, 0.36 of 1.8 at 20,000).
+__global__ __launch_bounds__(WAVE) void k_cr_gate(CrArgs a) {
+    unsigned long long next = threadIdx.x < CR_BINS ? a.next[threadIdx.x] : 0ull;
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) next += __shfl_xor(next, o, WAVE);
+    if (threadIdx.x == 0 && 16 * next >= 15 * a.m) a.ctl[0] = 1u;
 }
 
 template <int SLOTS, int FR, int LV>
@@ -243,16 +257,6 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
     const uint32_t src = e < a.m ? (uint32_t)(a.edge[e] >> 32) : 0u;
     const bool head = mine && (e == 0 || (uint32_t)(a.edge[e - 1] >> 32) != src);
     if (__hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-    // The edges that follow an edge, on average: near one a walk hardly ends, above it most sources reach most of
-    // the graph.  From 15/16 the attempt ends here (at 0.95 the walks would take as long as the hash loop, and
-    // finding it out by the lists took 0.6 ms of 7.3 at 2^20 vertices, 0.36 of 1.8 at 20,000).
-    unsigned long long next = lane < CR_BINS ? a.next[lane] : 0ull;
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) next += __shfl_xor(next, o, WAVE);
-    if (16 * next >= 15 * a.m) {
-        if (b == 0 && lane == 0) a.ctl[0] = 1u;
-        return;
-    }
     const uint64_t heads = __ballot(head);
     const int row = __popcll(heads & ((2ull << min(lane, CR_EDGES - 1)) - 1ull)) - 1;  // -1: an earlier batch's
     const uint32_t last_src = __shfl(src, CR_EDGES - 1, WAVE);
@@ -431,6 +435,7 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_
     unsigned long long *total = a.next + CR_BINS + 2;
     const unsigned cus = (unsigned)ctx->num_cus;
     hipLaunchKernelGGL(k_cr_records, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL(k_cr_gate, dim3(1), dim3(WAVE), 0, ctx->stream, a);
     {
         Prof prof(ctx, XLOG_HIP_KERNEL_HASH_INSERT, 16.0 * (double)m);  // the edges and their records, read once
         hipLaunchKernelGGL(k_cr_walk, dim3((unsigned)nb), dim3(WAVE), 0, ctx->stream, a);
