@@ -77,6 +77,18 @@ def test_gives_up(provider):
     _check(provider, rng.integers(0, 700, (1400, 2)))  # most sources reach most of it
 
 
+@pytest.mark.parametrize("small,large", [(40, 0), (40, 1), (40, 20), (0, 40)])
+def test_large_runs_among_the_listed_sources(provider, small, large):
+    """The largest sets' launch with many sources: runs that its frontier holds (up to 2,048 edges) and runs that it
+    refuses at their first push, when other workgroups of the launch are still starting and find the attempt ended."""
+    stars, first = [], 0
+    for k in range(small + large):
+        n = 600 + 30 * k if k < small else 2049 + 17 * k
+        stars.append(_star(first, first + 1, n))
+        first += n + 1
+    _check(provider, np.concatenate(stars[::2] + stars[1::2] + [_padding(first, 3000)]))
+
+
 def test_iteration_limit(provider):
     path = np.stack([np.arange(60), np.arange(1, 61)], 1)
     e = _spread(np.concatenate([path, _padding(61, 100)]))

@@ -61,6 +61,14 @@ struct CrArgs {
     uint32_t region, region_n;  // of scratch, for the listed sources
 };
 
+// the attempt's end: any block of a launch may raise it while others of the same launch are still starting
+__device__ __forceinline__ void cr_give_up(const CrArgs &a) {
+    __hip_atomic_store(a.ctl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint32_t cr_gave_up(const CrArgs &a) {
+    return __hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t cr_run(const CrArgs &a, uint32_t key, uint32_t *start) {
     uint64_t h = (uint64_t)(((uint64_t)key * 0x9E3779B97F4A7C15ull) >> (64 - a.bits));
@@ -102,7 +110,7 @@ __global__ __launch_bounds__(WAVE) void k_cr_gate(CrArgs a) {
     unsigned long long next = threadIdx.x < CR_BINS ? a.next[threadIdx.x] : 0ull;
 #pragma unroll
     for (int o = WAVE / 2; o > 0; o >>= 1) next += __shfl_xor(next, o, WAVE);
-    if (threadIdx.x == 0 && 16 * next >= 15 * a.m) a.ctl[0] = 1u;
+    if (threadIdx.x == 0 && 16 * next >= 15 * a.m) cr_give_up(a);
 }
 
 template <int SLOTS, int FR, int LV>
@@ -256,7 +264,7 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
     const bool mine = lane < CR_EDGES && e < a.m;
     const uint32_t src = e < a.m ? (uint32_t)(a.edge[e] >> 32) : 0u;
     const bool head = mine && (e == 0 || (uint32_t)(a.edge[e - 1] >> 32) != src);
-    if (__hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+    if (__builtin_amdgcn_readfirstlane((int)cr_gave_up(a))) return;  // (the workgroup is one wave)
     const uint64_t heads = __ballot(head);
     const int row = __popcll(heads & ((2ull << min(lane, CR_EDGES - 1)) - 1ull)) - 1;  // -1: an earlier batch's
     const uint32_t last_src = __shfl(src, CR_EDGES - 1, WAVE);
@@ -291,7 +299,7 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
     if (at < CR_LISTED + (uint32_t)b)
         a.list[0][at] = (uint32_t)e;
     else
-        a.ctl[0] = 1u;
+        cr_give_up(a);
 }
 
 // the listed sources, one at a time; those that do not fit go to the next
@@ -299,12 +307,16 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
 template <int T, int SLOTS, int FR, int LV, int TIER>
 __global__ __launch_bounds__(T) void k_cr_walk_one(CrArgs a, uint32_t cap) {
     __shared__ CrLds<SLOTS, FR, LV> l;
-    if (a.ctl[0]) return;  // by an earlier launch
+    // One thread reads whether the attempt has ended: blocks of this launch raise it, too, and waves that read it each
+    // for themselves could part, some leaving before the barriers that reset what the others go on to use.
+    if (threadIdx.x == 0) l.item = cr_gave_up(a);
+    __syncthreads();
+    if (l.item) return;
     const uint32_t n = min(a.ctl[TIER], a.list_cap[TIER - 1]);
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
         cr_reset<T, SLOTS>(l);
         if (threadIdx.x == 0) {
-            if (__hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) l.fail = 1;
+            if (cr_gave_up(a)) l.fail = 1;
             const uint32_t src = (uint32_t)(a.edge[a.list[TIER - 1][i]] >> 32);
             uint32_t start = 0;
             const uint32_t len = cr_run(a, src, &start);
@@ -320,7 +332,7 @@ __global__ __launch_bounds__(T) void k_cr_walk_one(CrArgs a, uint32_t cap) {
                 if (TIER == 1 && j < a.list_cap[1])
                     a.list[1][j] = e;
                 else
-                    a.ctl[0] = 1u;
+                    cr_give_up(a);
             }
             continue;
         }
@@ -333,7 +345,7 @@ __global__ __launch_bounds__(T) void k_cr_walk_one(CrArgs a, uint32_t cap) {
                 a.cnt[e] = total;
                 a.pos[e] = a.region + p;
             } else {
-                a.ctl[0] = 1u;
+                cr_give_up(a);
             }
         }
         __syncthreads();
