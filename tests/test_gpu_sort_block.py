@@ -51,13 +51,77 @@ def test_stable_by_column(provider, kind, n):
 @pytest.mark.parametrize("kind", ["hashed", "dense", "hub", "few", "equal"])
 @pytest.mark.parametrize("n", [16385, 32768, 32769, 100003, (1 << 20) - 1, 1 << 20, (1 << 20) + 1])
 def test_bucket_sort(provider, kind, n):
-    """The bucket sort at its size edges and where the number of buckets changes; a value with more repeats than a
-    bucket holds (few, equal) falls back to the digit passes."""
+    """The bucket sort at its size edges and where the number of buckets changes."""
     k = _keys(kind, n, np.random.default_rng(n))
     R = provider.create_buffer_from_packed(k)
     assert np.array_equal(provider.download_packed(provider.sort(R, [0, 1])), np.sort(k))
     assert np.array_equal(provider.download_packed(provider.dedup_full_row(R)), np.unique(k))
     assert np.array_equal(provider.download_packed(R), k)
+
+
+@pytest.fixture
+def launches(provider):
+    """A function giving the launches of each kernel kind in a call."""
+    def count(call):
+        provider.profile_enable(True)
+        try:
+            provider.profile_reset()
+            call()
+            return {k: v["launches"] for k, v in provider.profile_read().items()}
+        finally:
+            provider.profile_enable(False)
+    return count
+
+
+@pytest.mark.parametrize("kind", ["few", "equal", "equal 0", "equal ends", "hub", "hubs", "next to hubs"])
+@pytest.mark.parametrize("n", [20000, 100003, 1 << 20])
+def test_bucket_sort_repeats(provider, launches, kind, n):
+    """Values with more repeats than a bucket's region holds (4,096 keys) are sorted without digit passes."""
+    rng = np.random.default_rng(n)
+    top = (1 << 64) - 1
+    if kind == "equal 0":
+        k = np.zeros(n, dtype=np.uint64)
+    elif kind == "equal ends":
+        k = rng.choice(np.array([0, top], dtype=np.uint64), n)
+    elif kind in ("few", "equal"):
+        k = _keys(kind, n, rng)
+    else:  # among hashed keys: one value, four with the ends, and values whose neighbours are there, too
+        k = rng.integers(0, 1 << 64, n, dtype=np.uint64)
+        hubs = {"hub": [12345 << 30], "hubs": [0, 1 << 40, (1 << 40) + 1, top],
+                "next to hubs": [(5 << 40) + d for d in (-1, 0, 1)]}[kind]
+        at = rng.random(n) < 0.6
+        k[at] = rng.choice(np.array(hubs, dtype=np.uint64), int(at.sum()))
+    R = provider.create_buffer_from_packed(k)
+    out = {}
+    ran = launches(lambda: out.update(s=provider.sort(R, [0, 1]), d=provider.dedup_full_row(R)))
+    assert np.array_equal(provider.download_packed(out["s"]), np.sort(k))
+    assert np.array_equal(provider.download_packed(out["d"]), np.unique(k))
+    assert ran["sort_pass"] == 0 and ran["sort_segments"] == 2
+
+
+def _unlucky(k):
+    """The keys with the smallest one's repeats where the bucket sort takes its sample: one bucket gets the others."""
+    n = len(k)
+    bits = next(b for b in range(1, 32) if (n >> b) <= 1024)
+    i = np.arange(8 << bits, dtype=np.uint64)
+    step = np.uint64(n // (8 << bits))
+    at = i * step + (((i * np.uint64(0x9E3779B1)) & np.uint64(0xFFFFFFFF)) >> np.uint64(8)) % step
+    k = k.copy()
+    k[at] = k.min()
+    return k
+
+
+@pytest.mark.parametrize("n", [16385, 100003, 1 << 20])
+def test_bucket_sort_unlucky_sample(provider, launches, n):
+    """A bucket that outgrows its region: the digit passes sort the keys instead."""
+    k = _unlucky(np.random.default_rng(n).integers(0, 1 << 64, n, dtype=np.uint64))
+    R = provider.create_buffer_from_packed(k)
+    out = {}
+    ran = launches(lambda: out.update(s=provider.sort(R, [0, 1]), d=provider.dedup_full_row(R)))
+    assert np.array_equal(provider.download_packed(out["s"]), np.sort(k))
+    assert np.array_equal(provider.download_packed(out["d"]), np.unique(k))
+    assert np.array_equal(provider.download_packed(R), k)
+    assert ran["sort_pass"] > 0 and ran["sort_segments"] == 2
 
 
 @pytest.mark.parametrize("order", ["ascending", "descending", "runs"])
@@ -70,13 +134,19 @@ def test_bucket_sort_ordered_input(provider, order):
     assert np.array_equal(provider.download_packed(provider.dedup_full_row(R)), np.unique(k))
 
 
-def test_fixpoint_with_repeated_facts(provider):
-    """A relation whose buckets do not fit (one fact repeated 60,000 times) inside a program."""
+@pytest.mark.parametrize("unlucky", [False, True])
+def test_fixpoint_with_repeated_facts(provider, unlucky):
+    """One fact repeated 60,000 times inside a program, and one where the sample sees no other, so that the buckets do
+    not fit."""
     import oracle
     from xlog_amd import datagen, tc_plan
 
     s, d = datagen.random_digraph(3000, 4000, 5)
     e = np.concatenate([pack(s, d), np.full(60000, pack(s[:1], d[:1])[0], dtype=np.uint64)])
+    if unlucky:
+        e = np.roll(np.sort(np.tile(np.unique(e), 16)), 7)
+        e = _unlucky(e)
+        s, d = (e >> np.uint64(32)).astype(np.uint32), e.astype(np.uint32)
     outs, st = provider.fixpoint(tc_plan(), [provider.create_buffer_from_packed(e), None])
     ref = oracle.bfs_tc(3000, s, d)
     assert np.array_equal(provider.download_packed(outs[1]), ref["relation"]) and st["iterations"] == ref["iterations"]

@@ -264,7 +264,8 @@ __device__ __forceinline__ void block_sort(const uint64_t *in, uint32_t n, uint6
         uint32_t sum = 0;
         for (int w = 0; w < WAVES; ++w) sum += sm.part2[w];
         __syncthreads();
-        sorted = sum <= BLOCK_SORT_BIN * n;  // block-uniform
+        const bool exact = nlo + nhi <= BIN_BITS;  // a bin's keys are equal: nothing to rank
+        sorted = exact || sum <= BLOCK_SORT_BIN * n;  // block-uniform
         if (sorted) {
 #pragma unroll
             for (int q = 0; q < PER; ++q) {
@@ -278,30 +279,32 @@ __device__ __forceinline__ void block_sort(const uint64_t *in, uint32_t n, uint6
                 if ((uint32_t)r < rounds && i < n) sm.key[sm.bin[bin_of(k[r])] + slot[r]] = k[r];
             }
             __syncthreads();
-            uint32_t to[ITEMS];
+            if (!exact) {
+                uint32_t to[ITEMS];
 #pragma unroll
-            for (int r = 0; r < ITEMS; ++r) {
-                const uint32_t i = base + r * WAVE;
-                to[r] = 0;
-                if ((uint32_t)r < rounds && i < n) {
-                    k[r] = sm.key[i];
-                    const uint32_t b = bin_of(k[r]);
-                    const uint32_t lo = sm.bin[b], hi = b + 1 < BINS ? sm.bin[b + 1] : n;
-                    uint32_t rank = lo;
-                    for (uint32_t j = lo; j < hi; ++j) {
-                        const uint64_t x = sm.key[j];
-                        rank += (x < k[r] || (x == k[r] && j < i)) ? 1u : 0u;
+                for (int r = 0; r < ITEMS; ++r) {
+                    const uint32_t i = base + r * WAVE;
+                    to[r] = 0;
+                    if ((uint32_t)r < rounds && i < n) {
+                        k[r] = sm.key[i];
+                        const uint32_t b = bin_of(k[r]);
+                        const uint32_t lo = sm.bin[b], hi = b + 1 < BINS ? sm.bin[b + 1] : n;
+                        uint32_t rank = lo;
+                        for (uint32_t j = lo; j < hi; ++j) {
+                            const uint64_t x = sm.key[j];
+                            rank += (x < k[r] || (x == k[r] && j < i)) ? 1u : 0u;
+                        }
+                        to[r] = rank;
                     }
-                    to[r] = rank;
                 }
-            }
-            __syncthreads();
+                __syncthreads();
 #pragma unroll
-            for (int r = 0; r < ITEMS; ++r) {
-                const uint32_t i = base + r * WAVE;
-                if ((uint32_t)r < rounds && i < n) sm.key[to[r]] = k[r];
+                for (int r = 0; r < ITEMS; ++r) {
+                    const uint32_t i = base + r * WAVE;
+                    if ((uint32_t)r < rounds && i < n) sm.key[to[r]] = k[r];
+                }
+                __syncthreads();
             }
-            __syncthreads();
         }
     }
     if (!sorted) {
@@ -425,10 +428,14 @@ __global__ __launch_bounds__(BS_TB) void k_block_sort(const uint64_t *in, uint32
 // it (or its unique keys, gathered by a fourth launch), against a histogram and
 // up to eight passes of 9 to 20 us that leave most CUs idle at these sizes (a
 // dedup of 10^5 hashed pairs 145 -> 42 us, of 10^6 196 -> 89, of 10^6 pairs of
-// ids below 1,000 121 -> 84; the digit passes of 4 * 10^6 pairs are faster).  Bounds from a sample follow any distribution (hub ids included); only
-// one value's repeats, or a sample far off, can fill a bucket, which sets
-// `over`: the caller then takes the digit passes.  The buckets are filled in
-// arrival order (whole keys: it does not show).
+// ids below 1,000 121 -> 84; the digit passes of 4 * 10^6 pairs are faster).
+// Bounds from a sample follow any distribution.  A value with many repeats is
+// two bounds or more: the bucket between them holds that value alone and is
+// only counted, so it has no capacity (with the repeats in a region of 4,096
+// keys, a value with more of them cost the attempt: a dedup of 10^6 pairs of
+// which 60 % are one 320 us, by digit passes 207, so 134).  A sample far off
+// can fill another bucket, which sets `over`: the caller then takes the digit
+// passes.  The buckets are filled in arrival order (whole keys: it does not show).
 constexpr int BK_TB = 512, BK_ITEMS = 8, BK_KEYS = BK_TB * BK_ITEMS, BK_MAX_BITS = 10;
 constexpr uint32_t BK_SAMPLE = 8 << BK_MAX_BITS;  // eight keys per bucket: the fullest holds about 2.5 times the average
 struct BucketState {
@@ -436,6 +443,8 @@ struct BucketState {
     uint32_t cursor[1 << BK_MAX_BITS], uniq[1 << BK_MAX_BITS];  // keys, unique keys of each bucket
     uint64_t bound[1 << BK_MAX_BITS];  // bucket b holds the keys x with bound[b - 1] <= x < bound[b]
 };
+// bucket b holds one value, bound[b]: its bounds are equal (the last bound is the largest key)
+__device__ __forceinline__ bool bucket_of_one(const uint64_t *bound, uint32_t b) { return b > 0 && bound[b - 1] == bound[b]; }
 __global__ __launch_bounds__(BS_TB) void k_bucket_sample(const uint64_t *__restrict__ in, uint64_t n, BucketState *st,
                                                          int bits, uint64_t *__restrict__ sample) {
     __shared__ BsSmem<BS_TB, BK_SAMPLE / BS_TB> sm;
@@ -462,11 +471,13 @@ __global__ __launch_bounds__(BC_TB) void k_bucket_scatter(const uint64_t *__rest
     uint64_t k[BC_ITEMS];
 #pragma unroll
     for (int r = 0; r < BC_ITEMS; ++r) k[r] = base + r * BC_TB < n ? in[base + r * BC_TB] : 0ull;
+    int repeats = 0;  // some value is two bounds
     for (int i = tid; i < nb; i += BC_TB) {
         s_cnt[i] = 0;
         s_bound[i] = st->bound[i];
+        repeats |= bucket_of_one(st->bound, i) ? 1 : 0;
     }
-    __syncthreads();
+    repeats = __syncthreads_or(repeats);
     // the number of bounds <= the key (the last bound is no bound: every search ends below it)
     uint32_t b[BC_ITEMS], rank[BC_ITEMS];
 #pragma unroll
@@ -475,20 +486,41 @@ __global__ __launch_bounds__(BC_TB) void k_bucket_scatter(const uint64_t *__rest
 #pragma unroll
         for (int r = 0; r < BC_ITEMS; ++r) b[r] += s_bound[b[r] + step - 1] <= k[r] ? step : 0;
     }
+    uint32_t one = 0;  // bit r: key r goes to a bucket of one value
+    if (!repeats) {
 #pragma unroll
-    for (int r = 0; r < BC_ITEMS; ++r) rank[r] = base + r * BC_TB < n ? atomicAdd(&s_cnt[b[r]], 1u) : 0u;
+        for (int r = 0; r < BC_ITEMS; ++r) rank[r] = base + r * BC_TB < n ? atomicAdd(&s_cnt[b[r]], 1u) : 0u;
+    } else {
+        const int lane = tid & (WAVE - 1);
+#pragma unroll
+        for (int r = 0; r < BC_ITEMS; ++r) {
+            // (between two bounds equal to the key, not above them)
+            if (b[r] > 1 && s_bound[b[r] - 1] == k[r] && s_bound[b[r] - 2] == k[r]) --b[r];
+            const bool live = base + r * BC_TB < n, alone = live && bucket_of_one(s_bound, b[r]);
+            one |= alone ? 1u << r : 0u;
+            // of the wave's repeats, the first one's are counted in one addition
+            const uint64_t todo = __ballot(alone);
+            const int first = todo ? __ffsll((unsigned long long)todo) - 1 : 0;
+            const uint64_t same = __ballot(alone && b[r] == (uint32_t)__builtin_amdgcn_readlane((int)b[r], first));
+            const bool mine = (same >> lane) & 1ull;
+            rank[r] = 0;
+            if (live && (!mine || lane == first))
+                rank[r] = atomicAdd(&s_cnt[b[r]], mine ? (uint32_t)__popcll(same) : 1u);
+        }
+    }
     __syncthreads();
     for (int i = tid; i < nb; i += BC_TB)
         if (s_cnt[i]) {
             const uint32_t c = s_cnt[i], at = atomicAdd(&st->cursor[i], c);
-            if (at + c > (uint32_t)BK_KEYS) st->over = 1;
+            if (at + c > (uint32_t)BK_KEYS && !bucket_of_one(s_bound, i)) st->over = 1;
             s_cnt[i] = at;
         }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < BC_ITEMS; ++r) {
         const uint32_t at = s_cnt[b[r]] + rank[r];
-        if (base + r * BC_TB < n && at < (uint32_t)BK_KEYS) out[(uint64_t)b[r] * BK_KEYS + at] = k[r];
+        if (base + r * BC_TB < n && !((one >> r) & 1u) && at < (uint32_t)BK_KEYS)
+            out[(uint64_t)b[r] * BK_KEYS + at] = k[r];
     }
 }
 __device__ __forceinline__ uint32_t bucket_block_total(uint32_t v, uint32_t *part) {
@@ -509,21 +541,50 @@ __device__ __forceinline__ uint32_t bucket_block_total(uint32_t v, uint32_t *par
 template <bool UNIQUE>
 __global__ __launch_bounds__(BK_TB) void k_bucket_sort(uint64_t *regions, BucketState *st, uint64_t *__restrict__ out) {
     __shared__ BsSmem<BK_TB, BK_ITEMS> sm;
+    __shared__ uint32_t s_at, s_listed;
+    __shared__ uint3 s_list[UNIQUE ? 1 : BUCKET_SORT_KEYS / BK_KEYS];  // bucket, place, repeats
     const int tid = threadIdx.x;
     if (st->over) return;
     const uint32_t t = blockIdx.x, n = st->cursor[t];
     uint64_t *region = regions + (uint64_t)t * BK_KEYS;
     uint64_t k[BK_ITEMS];
-    if (n) block_sort<BK_TB, BK_ITEMS>(region, n, ~0ull, false, sm, k);  // block-uniform
+    const bool one = bucket_of_one(st->bound, t);  // block-uniform
+    if (n && !one) block_sort<BK_TB, BK_ITEMS>(region, n, ~0ull, false, sm, k);
     if (!UNIQUE) {
-        uint32_t before = 0;
-        for (uint32_t i = tid; i < t; i += BK_TB) before += st->cursor[i];
-        before = bucket_block_total(before, sm.part);
-        for (uint32_t i = tid; i < n; i += BK_TB) out[before + i] = sm.key[i];
+        // every bucket's place; values with more repeats than one workgroup should write are listed
+        constexpr int PER = (1 << BK_MAX_BITS) / BK_TB;
+        uint32_t c[PER], at = 0;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            c[q] = (uint32_t)(tid * PER + q) < gridDim.x ? st->cursor[tid * PER + q] : 0u;
+            at += c[q];
+        }
+        const uint32_t x = wave_incl_scan(at, tid & (WAVE - 1));
+        if ((tid & (WAVE - 1)) == WAVE - 1) sm.part[tid >> 6] = x;
+        if (tid == 0) s_listed = 0;
+        __syncthreads();
+        at = x - at;
+        for (int w = 0; w < tid >> 6; ++w) at += sm.part[w];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            if ((uint32_t)(tid * PER + q) == t) s_at = at;
+            if (c[q] > (uint32_t)BK_KEYS) s_list[atomicAdd(&s_listed, 1u)] = make_uint3(tid * PER + q, at, c[q]);
+            at += c[q];
+        }
+        __syncthreads();
+        if (n <= (uint32_t)BK_KEYS)
+            for (uint32_t i = tid; i < n; i += BK_TB) out[s_at + i] = one ? st->bound[t] : sm.key[i];
+        for (uint32_t i = 0; i < s_listed; ++i) {
+            const uint64_t v = st->bound[s_list[i].x];
+            for (uint32_t j = t * BK_TB + tid; j < s_list[i].z; j += gridDim.x * BK_TB) out[s_list[i].y + j] = v;
+        }
         return;
     }
     uint32_t total = 0;
-    if (n) {
+    if (n && one) {
+        if (tid == 0) region[0] = st->bound[t];
+        total = 1;
+    } else if (n) {
         uint64_t bal[BK_ITEMS];
         uint32_t pos;
         total = block_unique<BK_TB, BK_ITEMS>(n, sm, k, bal, &pos);
