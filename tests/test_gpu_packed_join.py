@@ -1,11 +1,12 @@
 """GPU parity of joins whose keys are packed into one u32 (their own slots, mixed, or too wide: the dictionaries) and of
-the small build sides (bucket sort, the fallback for a key with more rows than a bucket holds), against numpy: inner joins
-in left-row-major, right-row order, semi and anti joins as the left rows with and without a match."""
+the small build sides (bucket sort, keys with more rows than a bucket holds, the fallback where its sample misleads), against
+numpy: inner joins in left-row-major, right-row order, semi and anti joins as the left rows with and without a match."""
 from collections import defaultdict
 
 import numpy as np
 import pytest
 
+from test_gpu_sort_block import launches, unlucky  # noqa: F401  (launches: a fixture)
 from xlog_amd import JOIN_ANTI, JOIN_INNER, JOIN_SEMI
 
 pytestmark = pytest.mark.gpu
@@ -79,3 +80,27 @@ def test_hub_keys(provider, wide):
     right = [key] + _cols(rng, len(key), (1 << 32,) * (2 if wide else 1))
     left = [np.array([5, 6, 0xFFFFFFFF, 1 << 31, 7], np.uint32), np.arange(5, dtype=np.uint32)]
     _check(provider, left, right, [0], [0])
+
+
+@pytest.mark.parametrize("keys", [1, 2])
+@pytest.mark.parametrize("nr", [16385, 60000, 1 << 20])
+def test_unlucky_sample(provider, launches, keys, nr):
+    """A build side whose sample sees one key only: the index that was begun is dropped, and the second one sorts by
+    digit passes at once."""
+    rng = np.random.default_rng(nr)
+    one = unlucky(rng.integers(1, 250, nr).astype(np.uint32))
+    right = [one] + _cols(rng, nr, (200, 1 << 32) if keys == 2 else (1 << 32,))
+    left = [np.arange(0, 300, 7, dtype=np.uint32)] + _cols(rng, 43, (250,))
+    L, R = provider.create_buffer_from_u32_columns(left), provider.create_buffer_from_u32_columns(right)
+    on = list(range(keys))
+    ran = launches(lambda: provider.hash_join_v2(L, R, on, on, JOIN_INNER))
+    assert ran["sort_segments"] == 1 and ran["sort_pass"] > 0
+    if nr < 1 << 20:
+        _check(provider, left, right, on, on)
+    else:  # the pairs of left and right rows alone
+        out = provider.hash_join_v2(L, R, on, on, JOIN_INNER)
+        code = lambda cols: sum(c.astype(np.int64) << (16 * i) for i, c in enumerate(cols[:keys]))  # noqa: E731
+        order = np.argsort(code(right), kind="stable")
+        lo, hi = (np.searchsorted(code(right)[order], code(left), s) for s in ("left", "right"))
+        want = np.concatenate([order[a:b] for a, b in zip(lo, hi)])
+        assert np.array_equal(provider.download_column(out, len(left) + keys), right[keys][want])

@@ -99,7 +99,7 @@ def test_bucket_sort_repeats(provider, launches, kind, n):
     assert ran["sort_pass"] == 0 and ran["sort_segments"] == 2
 
 
-def _unlucky(k):
+def unlucky(k):
     """The keys with the smallest one's repeats where the bucket sort takes its sample: one bucket gets the others."""
     n = len(k)
     bits = next(b for b in range(1, 32) if (n >> b) <= 1024)
@@ -114,7 +114,7 @@ def _unlucky(k):
 @pytest.mark.parametrize("n", [16385, 100003, 1 << 20])
 def test_bucket_sort_unlucky_sample(provider, launches, n):
     """A bucket that outgrows its region: the digit passes sort the keys instead."""
-    k = _unlucky(np.random.default_rng(n).integers(0, 1 << 64, n, dtype=np.uint64))
+    k = unlucky(np.random.default_rng(n).integers(0, 1 << 64, n, dtype=np.uint64))
     R = provider.create_buffer_from_packed(k)
     out = {}
     ran = launches(lambda: out.update(s=provider.sort(R, [0, 1]), d=provider.dedup_full_row(R)))
@@ -134,8 +134,8 @@ def test_bucket_sort_ordered_input(provider, order):
     assert np.array_equal(provider.download_packed(provider.dedup_full_row(R)), np.unique(k))
 
 
-@pytest.mark.parametrize("unlucky", [False, True])
-def test_fixpoint_with_repeated_facts(provider, unlucky):
+@pytest.mark.parametrize("misled", [False, True])
+def test_fixpoint_with_repeated_facts(provider, misled):
     """One fact repeated 60,000 times inside a program, and one where the sample sees no other, so that the buckets do
     not fit."""
     import oracle
@@ -143,9 +143,9 @@ def test_fixpoint_with_repeated_facts(provider, unlucky):
 
     s, d = datagen.random_digraph(3000, 4000, 5)
     e = np.concatenate([pack(s, d), np.full(60000, pack(s[:1], d[:1])[0], dtype=np.uint64)])
-    if unlucky:
+    if misled:
         e = np.roll(np.sort(np.tile(np.unique(e), 16)), 7)
-        e = _unlucky(e)
+        e = unlucky(e)
         s, d = (e >> np.uint64(32)).astype(np.uint32), e.astype(np.uint32)
     outs, st = provider.fixpoint(tc_plan(), [provider.create_buffer_from_packed(e), None])
     ref = oracle.bfs_tc(3000, s, d)

@@ -1397,8 +1397,8 @@ __global__ void k_pack_rows(RelView in, KeyPack kp, uint64_t n, uint64_t *__rest
     }
 }
 // the payloads of sorted (key << 32) | row words: column c of the row, or the
-// row itself when c is negative (rows clamped: after a bucket sort that did not
-// fit, the words are anything)
+// row itself when c is negative (rows clamped: a bucket sort that did not fit
+// leaves words that are no rows)
 __global__ void k_row_payload(RelView in, int c, const uint64_t *__restrict__ sorted, uint64_t n,
                               uint32_t *__restrict__ payload) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -1444,11 +1444,12 @@ static KeyPack on_columns(const KeyPack &kp, const std::vector<int> &cols) {
 }
 
 // Run index over packed keys, each run's rows in input order, with payloads as
-// k_row_payload.  (key << 32) | row words are all different, so a whole-key sort
-// gives that order.  Small build sides are sorted by buckets and indexed with
-// nothing read back (the table is sized for as many runs as rows): *over then
-// points at a device word to be read with the probe's total, non-zero (low
-// half) when the sort did not fit and the index is to be built again without.
+// k_row_payload.  Small build sides are sorted by buckets, as whole words (they
+// are all different, so that gives that order), and indexed with nothing read
+// back (the table is sized for as many runs as rows): *over then points at a
+// device word to be read with the probe's total.  Its low half is not zero when
+// the sort did not fit (a sample far off: keys with many rows do fit); then the
+// index holds nothing and is to be built again without `small`.
 static void build_row_index(Ctx *ctx, const xlog_hip_rel *r, const KeyPack &kp, int payload_col, bool small,
                             JoinIndex &J, Buf<uint64_t> &state, const uint64_t **over) {
     const uint64_t n = r->rows;
@@ -1462,9 +1463,10 @@ static void build_row_index(Ctx *ctx, const xlog_hip_rel *r, const KeyPack &kp, 
         bucket_sort(ctx, rows.p, n, sorted.p, nullptr, state);
         rows.reset(sorted.release());
         *over = state.p;
+    } else if (n <= BLOCK_SORT_KEYS) {
+        rows.reset(sort_keys(ctx, rows.release(), n, true, 0, 8));
     } else {
-        // (a stable sort by the key, which reads its histograms back, above the bucket sort's sizes)
-        rows.reset(sort_keys(ctx, rows.release(), n, true, n <= BUCKET_SORT_KEYS ? 0 : 4, 8));
+        rows.reset(sort_keys(ctx, rows.release(), n, true, 4, 8));  // stable; digit passes
     }
     LAUNCH_1D(k_row_payload, n, view_of(r), payload_col, rows.p, n, J.payload.p);
     J.ix.direct = kp.bits < 32 && !kp.mix;
@@ -1481,7 +1483,9 @@ static void build_row_index(Ctx *ctx, const xlog_hip_rel *r, const KeyPack &kp, 
     J.ix.table = Buf<unsigned long long>(ctx, 2 * slots);
     J.ix.table_mask = slots - 1;
     J.ix.nruns = n;  // (a bound)
-    run_index_insert_dev(ctx, run_key.p, run_start.p, cnt.p, n, cnt.p + 1, J.ix, nullptr);
+    // (after a sort that did not fit, the runs are of words that repeat anyhow, and inserting those would probe on and on)
+    run_index_insert_dev(ctx, run_key.p, run_start.p, cnt.p, n, cnt.p + 1, J.ix,
+                         *over ? reinterpret_cast<const uint32_t *>(*over) : nullptr);
 }
 static bool small_build(uint64_t n) { return n <= BLOCK_SORT_KEYS || bucket_sort_takes(n); }
 
@@ -1503,7 +1507,7 @@ static uint64_t row_index_join(Ctx *ctx, const uint64_t *probe, uint64_t nl, int
         job.ix = &J.ix;
         job.payload = J.payload.p;
         const uint64_t total = probe_prepare(ctx, job);
-        if (job.also && (uint32_t)job.also_value) {  // a key with more rows than a bucket holds
+        if (job.also && (uint32_t)job.also_value) {  // a bucket outgrew its region
             small = false;
             continue;
         }

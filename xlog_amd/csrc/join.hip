@@ -106,13 +106,14 @@ __global__ void k_insert_dev(const uint32_t *__restrict__ run_key, const uint64_
 // runs come in key order, so their slots are written in order, with no atomic.
 __global__ void k_insert_direct(const uint32_t *__restrict__ run_key, const uint64_t *__restrict__ run_start,
                                 const uint64_t *d_nruns, uint64_t runs_bound, const uint64_t *d_n,
-                                unsigned long long *table, uint64_t mask) {
+                                unsigned long long *table, uint64_t mask, const uint32_t *stop) {
+    if (stop && *stop) return;
     const uint64_t nruns = *d_nruns < runs_bound ? *d_nruns : runs_bound, n = *d_n;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < nruns; r += stride) {
         const uint32_t key = run_key[r];
         const uint64_t st = run_start[r], en = r + 1 < nruns ? run_start[r + 1] : n;
-        if (key > mask) continue;  // (only in the words of a sort that did not fit)
+        if (key > mask) continue;  // (every key is below the table's size; keeps a bad one in bounds)
         *reinterpret_cast<u64x2 *>(table + 2 * (uint64_t)key) = u64x2{((unsigned long long)key << 32) | (en - st), st};
     }
 }
@@ -820,11 +821,10 @@ void run_index_insert_dev(Ctx *ctx, const uint32_t *run_key, const uint64_t *run
                           uint64_t runs_bound, const uint64_t *d_n, RunIndex &ix, const uint32_t *stop) {
     const uint64_t slots = ix.table_mask + 1;
     if (ix.direct) {
-        XH_REQUIRE(!stop, XLOG_HIP_INVALID_ARG, "run index: a direct table in a queued iteration");
         fill_u64(ctx, reinterpret_cast<uint64_t *>(ix.table.p), 0ull, 2 * slots);
         if (!runs_bound) return;
         hipLaunchKernelGGL(k_insert_direct, dim3(grid_for(runs_bound, 256, 16384)), dim3(256), 0, ctx->stream, run_key,
-                           run_start, d_nruns, runs_bound, d_n, ix.table.p, ix.table_mask);
+                           run_start, d_nruns, runs_bound, d_n, ix.table.p, ix.table_mask, stop);
         XH_CHECK_HIP(hipGetLastError());
         return;
     }
