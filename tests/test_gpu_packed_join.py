@@ -104,3 +104,25 @@ def test_unlucky_sample(provider, launches, keys, nr):
         lo, hi = (np.searchsorted(code(right)[order], code(left), s) for s in ("left", "right"))
         want = np.concatenate([order[a:b] for a, b in zip(lo, hi)])
         assert np.array_equal(provider.download_column(out, len(left) + keys), right[keys][want])
+
+
+@pytest.mark.parametrize("key", ["equal", "two", "hub", "collide"])
+@pytest.mark.parametrize("nr", [1, 1023, 1025, 40000, 600000])
+def test_key_set_of_repeats(provider, key, nr):
+    """Semi and anti joins against keys that most build rows share, with single rows of other keys among them."""
+    rng = np.random.default_rng(nr)
+    if key == "equal":
+        k = np.full(nr, 0xFFFFFFFF, dtype=np.uint32)
+    elif key == "two":
+        k = rng.choice(np.array([0, 77], np.uint32), nr)
+    elif key == "hub":
+        k = np.where(rng.random(nr) < 0.9, 5, rng.integers(0, 1 << 32, nr)).astype(np.uint32)
+    else:  # a few hundred keys in turn, so that the keys last seen change all the time
+        k = (np.arange(nr, dtype=np.uint32) * np.uint32(2654435761)) % np.uint32(499) * np.uint32(8192)
+    left = [np.concatenate([k[:: max(1, nr // 2000)], rng.integers(0, 1 << 32, 500, dtype=np.uint32)]).astype(np.uint32)]
+    left.append(np.arange(len(left[0]), dtype=np.uint32))
+    L, R = provider.create_buffer_from_u32_columns(left), provider.create_buffer_from_u32_columns([k, k])
+    hit = np.isin(left[0], k)
+    for kind, keep in ((JOIN_SEMI, hit), (JOIN_ANTI, ~hit)):
+        out = provider.hash_join_v2(L, R, [0], [0], kind)
+        assert np.array_equal(provider.download_column(out, 1), left[1][keep])
