@@ -1487,7 +1487,13 @@ static void build_row_index(Ctx *ctx, const xlog_hip_rel *r, const KeyPack &kp, 
     run_index_insert_dev(ctx, run_key.p, run_start.p, cnt.p, n, cnt.p + 1, J.ix,
                          *over ? reinterpret_cast<const uint32_t *>(*over) : nullptr);
 }
-static bool small_build(uint64_t n) { return n <= BLOCK_SORT_KEYS || bucket_sort_takes(n); }
+// One key column: up to 3 * 2^17 rows.  Beyond, the digit passes, few when the keys have few bits, and a table sized by
+// the runs found take less (10^6 rows a side, by buckets and by digit passes: Zipf keys 213 / 157 us, 1,000 keys 162 /
+// 117, ids 208 / 196, hashed 272 / 275; 4 * 10^5 rows: 153 / 138, 108 / 106, 131 / 143, 158 / 187).  Keys packed from
+// several columns have most of 31 bits: buckets as far as they go (10^6 rows on ids and a column of 64 values 294 / 327).
+static bool small_build(uint64_t n, int key_cols) {
+    return n <= BLOCK_SORT_KEYS || ((key_cols > 1 || n <= (3ull << 17)) && bucket_sort_takes(n));
+}
 
 // INNER join of non-empty inputs: probe words of the left side (l's own rows
 // with their key in word pcol, or packed ones) against the row index of r, the
@@ -1495,7 +1501,7 @@ static bool small_build(uint64_t n) { return n <= BLOCK_SORT_KEYS || bucket_sort
 static uint64_t row_index_join(Ctx *ctx, const uint64_t *probe, uint64_t nl, int pcol, const xlog_hip_rel *r,
                                const KeyPack &kp, int payload_col, int out_arity, const int oc[4], Buf<uint64_t> &o0,
                                Buf<uint64_t> &o1) {
-    bool small = small_build(r->rows);
+    bool small = small_build(r->rows, kp.n);
     for (;;) {
         JoinIndex J;
         Buf<uint64_t> state;
@@ -1592,7 +1598,7 @@ static xlog_hip_rel *op_join(Ctx *ctx, const xlog_hip_rel *l, const xlog_hip_rel
     const int pcol = probe_vidx(l->arity, lk);
     if ((type == XLOG_HIP_JOIN_SEMI || type == XLOG_HIP_JOIN_ANTI) && l->rows && r->rows)
         return key_set_join(ctx, l, l->w[0], pcol, r->w[0], r->rows, probe_vidx(r->arity, rk), type, false);
-    if (type == XLOG_HIP_JOIN_INNER && l->rows && small_build(r->rows) &&
+    if (type == XLOG_HIP_JOIN_INNER && l->rows && small_build(r->rows, 1) &&
         !((r->flags & REL_CANONICAL) && r->arity == 2 && rk == 0)) {  // (those are in key order already)
         int oc[4] = {0, 0, 0, 0};
         const int out_arity = join_values(l, r->arity, rk, out_cols, oc);
