@@ -69,6 +69,40 @@ def test_run_lengths(provider, run):
     _check(provider, [c[rng.permutation(n)] if i else c for i, c in enumerate(cols)], [0, 1, 2, 3])
 
 
+def _hashed(rng, n, distinct):
+    """A column of 32-bit values, `distinct` of them (0: any)."""
+    if not distinct:
+        return rng.integers(0, 1 << 32, n).astype(np.uint32)
+    return rng.choice(rng.integers(0, 1 << 32, distinct), n).astype(np.uint32)
+
+
+# distinct values of each column: the first has few, all have few, a first that hardly splits the rows
+@pytest.mark.parametrize("distinct", [(3, 0, 0), (100, 0, 0, 0), (20, 20, 20, 20), (1, 0, 5, 0), (2, 2, 2, 0, 2, 2),
+                                      (7, 7, 7, 7, 7, 7, 7, 7), (50, 1000, 3, 1000)])
+@pytest.mark.parametrize("n", [16384, 16385, 70001, (1 << 20) + 3])
+def test_long_runs(provider, distinct, n):
+    """Runs of equal prefix that are sorted again by the key's next bits, once or several times, and those that go by
+    pieces of the whole key."""
+    rng = np.random.default_rng(n)
+    _check(provider, [_hashed(rng, n, d) for d in distinct], list(range(len(distinct))))
+
+
+@pytest.mark.parametrize("share", [0.001, 0.1, 0.9, 1.0])
+def test_hub_among_short_runs(provider, share):
+    """The rows of one value are sorted again and the others stay where the first sort put them."""
+    n = 200003
+    rng = np.random.default_rng(9)
+    cols = [_hashed(rng, n, 0) for _ in range(4)]
+    cols[0][rng.random(n) < share] = 0xFFFFFFFF
+    cols[1][rng.random(n) < 0.3] = 0
+    src, dst = rng.integers(0, n, n // 4), rng.integers(0, n, n // 4)
+    for c in cols:
+        c[dst] = c[src]
+    _check(provider, cols, [0, 1, 2, 3])
+    _check(provider, cols, [0, 3])
+    _check(provider, cols[:3], [0, 2, 1])
+
+
 @pytest.mark.parametrize("n", [(1 << 20) + 7, (1 << 22) + 1])
 def test_large(provider, n):
     _check(provider, _rows(np.random.default_rng(5), n, 3, "ties"), [0, 1, 2])

@@ -4,6 +4,7 @@
 #include "host.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <array>
 #include <chrono>
 #include <cerrno>
@@ -388,7 +389,7 @@ std::vector<Bags> bags_per_pred(Ctx *ctx, uint32_t n) {
 // digit_lo / digit_hi restrict the sort to 8-bit digits [lo, hi) (4..8 = by
 // the high word only, stable otherwise).
 uint64_t *sort_keys(Ctx *ctx, uint64_t *keys, uint64_t n, bool keys_owned, int digit_lo, int digit_hi,
-                    uint32_t known_digits, bool *whole) {
+                    uint32_t known_digits, bool *whole, int in_order) {
     if (whole) *whole = false;
     // a consumed input is freed if an error unwinds from here
     Owned in_guard(ctx, keys_owned ? keys : nullptr);
@@ -405,7 +406,7 @@ uint64_t *sort_keys(Ctx *ctx, uint64_t *keys, uint64_t n, bool keys_owned, int d
         uint64_t *a = ga.p, *b = gb.p;
         // without keys_owned the first pass reads the caller's keys; both ping-pong buffers are ours
         radix_sort_u64(ctx, &a, &b, n, digit_lo, digit_hi, keys_owned ? nullptr : keys, known_digits,
-                       nullptr, whole);
+                       nullptr, whole, in_order);
         ga.release();
         gb.release();
         ctx->free(b);
@@ -541,52 +542,50 @@ static void canonical_keys(Ctx *ctx, const xlog_hip_rel *r, Canon &c) {
 // equal prefix in input order.  Then one pass fetches the rows in that order
 // (from a copy that holds a row's words together: one line a row, where word
 // arrays cost one each), orders each run of equal prefix by the rest of the key
-// when the prefix does not hold all of it, and writes rows and group flags.  A
-// run of more than RUN_MAX rows leaves it incomplete: the key is then taken in
-// pieces of prefix length from its low end, one sort each.
+// when the prefix does not hold all of it, and writes rows and group flags.
+// Runs of more than RUN_MAX rows it leaves out.  Their rows alone are sorted
+// again, by (run, the key's next bits, row's number), and so on.  Where that
+// would go on for long (most rows, runs that each bit splits little), the whole
+// key is taken in pieces from its low end instead, one stable sort of (piece,
+// row's number) each, by the piece's digits.
 // (Dedup of 10^7 rows of four columns, 86 bits: four key + payload sorts with
-// their gathers 2.3 ms, one prefix sort and this pass, 0.24 of it, 0.73.)
+// their gathers 2.3 ms, one prefix sort and this pass, 0.24 of it, 0.73.  Four
+// hashed columns, 128 bits: 2.60 / 0.72 ms; the first with a value that a tenth
+// of the rows have 2.60 / 1.47, with 100 values in all 2.59 / 2.02.  What gains
+// nothing are hashed columns of a few values each, where 40 bits of the key tell
+// as little as 10: 20 values in each 2.47 / 2.80, 10^6 rows 0.54 / 0.82.)
 // ---------------------------------------------------------------------------
 struct KeyBits {
     int n = 0, total = 0;
     int col[MAX_ARITY] = {0}, len[MAX_ARITY] = {0};  // distinct columns, bits they use
+    bool known = true;                               // (or may use)
 };
-struct KeyPiece {  // bits [lo, lo + bits) of the number, at the top of 64; the row's number below them
+struct KeyPiece {  // bits [lo, lo + bits) of the number, at the top of 64; the row's number in row_bits from row_shift up
     int n = 0, bits = 0;
     int col[MAX_ARITY] = {0}, rs[MAX_ARITY] = {0}, ls[MAX_ARITY] = {0};
     uint32_t mask[MAX_ARITY] = {0};
     int row_bits = 0, row_shift = 0;
 };
 namespace {
-// with aos: the row's W words together; with perm: of row perm[i] (and i for the row's number)
+// with aos: the row's W words together; with prev: of the rows that those words number (from prev_shift up); with
+// group: the group's number (group[i + 1] - 1) above the piece
 template <int W>
-__global__ __launch_bounds__(256) void k_key_pieces(RelView in, KeyPiece kp, const uint32_t *__restrict__ perm, uint64_t n,
-                                                    uint64_t *__restrict__ out, uint64_t *__restrict__ aos) {
+__global__ __launch_bounds__(256) void k_key_pieces(RelView in, KeyPiece kp, uint64_t n, uint64_t *__restrict__ out,
+                                                    uint64_t *__restrict__ aos, const uint64_t *__restrict__ prev,
+                                                    int prev_shift, const uint32_t *__restrict__ group, int group_bits) {
     const uint64_t stride = (uint64_t)gridDim.x * 256;
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
-        const uint64_t r = perm ? perm[i] : i;
-        uint64_t w = i << kp.row_shift;
+        const uint64_t r = prev ? (prev[i] >> prev_shift) & ((1ull << kp.row_bits) - 1) : i;
+        uint64_t w = r << kp.row_shift;
         for (int t = 0; t < kp.n; ++t)
             w |= (uint64_t)((col_value(in, kp.col[t], r) >> kp.rs[t]) & kp.mask[t]) << kp.ls[t];
+        if (group) w |= (uint64_t)(group[i + 1] - 1) << (64 - group_bits);
         out[i] = w;
         if (aos) {
 #pragma unroll
             for (int q = 0; q < W; ++q) aos[i * W + q] = in.w[q][r];
         }
     }
-}
-// out[i] = the row of sorted piece i (through perm when given)
-__global__ void k_piece_rows(const uint64_t *__restrict__ sorted, KeyPiece kp, const uint32_t *__restrict__ perm, uint64_t n,
-                             uint32_t *__restrict__ out) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const uint32_t r = (uint32_t)(sorted[i] >> kp.row_shift) & (uint32_t)((1ull << kp.row_bits) - 1);
-        out[i] = perm ? perm[r] : r;
-    }
-}
-__global__ void k_key_of_rows(const uint32_t *__restrict__ perm, uint64_t n, int shift, uint64_t *__restrict__ out) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) out[i] = (uint64_t)perm[i] << shift;
 }
 constexpr int ROWS_TB = 512, ROWS_TILE = 1024, RUN_MAX = 64;
 // -1, 0, 1: the key columns of row a against those of row b
@@ -600,11 +599,13 @@ __device__ __forceinline__ int compare_rows(const uint64_t *a, const uint64_t *b
     return 0;
 }
 // A tile takes the runs of equal prefix that start in it (ties: they are ordered
-// by the whole key; otherwise the order is final and a run is only a group).
+// by the whole key, and long ones left out; otherwise the order is final and a
+// run is only a group).  With pos, row i of the order goes to place pos[i].
 template <int W>
 __global__ __launch_bounds__(ROWS_TB) void k_sorted_rows(const uint64_t *__restrict__ sorted, KeyPiece kp, uint64_t n,
                                                          const uint64_t *__restrict__ aos, KeyBits kb, int arity, int ties,
-                                                         RelOut out, uint8_t *__restrict__ flags, uint64_t *d_long) {
+                                                         RelOut out, uint8_t *__restrict__ flags, uint64_t *d_long,
+                                                         const uint32_t *__restrict__ pos) {
     constexpr int SPAN = ROWS_TILE + RUN_MAX + 1;  // (one past the longest run shows its end)
     __shared__ uint64_t s_key[SPAN];
     __shared__ uint64_t s_row[SPAN * W];
@@ -639,9 +640,10 @@ __global__ __launch_bounds__(ROWS_TB) void k_sorted_rows(const uint64_t *__restr
         for (int q = 0; q < LD; ++q) {
             const int i = q * ROWS_TB + tid;
             if (i >= own) continue;
+            const uint64_t o = pos ? pos[base + i] : base + i;
 #pragma unroll
-            for (int j = 0; j < W; ++j) out.w[j][base + i] = row[q][j];
-            if (flags) flags[base + i] = i ? s_key[i] != s_key[i - 1] : (base == 0 || s_key[0] != before);
+            for (int j = 0; j < W; ++j) out.w[j][o] = row[q][j];
+            if (flags) flags[o] = i ? s_key[i] != s_key[i - 1] : (base == 0 || s_key[0] != before);
         }
         return;
     }
@@ -654,7 +656,7 @@ __global__ __launch_bounds__(ROWS_TB) void k_sorted_rows(const uint64_t *__restr
         int e = i + 1;
         while (e < len && s_key[e] == k && e - a <= RUN_MAX) ++e;
         if (e - a > RUN_MAX) {
-            *d_long = 1;
+            if ((uint32_t)__ffsll((unsigned long long)__ballot(true)) - 1 == (threadIdx.x & (WAVE - 1))) *d_long = 1;
             continue;
         }
         int rank = 0, same = 0;
@@ -664,10 +666,43 @@ __global__ __launch_bounds__(ROWS_TB) void k_sorted_rows(const uint64_t *__restr
             rank += (c < 0 || (c == 0 && j < i)) ? 1 : 0;
             same |= (c == 0 && j < i) ? 1 : 0;
         }
-        const uint64_t o = base + a + rank;
+        const uint64_t o = pos ? pos[base + a + rank] : base + a + rank;
 #pragma unroll
         for (int j = 0; j < W; ++j) out.w[j][o] = s_row[i * W + j];
         if (flags) flags[o] = !same;
+    }
+}
+// in_long[i] = 1 for the sorted words whose run of equal prefix has more than RUN_MAX (in_long[n] = 0: n + 1 entries)
+__global__ void k_long_runs(const uint64_t *__restrict__ sorted, KeyPiece kp, uint64_t n, uint32_t *__restrict__ in_long) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    const int shift = 64 - kp.bits;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i <= n; i += stride) {
+        uint32_t is_long = 0;
+        if (i < n) {
+            const uint64_t k = sorted[i] >> shift;
+            uint64_t lo = i > (uint64_t)RUN_MAX ? i - RUN_MAX : 0, hi = i;  // the run's first, as far back as matters
+            while (lo < hi) {
+                const uint64_t mid = (lo + hi) >> 1;
+                if ((sorted[mid] >> shift) == k) hi = mid; else lo = mid + 1;
+            }
+            is_long = lo + RUN_MAX < n && (sorted[lo + RUN_MAX] >> shift) == k;
+        }
+        in_long[i] = is_long;
+    }
+}
+// the words of long runs (in_long: scanned) with their places, and head = 1 where a run begins (m + 1 entries)
+__global__ void k_long_take(const uint64_t *__restrict__ sorted, KeyPiece kp, uint64_t n,
+                            const uint32_t *__restrict__ in_long, const uint32_t *__restrict__ pos,
+                            uint64_t *__restrict__ out, uint32_t *__restrict__ out_pos, uint32_t *__restrict__ head) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    const int shift = 64 - kp.bits;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        const uint32_t q = in_long[i];
+        if (i == 0) head[in_long[n]] = 0;
+        if (in_long[i + 1] == q) continue;
+        out[q] = sorted[i];
+        out_pos[q] = pos ? pos[i] : (uint32_t)i;
+        head[q] = i == 0 || (sorted[i] >> shift) != (sorted[i - 1] >> shift);
     }
 }
 }  // namespace
@@ -677,6 +712,11 @@ static KeyBits key_bits(Ctx *ctx, const xlog_hip_rel *in, const std::vector<int>
     KeyBits kb;
     for (int c : cols)
         if (std::find(kb.col, kb.col + kb.n, c) == kb.col + kb.n) kb.col[kb.n++] = c;
+    if (kb.n == 1 && in->nwords() == 1) {  // the sort's own histograms tell as much
+        kb.len[0] = kb.total = 32;
+        kb.known = false;
+        return kb;
+    }
     Buf<unsigned long long> used(ctx, MAX_WORDS);
     fill_u64(ctx, reinterpret_cast<uint64_t *>(used.p), 0ull, MAX_WORDS);
     hipLaunchKernelGGL(k_key_bits, dim3(grid_for(in->rows, 256 * 8, 256), in->nwords()), dim3(256), 0, ctx->stream,
@@ -691,11 +731,12 @@ static KeyBits key_bits(Ctx *ctx, const xlog_hip_rel *in, const std::vector<int>
     }
     return kb;
 }
-static KeyPiece key_piece(const KeyBits &kb, int lo, int bits, uint64_t n) {
+// (above: bits that the caller puts above the piece)
+static KeyPiece key_piece(const KeyBits &kb, int lo, int bits, uint64_t n, int above = 0) {
     KeyPiece kp;
-    kp.bits = bits;
+    kp.bits = above + bits;
     while (kp.row_bits < 31 && (1ull << kp.row_bits) < n) ++kp.row_bits;
-    kp.row_shift = 64 - bits - kp.row_bits;
+    kp.row_shift = 64 - kp.bits - kp.row_bits;
     int at = kb.total;  // bit above the column
     for (int t = 0; t < kb.n; ++t) {
         at -= kb.len[t];
@@ -704,23 +745,30 @@ static KeyPiece key_piece(const KeyBits &kb, int lo, int bits, uint64_t n) {
         kp.col[kp.n] = kb.col[t];
         kp.rs[kp.n] = a - at;
         kp.mask[kp.n] = b - a == 32 ? 0xFFFFFFFFu : (1u << (b - a)) - 1u;
-        kp.ls[kp.n++] = 64 - bits + (a - lo);
+        kp.ls[kp.n++] = 64 - kp.bits + (a - lo);
     }
     return kp;
 }
-template <int W>
-static void key_pieces(Ctx *ctx, const xlog_hip_rel *in, const KeyPiece &kp, const uint32_t *perm, uint64_t *out,
-                       uint64_t *aos) {
-    LAUNCH_1D(k_key_pieces<W>, in->rows, view_of(in), kp, perm, in->rows, out, aos);
-}
-// the piece keys of all rows, sorted (they are all different; digits below the row's number hold zeros or are in order)
-template <int W>
-static uint64_t *sorted_pieces(Ctx *ctx, const xlog_hip_rel *in, const KeyPiece &kp, const uint32_t *perm, uint64_t *aos) {
-    const uint64_t n = in->rows;
-    Owned w(ctx, alloc_keys(ctx, n));
-    key_pieces<W>(ctx, in, kp, perm, w.p, aos);
-    const bool whole = n <= BUCKET_SORT_KEYS || n >= (1ull << 22);
-    return sort_keys(ctx, w.release(), n, true, whole ? 0 : std::min(7, (64 - kp.bits) / 8), 8);
+// The long runs of an order by kp's words (sorted, n of them, places pos or
+// their own): their words, places and group numbers (one more than each, in
+// group[1 ..]).  Returns their number.
+struct LongRuns {
+    Buf<uint64_t> words;
+    Buf<uint32_t> pos, group;
+    uint64_t n = 0, groups = 0;
+};
+static void long_runs(Ctx *ctx, const uint64_t *sorted, const KeyPiece &kp, uint64_t n, const uint32_t *pos, LongRuns &out) {
+    Buf<uint32_t> in_long(ctx, n + 1);
+    Buf<unsigned long long> sum(ctx, 1);
+    LAUNCH_1D(k_long_runs, n + 1, sorted, kp, n, in_long.p);
+    scan_u32_inplace(ctx, in_long.p, n + 1, sum.p);
+    out.n = read_count(ctx, reinterpret_cast<const uint64_t *>(sum.p));
+    out.words = Buf<uint64_t>(ctx, out.n);
+    out.pos = Buf<uint32_t>(ctx, out.n);
+    out.group = Buf<uint32_t>(ctx, out.n + 1);
+    LAUNCH_1D(k_long_take, n, sorted, kp, n, in_long.p, pos, out.words.p, out.pos.p, out.group.p);
+    scan_u32_inplace(ctx, out.group.p, out.n + 1, sum.p);
+    out.groups = read_count(ctx, reinterpret_cast<const uint64_t *>(sum.p));
 }
 // Rows of `in` sorted by kb's columns (stable).  With flags: 1 for the first row
 // of every group of rows equal on those columns.
@@ -731,33 +779,65 @@ static xlog_hip_rel *sorted_rows(Ctx *ctx, const xlog_hip_rel *in, const KeyBits
     o->rows = n;
     KeyPiece kp = key_piece(kb, 0, 0, n);
     const int room = 64 - kp.row_bits;
-    const bool ties = kb.total > room;
-    kp = key_piece(kb, ties ? kb.total - room : 0, ties ? room : kb.total, n);
+    int left = std::max(0, kb.total - room);  // bits of the key below the prefix
+    kp = key_piece(kb, left, kb.total - left, n);
     Buf<uint64_t> aos(ctx, W > 1 ? n * W : 0), d_long(ctx, 1);
-    Owned w(ctx, sorted_pieces<W>(ctx, in, kp, nullptr, W > 1 ? aos.p : nullptr));
     const uint64_t *rows = W > 1 ? aos.p : in->w[0];
-    const dim3 grid((unsigned)((n + ROWS_TILE - 1) / ROWS_TILE));
-    if (ties) fill_u64(ctx, d_long.p, 0ull, 1);
-    hipLaunchKernelGGL(k_sorted_rows<W>, grid, dim3(ROWS_TB), 0, ctx->stream, w.p, kp, n, rows, kb, (int)in->arity,
-                       ties ? 1 : 0, out_of(o.get()), flags, d_long.p);
-    XH_CHECK_HIP(hipGetLastError());
-    if (!ties || read_count(ctx, d_long.p) == 0) return o.release();
-    // long runs: the key by pieces from its low end, each sort keeping the order of the one before
-    Buf<uint32_t> perm[2];
-    int cur = 0;
-    for (int lo = 0; lo < kb.total; lo += room) {
-        kp = key_piece(kb, lo, std::min(room, kb.total - lo), n);
+    Owned w(ctx, alloc_keys(ctx, n));
+    LAUNCH_1D(k_key_pieces<W>, n, view_of(in), kp, n, w.p, W > 1 ? aos.p : nullptr, nullptr, 0, nullptr, 0);
+    auto fetch = [&](const KeyPiece &p, uint64_t m, bool ties, uint8_t *f, const uint32_t *pos) {
+        hipLaunchKernelGGL(k_sorted_rows<W>, dim3((unsigned)((m + ROWS_TILE - 1) / ROWS_TILE)), dim3(ROWS_TB), 0,
+                           ctx->stream, w.p, p, m, rows, kb, (int)in->arity, ties ? 1 : 0, out_of(o.get()), f, d_long.p, pos);
+        XH_CHECK_HIP(hipGetLastError());
+    };
+    LongRuns runs;
+    for (uint64_t m = n;;) {
+        // (the words are all different; rows of equal prefix are in order)
+        // Short prefixes take the passes of their digits (10^6 rows by a column of 200 values 127 us by buckets, 68 so;
+        // of 5,000 128 / 88; of 32 bits 132 / 125, but 10^5 rows 69 / 95).
+        const int digit = std::min(7, (64 - kp.bits) / 8);
+        if (m > BLOCK_SORT_KEYS && !kb.known)
+            w.reset(sort_keys(ctx, w.release(), m, true, digit, 8));
+        else if (m > BLOCK_SORT_KEYS && (digit > 4 || (digit == 4 && m > (1ull << 18))))
+            w.reset(sort_keys(ctx, w.release(), m, true, digit, 8, 0xFFu & ~((1u << digit) - 1u)));
+        else
+            w.reset(sort_keys(ctx, w.release(), m, true, 0, 8, 0, nullptr, digit));
+        if (left) fill_u64(ctx, d_long.p, 0ull, 1);
+        fetch(kp, m, left > 0, flags, m < n ? runs.pos.p : nullptr);
+        if (!left || read_count(ctx, d_long.p) == 0) return o.release();
+        LongRuns next;
+        long_runs(ctx, w.p, kp, m, m < n ? runs.pos.p : nullptr, next);
+        int gbits = 0;
+        while ((1ull << gbits) < next.groups) ++gbits;
+        const int bits = std::min(left, room - gbits);
+        // (how many bits would make the runs short, if the rest of the key splits them as the bits so far did)
+        const double split = std::log2((double)next.groups) / (kb.total - left);
+        if (bits < std::min(left, 8) || (2 * next.n > n && next.groups >= 16 &&
+                         std::log2((double)next.n / next.groups / (RUN_MAX / 2)) > split * bits))
+            break;
+        const int shift = kp.row_shift;
+        left -= bits;
+        kp = key_piece(kb, left, bits, n, gbits);
+        runs = std::move(next);
+        m = runs.n;
         w.reset();
-        w.reset(sorted_pieces<W>(ctx, in, kp, lo ? perm[cur].p : nullptr, nullptr));
-        perm[cur ^ 1] = Buf<uint32_t>(ctx, n);
-        LAUNCH_1D(k_piece_rows, n, w.p, kp, lo ? perm[cur].p : nullptr, n, perm[cur ^ 1].p);
-        cur ^= 1;
+        w.reset(alloc_keys(ctx, m));
+        LAUNCH_1D(k_key_pieces<W>, m, view_of(in), kp, m, w.p, nullptr, runs.words.p, shift,
+                  gbits ? runs.group.p : nullptr, gbits);
     }
-    KeyPiece all = key_piece(kb, 0, 0, n);  // (row numbers alone: the order is final)
-    LAUNCH_1D(k_key_of_rows, n, perm[cur].p, n, all.row_shift, w.p);
-    hipLaunchKernelGGL(k_sorted_rows<W>, grid, dim3(ROWS_TB), 0, ctx->stream, w.p, all, n, rows, kb, (int)in->arity, 0,
-                       out_of(o.get()), nullptr, d_long.p);
-    XH_CHECK_HIP(hipGetLastError());
+    // whole bytes of the key, as many as the row's number leaves, in pieces of about equal length
+    const int most = room & ~7, pieces = (kb.total + most - 1) / most, step = ((kb.total + pieces - 1) / pieces + 7) & ~7;
+    for (int lo = 0; lo < kb.total; lo += step) {
+        kp = key_piece(kb, lo, std::min(step, kb.total - lo), n);
+        kp.row_shift = 0;
+        Owned next(ctx, alloc_keys(ctx, n));
+        LAUNCH_1D(k_key_pieces<W>, n, view_of(in), kp, n, next.p, nullptr, lo ? w.p : nullptr, 0, nullptr, 0);
+        w.reset();
+        const int digit = (64 - kp.bits) / 8;
+        w.reset(sort_keys(ctx, next.release(), n, true, digit, 8, 0xFFu & ~((1u << digit) - 1u)));
+    }
+    kp.bits = 0;  // (the order is final)
+    fetch(kp, n, false, nullptr, nullptr);
     if (flags) {
         ProjSpec ks{(int)in->arity, kb.n, {0}};
         for (int t = 0; t < kb.n; ++t) ks.cols[t] = kb.col[t];

@@ -98,7 +98,7 @@ void project_pairs(Ctx *ctx, const uint64_t *in, uint64_t n, int h0, int h1, uin
 // from the histograms); whole (a sort of digits 4..7): set when the keys came
 // out ordered by the whole key (the segment route).
 uint64_t *sort_keys(Ctx *ctx, uint64_t *keys, uint64_t n, bool keys_owned, int digit_lo = 0, int digit_hi = 8,
-                    uint32_t known_digits = 0, bool *whole = nullptr);
+                    uint32_t known_digits = 0, bool *whole = nullptr, int in_order = 0);
 // Sorted unique copy of n keys into a new buffer *out, the count to *d_count (device).
 bool bucket_unique_keys_async(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t **out, uint64_t *d_count);
 void sort_unique_keys_async(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t **out, uint64_t *d_count,

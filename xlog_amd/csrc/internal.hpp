@@ -343,8 +343,11 @@ bool sort_tickets();
 // With `whole` (a keys-only sort of the high word, digits 4..7, of at least
 // 2^22 keys) the sort may order the keys by the whole key instead, through the
 // segment route; *whole tells whether it did.
-int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, int digit_lo = 0, int digit_hi = 8, const uint64_t *src = nullptr,
-                   uint32_t known_digits = 0, SortUnique *uq = nullptr, bool *whole = nullptr);
+// in_order (a sort of the whole key): keys that agree on the digits from
+// in_order up come in order already, so digit passes begin there.
+int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, int digit_lo = 0, int digit_hi = 8,
+                   const uint64_t *src = nullptr, uint32_t known_digits = 0, SortUnique *uq = nullptr,
+                   bool *whole = nullptr, int in_order = 0);
 // A keys-only sort of a queued iteration: the key count on the device
 // (*d_n <= n_bound, the bound the launches are sized for), exactly the digit
 // passes of known_digits (no read-back), and the stop flag (a raised flag:

@@ -1237,8 +1237,8 @@ bool block_sort_unique(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *out
     XH_CHECK_HIP(hipGetLastError());
     return true;
 }
-int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, int digit_lo, int digit_hi, const uint64_t *src, uint32_t known_digits,
-                   SortUnique *uq, bool *whole) {
+int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, int digit_lo, int digit_hi,
+                   const uint64_t *src, uint32_t known_digits, SortUnique *uq, bool *whole, int in_order) {
     if (whole) *whole = false;
     if (n < 2 || digit_lo >= digit_hi) {
         if (src && n) XH_CHECK_HIP(hipMemcpyAsync(*keys, src, n * 8, hipMemcpyDeviceToDevice, ctx->stream));
@@ -1302,7 +1302,8 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, i
         XH_CHECK_HIP(hipGetLastError());
     };
     fill_u32(ctx, hist, 0u, 8 * 256);
-    histograms(src ? src : *keys, hybrid_candidate ? 4 : digit_lo, digit_hi);
+    int first = std::max(digit_lo, in_order);
+    histograms(src ? src : *keys, hybrid_candidate ? 4 : first, digit_hi);
     int passes = 0;
     int cur = 0;  // status buffer for the next pass
     if (st.dirty[0] == 0) cur = 0; else if (st.dirty[1] == 0) cur = 1; else cur = 0;
@@ -1356,8 +1357,7 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, i
     uint32_t h_hist[8 * 256];
     static_assert(sizeof(h_hist) <= Ctx::HOST_STAGE_U64 * sizeof(uint64_t), "histograms exceed the staging");
     ctx->post_read(hist, sizeof(h_hist) / 8);
-    int first = digit_lo;
-    if (digit_hi - digit_lo >= 2 && !hybrid_candidate && !word_candidate) launch_pass(first++);
+    if (digit_hi - first >= 2 && !hybrid_candidate && !word_candidate) launch_pass(first++);
     ctx->wait_read();
     memcpy(h_hist, ctx->host_scalars, sizeof(h_hist));
     auto trivial = [&](int dgt) {
@@ -1391,18 +1391,19 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, i
         }
         // a segment above the on-chip capacity or a long run of unequal keys:
         // every digit's pass of the sort, from the keys as they are (any order
-        // sorts alike)
+        // sorts alike, and the passes so far were stable)
         if (word_candidate) {
             for (int dgt = 4; dgt < 8; ++dgt)
                 if (!trivial(dgt)) launch_pass(dgt);
             return passes;
         }
         low_word_histograms((passes == 0 && src) ? src : *keys);
-        for (int dgt = 0; dgt < 8; ++dgt)
+        for (int dgt = first; dgt < 8; ++dgt)
             if (!trivial(dgt)) launch_pass(dgt);
         return passes;
     }
-    if (hybrid_candidate && short_high_runs(h_hist, n)) {
+    // (with three digits in order the passes from there up are as few)
+    if (hybrid_candidate && first < 3 && short_high_runs(h_hist, n)) {
         // The high word's passes, then every run of equal high word sorted by
         // its low word in one pass instead of the low word's four passes.
         for (int dgt = 4; dgt < 8; ++dgt)
@@ -1424,12 +1425,12 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, i
             // high word, intact) takes every digit's pass; any order of the
             // keys sorts to the same result
             low_word_histograms(*keys);
-            for (int dgt = 0; dgt < 8; ++dgt)
+            for (int dgt = first; dgt < 8; ++dgt)
                 if (!trivial(dgt)) launch_pass(dgt);
             return passes;
         }
     }
-    if (hybrid_candidate) low_word_histograms(src ? src : *keys);
+    if (hybrid_candidate && first < 4) low_word_histograms(src ? src : *keys);
     for (int dgt = first; dgt < digit_hi; ++dgt)
         if (!trivial(dgt)) launch_pass(dgt);
     if (passes == 0 && src) XH_CHECK_HIP(hipMemcpyAsync(*keys, src, n * 8, hipMemcpyDeviceToDevice, ctx->stream));
