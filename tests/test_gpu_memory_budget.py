@@ -123,3 +123,38 @@ def test_failed_fixpoint_frees_its_device_memory(p, where):
     # second must end with exactly the live bytes it started with
     before = fail_once()
     assert fail_once() == before
+
+
+def _block(nbytes):
+    """What the pool takes for an allocation: four size classes per power of two."""
+    if nbytes < 256:
+        return 256
+    q = 1 << max(0, nbytes.bit_length() - 3)
+    return -(-nbytes // q) * q
+
+
+@pytest.fixture
+def within(p):
+    """A function that runs a call with a budget of some bytes above what is held."""
+    def run(nbytes, call):
+        gc.collect()
+        p.trim()
+        p.set_memory_budget(p.memory_stats()["in_use"] + nbytes)
+        try:
+            return call()
+        finally:
+            p.set_memory_budget(0)
+    return run
+
+
+SLACK = 5 << 19  # counters and the digit passes' look-back state
+
+
+@pytest.mark.parametrize("n", [100000, 1000000])
+def test_sorts_in_two_buffers(p, within, n):
+    """Sizes of the bucket sort, whose regions are four times the keys: without room for them the digit passes do."""
+    keys = np.random.default_rng(n).integers(0, 1 << 64, n, dtype=np.uint64)
+    rel = p.create_buffer_from_packed(keys)
+    need = 2 * _block(8 * n) + SLACK
+    assert np.array_equal(p.download_packed(within(need, lambda: p.dedup_full_row(rel))), np.unique(keys))
+    assert np.array_equal(p.download_packed(within(need, lambda: p.sort(rel, [0, 1]))), np.sort(keys))

@@ -500,7 +500,7 @@ bool bucket_unique_keys_async(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64
     if (!bucket_sort_takes(n)) return false;
     Owned o(ctx, alloc_keys(ctx, n));
     Buf<uint64_t> st;
-    bucket_sort(ctx, keys, n, o.p, d_count, st);
+    if (!bucket_sort(ctx, keys, n, o.p, d_count, st)) return false;
     *out = o.release();
     return true;
 }
@@ -1538,12 +1538,12 @@ static void build_row_index(Ctx *ctx, const xlog_hip_rel *r, const KeyPack &kp, 
     Owned rows(ctx, alloc_keys(ctx, n));
     LAUNCH_1D(k_pack_rows, n, view_of(r), kp, n, rows.p);
     J.payload = Buf<uint32_t>(ctx, n);
-    if (small && bucket_sort_takes(n)) {
-        Owned sorted(ctx, alloc_keys(ctx, n));
-        bucket_sort(ctx, rows.p, n, sorted.p, nullptr, state);
+    Owned sorted(ctx);
+    if (small && bucket_sort_takes(n) && fits_memory([&] { sorted.reset(alloc_keys(ctx, n)); }) &&
+        bucket_sort(ctx, rows.p, n, sorted.p, nullptr, state)) {
         rows.reset(sorted.release());
         *over = state.p;
-    } else if (n <= BLOCK_SORT_KEYS) {
+    } else if (sorted.reset(); n <= BLOCK_SORT_KEYS) {
         rows.reset(sort_keys(ctx, rows.release(), n, true, 0, 8));
     } else {
         rows.reset(sort_keys(ctx, rows.release(), n, true, 4, 8));  // stable; digit passes

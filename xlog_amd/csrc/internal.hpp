@@ -112,6 +112,19 @@ struct Buf {
     T *release() { T *q = p; p = nullptr; n = 0; return q; }
 };
 
+// Whether f ran to its end; false when it met with XLOG_HIP_OOM.  For a route
+// that needs more memory than another one that gives the same result.
+template <typename F>
+bool fits_memory(F f) {
+    try {
+        f();
+        return true;
+    } catch (const Error &e) {
+        if (e.code != XLOG_HIP_OOM) throw;
+        return false;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // context: one device, one stream, the pool and the small persistent device
 // state used by the single-pass (decoupled look-back) kernels.
@@ -330,11 +343,12 @@ bool block_sort_unique(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *out
 // sort's) from in to out (n entries each, not shared).  With d_count the unique
 // keys, their number to *d_count (device).  A bucket too long for LDS leaves
 // out incomplete, *d_count = ~0 and the low half of state's first word
-// non-zero: the caller then sorts otherwise.
+// non-zero: the caller then sorts otherwise.  false, and nothing done, when the
+// buckets' regions (about four times the keys) are not to be had.
 // bucket_sort_takes: the sizes it is for (no: another sort was asked for).
 constexpr uint64_t BUCKET_SORT_KEYS = 1ull << 20;
 bool bucket_sort_takes(uint64_t n);
-void bucket_sort(Ctx *ctx, const uint64_t *in, uint64_t n, uint64_t *out, uint64_t *d_count, Buf<uint64_t> &state);
+bool bucket_sort(Ctx *ctx, const uint64_t *in, uint64_t n, uint64_t *out, uint64_t *d_count, Buf<uint64_t> &state);
 // XLOG_HIP_SORT_TICKETS=1 (read at each sort): the radix pass and the
 // short-run unique order their tiles by an atomic start ticket instead of the
 // workgroup index, so that their look-back does not rest on workgroups

@@ -1207,13 +1207,17 @@ static bool sort_block() {
     return !getenv("XLOG_HIP_SORT_TICKETS") && !getenv("XLOG_HIP_SORT_PERSIST") && !getenv("XLOG_HIP_SORT_SPIN");
 }
 bool bucket_sort_takes(uint64_t n) { return n > BLOCK_SORT_KEYS && n <= BUCKET_SORT_KEYS && sort_block(); }
-void bucket_sort(Ctx *ctx, const uint64_t *in, uint64_t n, uint64_t *out, uint64_t *d_count, Buf<uint64_t> &state) {
+bool bucket_sort(Ctx *ctx, const uint64_t *in, uint64_t n, uint64_t *out, uint64_t *d_count, Buf<uint64_t> &state) {
     int bits = 1;
     while ((n >> bits) > 1024) ++bits;
     XH_REQUIRE(n > BLOCK_SORT_KEYS && n <= BUCKET_SORT_KEYS && bits <= BK_MAX_BITS, XLOG_HIP_INVALID_ARG,
                "bucket sort: number of keys");
-    Buf<uint64_t> regions(ctx, (uint64_t)BK_KEYS << bits);
-    state = Buf<uint64_t>(ctx, sizeof(BucketState) / 8);
+    Buf<uint64_t> regions;
+    if (!fits_memory([&] {
+            regions = Buf<uint64_t>(ctx, (uint64_t)BK_KEYS << bits);
+            state = Buf<uint64_t>(ctx, sizeof(BucketState) / 8);
+        }))
+        return false;
     BucketState *st = reinterpret_cast<BucketState *>(state.p);
     // (the sample's keys pass through the regions, which the scatter fills afterwards)
     hipLaunchKernelGGL(k_bucket_sample, dim3(1), dim3(BS_TB), 0, ctx->stream, in, n, st, bits, regions.p);
@@ -1227,6 +1231,7 @@ void bucket_sort(Ctx *ctx, const uint64_t *in, uint64_t n, uint64_t *out, uint64
         hipLaunchKernelGGL(k_bucket_sort<false>, dim3(1u << bits), dim3(BK_TB), 0, ctx->stream, regions.p, st, out);
     }
     XH_CHECK_HIP(hipGetLastError());
+    return true;
 }
 
 bool block_sort_unique(Ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *out, uint64_t *d_count) {
@@ -1260,11 +1265,12 @@ int radix_sort_u64(Ctx *ctx, uint64_t **keys, uint64_t **keys_alt, uint64_t n, i
     }
     if (digit_lo == 0 && digit_hi == 8 && !known_digits && !uq && bucket_sort_takes(n)) {
         Buf<uint64_t> st;
-        bucket_sort(ctx, src ? src : *keys, n, *keys_alt, nullptr, st);
-        ctx->read_scalars(st.p, 1);
-        if (!(uint32_t)ctx->host_scalars[0]) {  // BucketState::over
-            std::swap(*keys, *keys_alt);
-            return 2;
+        if (bucket_sort(ctx, src ? src : *keys, n, *keys_alt, nullptr, st)) {
+            ctx->read_scalars(st.p, 1);
+            if (!(uint32_t)ctx->host_scalars[0]) {  // BucketState::over
+                std::swap(*keys, *keys_alt);
+                return 2;
+            }
         }
     }
     const uint64_t tile_keys = (uint64_t)SORT_BLOCK_K * SORT_ITEMS_K;
