@@ -158,3 +158,30 @@ def test_sorts_in_two_buffers(p, within, n):
     need = 2 * _block(8 * n) + SLACK
     assert np.array_equal(p.download_packed(within(need, lambda: p.dedup_full_row(rel))), np.unique(keys))
     assert np.array_equal(p.download_packed(within(need, lambda: p.sort(rel, [0, 1]))), np.sort(keys))
+
+
+@pytest.mark.parametrize("arity,first", [(3, 1 << 32), (4, 1 << 32), (6, 3), (8, 1 << 32), (4, 1)])
+@pytest.mark.parametrize("keys", ["all", "one"])
+@pytest.mark.parametrize("n", [12000, 700000])
+def test_row_sorts_without_a_copy_of_the_rows(p, within, arity, first, keys, n):
+    """Room for four bytes per row beside the sorted rows, or for two words: the rows are not copied and the key goes by
+    pieces."""
+    rng = np.random.default_rng(n + arity)
+    cols = [rng.integers(0, first if c == 0 else 1 << 32, n).astype(np.uint32) for c in range(arity)]
+    rel = p.create_buffer_from_u32_columns(cols)
+    by = list(range(arity)) if keys == "all" else [1]
+    words = (arity + 1) // 2
+    need = max(words * _block(8 * n) + _block(4 * n), 2 * _block(8 * n)) + (SLACK if n > 16384 else 1 << 16)
+    out = within(need, lambda: p.sort(rel, by))
+    order = np.lexsort([cols[c] for c in reversed(by)])
+    for c in range(arity):
+        assert np.array_equal(p.download_column(out, c), cols[c][order]), c
+    del out
+    cols[0][:] = cols[0][0]
+    rel = p.create_buffer_from_u32_columns([np.concatenate([c, c]) for c in cols])  # every row twice
+    out = within((3 * words + 1) * _block(16 * n) + SLACK, lambda: p.dedup(rel, by))
+    order = np.lexsort([cols[c] for c in reversed(by)])
+    first_of = np.ones(n, bool)
+    first_of[1:] = np.any([cols[c][order][1:] != cols[c][order][:-1] for c in by], axis=0)
+    for c in range(arity):
+        assert np.array_equal(p.download_column(out, c), cols[c][order][first_of]), c

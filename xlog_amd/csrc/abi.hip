@@ -672,6 +672,17 @@ __global__ __launch_bounds__(ROWS_TB) void k_sorted_rows(const uint64_t *__restr
         if (flags) flags[o] = !same;
     }
 }
+// the rows that words number (row_shift 0), and a word array in that order
+__global__ void k_rows_of(const uint64_t *__restrict__ words, int row_bits, uint64_t n, uint32_t *__restrict__ out) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+        out[i] = (uint32_t)(words[i] & ((1ull << row_bits) - 1));
+}
+__global__ void k_take_rows(const uint64_t *__restrict__ in, const uint32_t *__restrict__ rows, uint64_t n,
+                            uint64_t *__restrict__ out) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) out[i] = in[rows[i]];
+}
 // in_long[i] = 1 for the sorted words whose run of equal prefix has more than RUN_MAX (in_long[n] = 0: n + 1 entries)
 __global__ void k_long_runs(const uint64_t *__restrict__ sorted, KeyPiece kp, uint64_t n, uint32_t *__restrict__ in_long) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -770,26 +781,31 @@ static void long_runs(Ctx *ctx, const uint64_t *sorted, const KeyPiece &kp, uint
     scan_u32_inplace(ctx, out.group.p, out.n + 1, sum.p);
     out.groups = read_count(ctx, reinterpret_cast<const uint64_t *>(sum.p));
 }
-// Rows of `in` sorted by kb's columns (stable).  With flags: 1 for the first row
-// of every group of rows equal on those columns.
+typedef std::unique_ptr<xlog_hip_rel, void (*)(xlog_hip_rel *)> RelOwner;
 template <int W>
-static xlog_hip_rel *sorted_rows(Ctx *ctx, const xlog_hip_rel *in, const KeyBits &kb, uint8_t *flags) {
+static void fetch_rows(Ctx *ctx, const xlog_hip_rel *in, const KeyBits &kb, const uint64_t *w, const KeyPiece &kp,
+                       uint64_t n, const uint64_t *aos, bool ties, xlog_hip_rel *out, uint8_t *flags,
+                       uint64_t *d_long, const uint32_t *pos) {
+    hipLaunchKernelGGL(k_sorted_rows<W>, dim3((unsigned)((n + ROWS_TILE - 1) / ROWS_TILE)), dim3(ROWS_TB), 0, ctx->stream,
+                       w, kp, n, W > 1 ? aos : in->w[0], kb, (int)in->arity, ties ? 1 : 0, out_of(out), flags, d_long, pos);
+    XH_CHECK_HIP(hipGetLastError());
+}
+// By prefixes; false where pieces of the whole key are the better way on.  The
+// rows to o (allocated here), their copy to aos, where one is made.
+template <int W>
+static bool rows_by_prefix(Ctx *ctx, const xlog_hip_rel *in, const KeyBits &kb, uint8_t *flags, RelOwner &o,
+                           Buf<uint64_t> &aos) {
     const uint64_t n = in->rows;
-    std::unique_ptr<xlog_hip_rel, void (*)(xlog_hip_rel *)> o(rel_new(ctx, in->arity, n), rel_free);
+    o.reset(rel_new(ctx, in->arity, n));
     o->rows = n;
     KeyPiece kp = key_piece(kb, 0, 0, n);
     const int room = 64 - kp.row_bits;
     int left = std::max(0, kb.total - room);  // bits of the key below the prefix
     kp = key_piece(kb, left, kb.total - left, n);
-    Buf<uint64_t> aos(ctx, W > 1 ? n * W : 0), d_long(ctx, 1);
-    const uint64_t *rows = W > 1 ? aos.p : in->w[0];
+    if (W > 1) aos = Buf<uint64_t>(ctx, n * W);
+    Buf<uint64_t> d_long(ctx, 1);
     Owned w(ctx, alloc_keys(ctx, n));
     LAUNCH_1D(k_key_pieces<W>, n, view_of(in), kp, n, w.p, W > 1 ? aos.p : nullptr, nullptr, 0, nullptr, 0);
-    auto fetch = [&](const KeyPiece &p, uint64_t m, bool ties, uint8_t *f, const uint32_t *pos) {
-        hipLaunchKernelGGL(k_sorted_rows<W>, dim3((unsigned)((m + ROWS_TILE - 1) / ROWS_TILE)), dim3(ROWS_TB), 0,
-                           ctx->stream, w.p, p, m, rows, kb, (int)in->arity, ties ? 1 : 0, out_of(o.get()), f, d_long.p, pos);
-        XH_CHECK_HIP(hipGetLastError());
-    };
     LongRuns runs;
     for (uint64_t m = n;;) {
         // (the words are all different; rows of equal prefix are in order)
@@ -803,18 +819,19 @@ static xlog_hip_rel *sorted_rows(Ctx *ctx, const xlog_hip_rel *in, const KeyBits
         else
             w.reset(sort_keys(ctx, w.release(), m, true, 0, 8, 0, nullptr, digit));
         if (left) fill_u64(ctx, d_long.p, 0ull, 1);
-        fetch(kp, m, left > 0, flags, m < n ? runs.pos.p : nullptr);
-        if (!left || read_count(ctx, d_long.p) == 0) return o.release();
+        const uint32_t *pos = m < n ? runs.pos.p : nullptr;
+        fetch_rows<W>(ctx, in, kb, w.p, kp, m, aos.p, left > 0, o.get(), flags, d_long.p, pos);
+        if (!left || read_count(ctx, d_long.p) == 0) return true;
         LongRuns next;
-        long_runs(ctx, w.p, kp, m, m < n ? runs.pos.p : nullptr, next);
+        long_runs(ctx, w.p, kp, m, pos, next);
         int gbits = 0;
         while ((1ull << gbits) < next.groups) ++gbits;
         const int bits = std::min(left, room - gbits);
         // (how many bits would make the runs short, if the rest of the key splits them as the bits so far did)
         const double split = std::log2((double)next.groups) / (kb.total - left);
         if (bits < std::min(left, 8) || (2 * next.n > n && next.groups >= 16 &&
-                         std::log2((double)next.n / next.groups / (RUN_MAX / 2)) > split * bits))
-            break;
+                                         std::log2((double)next.n / next.groups / (RUN_MAX / 2)) > split * bits))
+            return false;
         const int shift = kp.row_shift;
         left -= bits;
         kp = key_piece(kb, left, bits, n, gbits);
@@ -825,24 +842,56 @@ static xlog_hip_rel *sorted_rows(Ctx *ctx, const xlog_hip_rel *in, const KeyBits
         LAUNCH_1D(k_key_pieces<W>, m, view_of(in), kp, m, w.p, nullptr, runs.words.p, shift,
                   gbits ? runs.group.p : nullptr, gbits);
     }
-    // whole bytes of the key, as many as the row's number leaves, in pieces of about equal length
-    const int most = room & ~7, pieces = (kb.total + most - 1) / most, step = ((kb.total + pieces - 1) / pieces + 7) & ~7;
-    for (int lo = 0; lo < kb.total; lo += step) {
-        kp = key_piece(kb, lo, std::min(step, kb.total - lo), n);
+}
+// By pieces of whole bytes, as many as the row's number leaves and of about
+// equal length: two buffers of keys, then the rows and four bytes for each of
+// them (o and aos when they are there already).
+template <int W>
+static void rows_by_pieces(Ctx *ctx, const xlog_hip_rel *in, const KeyBits &kb, uint8_t *flags, RelOwner &o,
+                           const Buf<uint64_t> &aos) {
+    const uint64_t n = in->rows;
+    KeyPiece kp = key_piece(kb, 0, 0, n);
+    const int most = (64 - kp.row_bits) & ~7, pieces = std::max(1, (kb.total + most - 1) / most),
+              step = ((kb.total + pieces - 1) / pieces + 7) & ~7;
+    Owned w(ctx);
+    for (int p = 0; p < pieces; ++p) {
+        kp = key_piece(kb, p * step, std::min(step, kb.total - p * step), n);
         kp.row_shift = 0;
         Owned next(ctx, alloc_keys(ctx, n));
-        LAUNCH_1D(k_key_pieces<W>, n, view_of(in), kp, n, next.p, nullptr, lo ? w.p : nullptr, 0, nullptr, 0);
+        LAUNCH_1D(k_key_pieces<W>, n, view_of(in), kp, n, next.p, nullptr, p ? w.p : nullptr, 0, nullptr, 0);
         w.reset();
         const int digit = (64 - kp.bits) / 8;
         w.reset(sort_keys(ctx, next.release(), n, true, digit, 8, 0xFFu & ~((1u << digit) - 1u)));
     }
-    kp.bits = 0;  // (the order is final)
-    fetch(kp, n, false, nullptr, nullptr);
+    if (o) {
+        kp.bits = 0;  // (the order is final)
+        fetch_rows<W>(ctx, in, kb, w.p, kp, n, aos.p, false, o.get(), nullptr, nullptr, nullptr);
+    } else {
+        Buf<uint32_t> order(ctx, n);
+        LAUNCH_1D(k_rows_of, n, w.p, kp.row_bits, n, order.p);
+        w.reset();
+        o.reset(rel_new(ctx, in->arity, n));
+        o->rows = n;
+        for (int q = 0; q < W; ++q) LAUNCH_1D(k_take_rows, n, in->w[q], order.p, n, o->w[q]);
+    }
     if (flags) {
         ProjSpec ks{(int)in->arity, kb.n, {0}};
         for (int t = 0; t < kb.n; ++t) ks.cols[t] = kb.col[t];
         LAUNCH_1D(k_group_flags, n, view_of(o.get()), ks, n, flags);
     }
+}
+// Rows of `in` sorted by kb's columns (stable).  With flags: 1 for the first row
+// of every group of rows equal on those columns.
+template <int W>
+static xlog_hip_rel *sorted_rows(Ctx *ctx, const xlog_hip_rel *in, const KeyBits &kb, uint8_t *flags) {
+    RelOwner o(nullptr, rel_free);
+    Buf<uint64_t> aos;
+    bool done = false;
+    if (!fits_memory([&] { done = rows_by_prefix<W>(ctx, in, kb, flags, o, aos); })) {
+        o.reset();
+        aos = Buf<uint64_t>();
+    }
+    if (!done) rows_by_pieces<W>(ctx, in, kb, flags, o, aos);
     return o.release();
 }
 static xlog_hip_rel *sort_rows(Ctx *ctx, const xlog_hip_rel *in, const std::vector<int> &cols, uint8_t *flags) {
