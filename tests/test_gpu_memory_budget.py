@@ -185,3 +185,40 @@ def test_row_sorts_without_a_copy_of_the_rows(p, within, arity, first, keys, n):
     first_of[1:] = np.any([cols[c][order][1:] != cols[c][order][:-1] for c in by], axis=0)
     for c in range(arity):
         assert np.array_equal(p.download_column(out, c), cols[c][order][first_of]), c
+
+
+# bytes per build row above the inputs that each join took as an index over its sorted keys (one key) or by dictionaries
+@pytest.mark.parametrize("kind,per_row", [("one", 100), ("few", 34), ("two", 96), ("two keys only", 96), ("wide", 92),
+                                          ("direct", 104), ("two few", 30)])
+@pytest.mark.parametrize("n", [300000, 1000000])
+def test_joins_without_room_for_packed_keys(p, within, kind, per_row, n):
+    """Joins and semi joins within what they took before keys were packed, by whatever route fits."""
+    rng = np.random.default_rng(n)
+    cols = lambda rows, *tops: [rng.integers(0, t, rows).astype(np.uint32) for t in tops]  # noqa: E731
+    nl, on = n, [0, 1]
+    if kind in ("one", "few"):
+        on, nl = [0], n if kind == "one" else 1000
+        tops = [100 if kind == "few" else n // 2, 1 << 32]
+    elif kind == "wide":
+        on, tops = [2], [50, 64, n]
+    else:
+        tops = [{"direct": 4 * n // 64, "two few": 50}.get(kind, n // 64), 64] + ([] if "only" in kind else [1 << 32])
+        nl = 1000 if kind == "two few" else n
+    left, right = cols(nl, *tops), cols(n, *tops)
+    L, R = p.create_buffer_from_u32_columns(left), p.create_buffer_from_u32_columns(right)
+    code = lambda c: sum(c[k].astype(np.int64) << (32 * i) for i, k in enumerate(on))  # noqa: E731
+    hit = np.isin(code(left), code(right))
+    from xlog_amd import JOIN_ANTI, JOIN_INNER, JOIN_SEMI
+
+    semi_row = {"two": 40, "direct": 40, "two keys only": 31, "wide": 40}.get(kind, per_row)
+    for how, keep in ((JOIN_SEMI, hit), (JOIN_ANTI, ~hit)):
+        out = within(semi_row * n + SLACK, lambda: p.hash_join_v2(L, R, on, on, how))
+        assert np.array_equal(p.download_column(out, 0), left[0][keep])
+        del out
+    if kind in ("few", "two few"):
+        return  # (outputs of many rows a key)
+    want = p.hash_join_v2(L, R, on, on, JOIN_INNER)
+    want = [p.download_column(want, c) for c in range(want.arity)]
+    got = within(per_row * n + SLACK, lambda: p.hash_join_v2(L, R, on, on, JOIN_INNER))
+    for c, w in enumerate(want):
+        assert np.array_equal(p.download_column(got, c), w), c

@@ -1562,8 +1562,10 @@ static bool key_pack(Ctx *ctx, const xlog_hip_rel *r, const std::vector<int> &rk
         kp.bits += len;
         if (kp.bits > 31) return false;
     }
-    // keys of few bits are their own slots (a table of at most 8 slots a row)
-    kp.mix = (1ull << kp.bits) > 8 * r->rows;
+    // Keys of few bits are their own slots of 16 bytes (2^20 rows on 20 bits 0.22 ms, mixed 0.27; 2^24 rows on 27 bits
+    // 2.69 / 3.24): at most 8 slots a row, as an index of that many runs may take 4, and neither more than a 64th of
+    // the device's memory nor a quarter of what a budget leaves.
+    kp.mix = (1ull << kp.bits) > std::min<uint64_t>({8 * r->rows, 1ull << 28, ctx->pool->headroom() / 64});
     return true;
 }
 static KeyPack on_columns(const KeyPack &kp, const std::vector<int> &cols) {
@@ -1675,16 +1677,9 @@ static xlog_hip_rel *empty_side_join(Ctx *ctx, const xlog_hip_rel *l, const xlog
     return rel_new(ctx, type == XLOG_HIP_JOIN_INNER ? l->arity + r->arity : l->arity, 0);
 }
 
-static xlog_hip_rel *op_join_keys(Ctx *ctx, const xlog_hip_rel *l, const xlog_hip_rel *r, const std::vector<int> &lk,
-                                  const std::vector<int> &rk, int type) {
-    check_key_lists(l, r, lk, rk, type);
-    if (l->rows == 0 || r->rows == 0) return empty_side_join(ctx, l, r, type);
-    KeyPack kp;
-    if (!key_pack(ctx, r, rk, kp)) {
-        KeyFold F;
-        fold_build(ctx, r, rk, F, type == XLOG_HIP_JOIN_INNER);
-        return keyed_join_probe(ctx, l, r, lk, F, type, 0);
-    }
+// The join of non-empty inputs with packed keys.
+static xlog_hip_rel *packed_join(Ctx *ctx, const xlog_hip_rel *l, const xlog_hip_rel *r, const std::vector<int> &lk,
+                                 const std::vector<int> &rk, const KeyPack &kp, int type) {
     const uint64_t nl = l->rows, nr = r->rows;
     Buf<uint64_t> probe(ctx, nl);
     LAUNCH_1D(k_pack_rows, nl, view_of(l), on_columns(kp, lk), nl, probe.p);
@@ -1706,11 +1701,24 @@ static xlog_hip_rel *op_join_keys(Ctx *ctx, const xlog_hip_rel *l, const xlog_hi
     const uint64_t n = row_index_join(ctx, probe.p, nl, 0, r, kp, payload_col, 2, oc, pairs, none);
     const uint32_t arity = l->arity + r->arity;
     if (n == 0) return rel_new(ctx, arity, 0);
-    std::unique_ptr<xlog_hip_rel, void (*)(xlog_hip_rel *)> o(rel_new(ctx, arity, n), rel_free);
+    RelOwner o(rel_new(ctx, arity, n), rel_free);
     o->rows = n;
     LAUNCH_1D(k_join_rows, n, view_of(l), view_of(r), join_map(l, r->arity, lk, rk, payload_col), pairs.p, n,
               out_of(o.get()));
     return o.release();
+}
+// Keys that do not pack, and joins whose packed keys, set or table do not fit
+// the device (its budget), go through the dictionaries.
+static xlog_hip_rel *op_join_keys(Ctx *ctx, const xlog_hip_rel *l, const xlog_hip_rel *r, const std::vector<int> &lk,
+                                  const std::vector<int> &rk, int type) {
+    check_key_lists(l, r, lk, rk, type);
+    if (l->rows == 0 || r->rows == 0) return empty_side_join(ctx, l, r, type);
+    KeyPack kp;
+    xlog_hip_rel *o = nullptr;
+    if (key_pack(ctx, r, rk, kp) && fits_memory([&] { o = packed_join(ctx, l, r, lk, rk, kp, type); })) return o;
+    KeyFold F;
+    fold_build(ctx, r, rk, F, type == XLOG_HIP_JOIN_INNER);
+    return keyed_join_probe(ctx, l, r, lk, F, type, 0);
 }
 
 static xlog_hip_rel *op_join(Ctx *ctx, const xlog_hip_rel *l, const xlog_hip_rel *r, uint32_t lk, uint32_t rk,
@@ -1725,8 +1733,11 @@ static xlog_hip_rel *op_join(Ctx *ctx, const xlog_hip_rel *l, const xlog_hip_rel
         return op_project(ctx, j, *out_cols);
     }
     const int pcol = probe_vidx(l->arity, lk);
-    if ((type == XLOG_HIP_JOIN_SEMI || type == XLOG_HIP_JOIN_ANTI) && l->rows && r->rows)
-        return key_set_join(ctx, l, l->w[0], pcol, r->w[0], r->rows, probe_vidx(r->arity, rk), type, false);
+    xlog_hip_rel *o = nullptr;  // (a set of keys is sized by the rows, the index below by the distinct keys)
+    if ((type == XLOG_HIP_JOIN_SEMI || type == XLOG_HIP_JOIN_ANTI) && l->rows && r->rows && fits_memory([&] {
+            o = key_set_join(ctx, l, l->w[0], pcol, r->w[0], r->rows, probe_vidx(r->arity, rk), type, false);
+        }))
+        return o;
     if (type == XLOG_HIP_JOIN_INNER && l->rows && small_build(r->rows, 1) &&
         !((r->flags & REL_CANONICAL) && r->arity == 2 && rk == 0)) {  // (those are in key order already)
         int oc[4] = {0, 0, 0, 0};
@@ -1734,10 +1745,17 @@ static xlog_hip_rel *op_join(Ctx *ctx, const xlog_hip_rel *l, const xlog_hip_rel
         KeyPack kp;
         key_pack(ctx, r, {(int)rk}, kp);
         Buf<uint64_t> o0, o1;
-        const uint64_t n = row_index_join(ctx, l->w[0], l->rows, pcol, r, kp, r->arity == 2 ? 1 - (int)rk : -1, out_arity,
-                                          oc, o0, o1);
-        if (n == 0) return rel_new(ctx, (uint32_t)out_arity, 0);
-        return rel_adopt(ctx, (uint32_t)out_arity, n, o0.release(), o1.release(), 0);
+        uint64_t n = 0;
+        // (its table is sized for as many runs as rows: without room for that, the index below)
+        if (fits_memory([&] {
+                n = row_index_join(ctx, l->w[0], l->rows, pcol, r, kp, r->arity == 2 ? 1 - (int)rk : -1, out_arity, oc, o0,
+                                   o1);
+            })) {
+            if (n == 0) return rel_new(ctx, (uint32_t)out_arity, 0);
+            return rel_adopt(ctx, (uint32_t)out_arity, n, o0.release(), o1.release(), 0);
+        }
+        o0 = Buf<uint64_t>();
+        o1 = Buf<uint64_t>();
     }
     JoinIndex J;
     build_join_index(ctx, r->w[0], r->rows, r->arity, (int)rk, (r->flags & REL_CANONICAL) != 0, J);
