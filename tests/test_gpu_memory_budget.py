@@ -222,3 +222,17 @@ def test_joins_without_room_for_packed_keys(p, within, kind, per_row, n):
     got = within(per_row * n + SLACK, lambda: p.hash_join_v2(L, R, on, on, JOIN_INNER))
     for c, w in enumerate(want):
         assert np.array_equal(p.download_column(got, c), w), c
+
+
+@pytest.mark.parametrize("nv,m,need", [(300, 300, 80_000), (1000, 900, 800_000), (1000, 1000, 900_000)])
+def test_small_closures_without_room_for_column_lists(p, within, nv, m, need):
+    """A closure over a small dense domain within what its bit matrices take."""
+    src, dst = datagen.random_digraph(nv, m, 3)
+    e = p.dedup_full_row(p.create_buffer_from_packed(pack(src, dst)))
+    outs_o, it_o, deltas_o = oracle.seminaive(tc_plan(), [np.unique(pack(src, dst)), None])
+    for budget in (need, 64 << 20):
+        outs, st = within(budget, lambda: p.fixpoint(tc_plan(), [e, None]))
+        assert np.array_equal(p.download_packed(outs[1]), outs_o[1])
+        assert st["iterations"] == it_o and st["delta_sizes"] == deltas_o
+        assert st["route"] == ROUTE_BITMAP
+        del outs

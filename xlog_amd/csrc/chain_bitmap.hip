@@ -1150,25 +1150,34 @@ void chain_fixpoint(Ctx *ctx, const std::vector<ChainRule> &rules, uint32_t n_pr
         if (rec.path.size() == 2 && !idb[rec.path[0].pred] && !rec.path[0].backward && rec.path[1].pred == seed_h &&
             !rec.path[1].backward && closure_columns_fits(domain, rows[rec.path[0].pred], rows[seed_e])) {
             const int f = rec.path[0].pred;
-            Buf<uint64_t> row_ptr(ctx, (uint64_t)domain + 1), R(ctx, (uint64_t)domain * words), rc(ctx, (uint64_t)domain + 1);
-            Buf<uint32_t> adj(ctx, rows[f] ? rows[f] : 1);
-            pairs_csr(ctx, keys[f], rows[f], domain, row_ptr.p, adj.p);
+            Buf<uint64_t> R, rc;
             std::vector<uint64_t> layers;
-            const uint64_t n = closure_columns(ctx, keys[f], rows[f], row_ptr.p, adj.p, keys[seed_e], rows[seed_e],
-                                               domain, words, max_iter, R.p, rc.p, layers);
-            uint64_t total = rows[seed_e];
-            deltas.push_back(total);
-            for (uint64_t v : layers) {
-                deltas.push_back(v);
-                total += v;
+            uint64_t n = 0;
+            // (its lists may take more than the matrices of a small domain: without room for them, the products below)
+            const bool fits = fits_memory([&] {
+                Buf<uint64_t> row_ptr(ctx, (uint64_t)domain + 1);
+                Buf<uint32_t> adj(ctx, rows[f] ? rows[f] : 1);
+                R = Buf<uint64_t>(ctx, (uint64_t)domain * words);
+                rc = Buf<uint64_t>(ctx, (uint64_t)domain + 1);
+                pairs_csr(ctx, keys[f], rows[f], domain, row_ptr.p, adj.p);
+                n = closure_columns(ctx, keys[f], rows[f], row_ptr.p, adj.p, keys[seed_e], rows[seed_e], domain, words,
+                                    max_iter, R.p, rc.p, layers);
+            });
+            if (fits) {
+                uint64_t total = rows[seed_e];
+                deltas.push_back(total);
+                for (uint64_t v : layers) {
+                    deltas.push_back(v);
+                    total += v;
+                }
+                const bool converged = n < max_iter;
+                if (converged) deltas.push_back(0);
+                *iterations = deltas.size() - 1;
+                XH_REQUIRE(converged, XLOG_HIP_ITERATION_LIMIT,
+                           "Recursive SCC iteration limit (" + std::to_string(max_iter) + ") exceeded");
+                out_n[seed_h] = bitmap_emit(ctx, R.p, domain, words, &out[seed_h], XLOG_HIP_KERNEL_CHAIN_EMIT, total, rc.p);
+                return;
             }
-            const bool converged = n < max_iter;
-            if (converged) deltas.push_back(0);
-            *iterations = deltas.size() - 1;
-            XH_REQUIRE(converged, XLOG_HIP_ITERATION_LIMIT,
-                       "Recursive SCC iteration limit (" + std::to_string(max_iter) + ") exceeded");
-            out_n[seed_h] = bitmap_emit(ctx, R.p, domain, words, &out[seed_h], XLOG_HIP_KERNEL_CHAIN_EMIT, total, rc.p);
-            return;
         }
     }
     run.setup(seed_cand);
