@@ -236,3 +236,13 @@ def test_small_closures_without_room_for_column_lists(p, within, nv, m, need):
         assert st["iterations"] == it_o and st["delta_sizes"] == deltas_o
         assert st["route"] == ROUTE_BITMAP
         del outs
+
+
+def test_difference_in_its_own_output(p, within):
+    """The difference of sets by merge keeps a flag per key; without room for it the keys' windows are searched."""
+    rng = np.random.default_rng(1)
+    a, b = (np.unique(rng.integers(0, 1 << 22, 2_000_000, dtype=np.uint64)) for _ in range(2))
+    A, B = (p.dedup_full_row(p.create_buffer_from_packed(k)) for k in (a, b))
+    want = np.setdiff1d(a, b)
+    assert np.array_equal(p.download_packed(p.diff_gpu(A, B)), want)  # (sizes the context's look-back state)
+    assert np.array_equal(p.download_packed(within(_block(8 * len(a)) + (1 << 17), lambda: p.diff_gpu(A, B))), want)

@@ -1019,8 +1019,8 @@ static xlog_hip_rel *op_diff(Ctx *ctx, const xlog_hip_rel *a, const xlog_hip_rel
     canonical_keys(ctx, b, cb);
     uint64_t *o = static_cast<uint64_t *>(ctx->alloc((ca.n ? ca.n : 1) * sizeof(uint64_t)));
     Buf<uint64_t> cnt(ctx, 1);
-    if (diff_by_merge_takes(ca.n, cb.n)) diff_by_merge(ctx, ca.k, ca.n, cb.k, cb.n, o, cnt.p);
-    else select_unique_diff(ctx, ca.k, ca.n, cb.k, cb.n, o, cnt.p);
+    if (!diff_by_merge_takes(ca.n, cb.n) || !diff_by_merge(ctx, ca.k, ca.n, cb.k, cb.n, o, cnt.p))
+        select_unique_diff(ctx, ca.k, ca.n, cb.k, cb.n, o, cnt.p);
     uint64_t n = read_count(ctx, cnt.p);
     return rel_adopt(ctx, a->arity, n, o, nullptr, REL_CANONICAL);
 }

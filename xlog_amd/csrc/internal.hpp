@@ -507,9 +507,10 @@ void merge_unique_sorted(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_
                          uint64_t *uniq, uint64_t *d_res);
 // The keys of the sorted set k that are not in the sorted set b, in order, by
 // the merge path of the two (select_unique_diff searches windows of b instead);
-// diff_by_merge_takes: the sizes for which that is faster.
+// diff_by_merge_takes: the sizes for which that is faster.  false, and nothing
+// done, when its flags (a byte per key) do not fit the device.
 bool diff_by_merge_takes(uint64_t n, uint64_t nb);
-void diff_by_merge(Ctx *ctx, const uint64_t *k, uint64_t n, const uint64_t *b, uint64_t nb, uint64_t *out,
+bool diff_by_merge(Ctx *ctx, const uint64_t *k, uint64_t n, const uint64_t *b, uint64_t nb, uint64_t *out,
                    uint64_t *d_count);
 
 // Sorted-run index over the high word of sorted packed keys (join build):

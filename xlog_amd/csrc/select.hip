@@ -1783,17 +1783,23 @@ void merge_unique_sorted(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_
     run_select(ctx, out, na + nb, SelUnique{out, uniq}, d_res + 1, nullptr, nullptr, d_res);
 }
 bool diff_by_merge_takes(uint64_t n, uint64_t nb) { return n >= (1ull << 12) && nb >= n / 2 && nb / 32 <= n; }
-void diff_by_merge(Ctx *ctx, const uint64_t *k, uint64_t n, const uint64_t *b, uint64_t nb, uint64_t *out,
+bool diff_by_merge(Ctx *ctx, const uint64_t *k, uint64_t n, const uint64_t *b, uint64_t nb, uint64_t *out,
                    uint64_t *d_count) {
     const uint64_t tiles = (n + nb + MRG_TILE - 1) / MRG_TILE;
     XH_REQUIRE(tiles < (1ull << 31), XLOG_HIP_CAPACITY_OVERFLOW, "diff: input too large");
-    Buf<uint64_t> split(ctx, tiles + 1);
-    Buf<uint8_t> flags(ctx, n);
+    Buf<uint64_t> split;
+    Buf<uint8_t> flags;
+    if (!fits_memory([&] {
+            split = Buf<uint64_t>(ctx, tiles + 1);
+            flags = Buf<uint8_t>(ctx, n);
+        }))
+        return false;
     hipLaunchKernelGGL(k_merge_partition, dim3((unsigned)((tiles + 1 + 255) / 256)), dim3(256), 0, ctx->stream, b, nb, k, n,
                        tiles, split.p, MergeDev{});
     hipLaunchKernelGGL(k_merge_absent, dim3((unsigned)tiles), dim3(MRG_BLOCK), 0, ctx->stream, b, nb, k, n, split.p, flags.p);
     XH_CHECK_HIP(hipGetLastError());
     select_flags(ctx, k, flags.p, n, out, d_count);
+    return true;
 }
 
 void pack_columns(Ctx *ctx, const uint32_t *c0, const uint32_t *c1, uint64_t n, uint64_t *out) {
