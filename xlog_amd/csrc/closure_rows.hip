@@ -22,8 +22,11 @@
 // batch is the largest that seldom outgrows it (32 edges: more sources listed,
 // the call 1.18 ms; 16: 1.17; 14 with sets of 512: 1.74).  The sources of a
 // batch that does not fit are listed and walked one by one with larger sets;
-// when they are many, or one of them outgrows the largest set, the attempt
-// ends early and the caller goes on with its loop over hash sets.
+// when they are many the attempt ends early and the caller goes on with its loop
+// over hash sets.  A few that outgrow the largest set are handed back instead:
+// the caller's loop then runs from their edges alone (when one of them ended the
+// attempt, a source with 10,000 edges among 2^19 others cost STAR_BEFORE us
+// where the loop alone took 1,300; so STAR_NOW).
 #include "internal.hpp"
 #include "host.hpp"
 
@@ -55,9 +58,10 @@ struct CrArgs {
     uint32_t *cnt, *pos;  // per edge that begins a source: pairs, their place in scratch (cnt 0 at the others)
     unsigned long long *layers;  // [CR_LAYERS][CR_BINS]
     unsigned long long *next;    // [CR_BINS] edges that follow an edge, over all edges
-    uint32_t *ctl;               // give up, sources listed for tier 2, for tier 3, pairs of both in scratch
-    uint32_t *list[2];
-    uint32_t list_cap[2];
+    // give up; sources listed for tier 2, for tier 3, handed back; pairs of tiers 2 and 3 in scratch
+    uint32_t *ctl;
+    uint32_t *list[3];
+    uint32_t list_cap[3];
     uint32_t region, region_n;  // of scratch, for the listed sources
 };
 
@@ -302,8 +306,7 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
         cr_give_up(a);
 }
 
-// the listed sources, one at a time; those that do not fit go to the next
-// list, or end the attempt
+// the listed sources, one at a time; those that do not fit go to the next list
 template <int T, int SLOTS, int FR, int LV, int TIER>
 __global__ __launch_bounds__(T) void k_cr_walk_one(CrArgs a, uint32_t cap) {
     __shared__ CrLds<SLOTS, FR, LV> l;
@@ -326,26 +329,29 @@ __global__ __launch_bounds__(T) void k_cr_walk_one(CrArgs a, uint32_t cap) {
         const int nl = cr_walk<T, SLOTS, FR, LV>(l, a, cap);
         __syncthreads();
         const uint32_t e = a.list[TIER - 1][i];
-        if (nl < 0) {
-            if (threadIdx.x == 0) {
-                const uint32_t j = TIER == 1 ? atomicAdd(&a.ctl[2], 1u) : ~0u;
-                if (TIER == 1 && j < a.list_cap[1])
-                    a.list[1][j] = e;
-                else
-                    cr_give_up(a);
+        auto pass_on = [&](int to) {  // to list `to`, where the source has no pairs of its own yet
+            const uint32_t j = atomicAdd(&a.ctl[1 + to], 1u);
+            if (j < a.list_cap[to]) {
+                a.list[to][j] = e;
+                a.cnt[e] = 0;
+            } else {
+                cr_give_up(a);
             }
+        };
+        if (nl < 0) {
+            if (threadIdx.x == 0) pass_on(TIER);
             continue;
         }
         const uint32_t total = l.total;
         if (threadIdx.x == 0) {
-            const uint32_t p = atomicAdd(&a.ctl[3], total);
+            const uint32_t p = atomicAdd(&a.ctl[4], total);
             const bool fits = p <= a.region_n && total <= a.region_n - p;
             l.item = fits ? p : ~0u;
             if (fits) {
                 a.cnt[e] = total;
                 a.pos[e] = a.region + p;
             } else {
-                cr_give_up(a);
+                pass_on(2);
             }
         }
         __syncthreads();
@@ -357,17 +363,28 @@ __global__ __launch_bounds__(T) void k_cr_walk_one(CrArgs a, uint32_t cap) {
     }
 }
 
-// result: [0] gave up, [1] pairs, [2 + k] pairs of layer k
+// a.list[2]'s sources as flags of their edges
+__global__ __launch_bounds__(256) void k_cr_rest(CrArgs a, uint32_t n, uint8_t *__restrict__ flags) {
+    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+        uint32_t start = 0;
+        const uint32_t len = cr_run(a, (uint32_t)(a.edge[a.list[2][i]] >> 32), &start);
+        for (uint32_t q = threadIdx.x; q < len; q += 256) flags[start + q] = 1;
+    }
+}
+
+// result: [0] gave up, [1] pairs, [2 + k] sources on list k, [5 + k] pairs of layer k
+constexpr int CR_HEAD = 5;
 __global__ __launch_bounds__(256) void k_cr_result(CrArgs a, const unsigned long long *total, uint64_t *result) {
     const int k = blockIdx.x * 256 + threadIdx.x;
     if (k == 0) {
         result[0] = a.ctl[0];
         result[1] = *total;
+        for (int q = 0; q < 3; ++q) result[2 + q] = a.ctl[1 + q];
     }
     if (k >= CR_LAYERS) return;
     unsigned long long s = 0;
     for (int b = 0; b < CR_BINS; ++b) s += a.layers[k * CR_BINS + b];
-    result[2 + k] = s;
+    result[CR_HEAD + k] = s;
 }
 
 // Closes the gaps: a wave per 64 edges, whose sources' pairs are one span of
@@ -397,7 +414,7 @@ __global__ __launch_bounds__(256) void k_cr_gather(const uint64_t *__restrict__ 
 
 // device bytes closure_rows takes besides the result
 static uint64_t closure_rows_bytes(uint64_t m) {
-    return ((m + CR_EDGES - 1) / CR_EDGES * CR_CAP1 + 16 * m + (1ull << 20)) * 8 + 93 * m + (1ull << 21);
+    return ((m + CR_EDGES - 1) / CR_EDGES * CR_CAP1 + 16 * m + (1ull << 20)) * 8 + 102 * m + (1ull << 21);
 }
 
 bool closure_rows_takes(Ctx *ctx, uint64_t m) {
@@ -405,7 +422,7 @@ bool closure_rows_takes(Ctx *ctx, uint64_t m) {
 }
 
 uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_iter, uint64_t *n,
-                       std::vector<uint64_t> &layers) {
+                       std::vector<uint64_t> &layers, Buf<uint64_t> &rest, uint64_t *rest_n) {
     XH_REQUIRE(m >= 1 && m <= (1ull << 24), XLOG_HIP_INVALID_ARG, "closure rows: relation too large");
     // the runs of E and their table, sized for m runs: no read-back
     RunIndex ix;
@@ -421,9 +438,9 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_
     const uint64_t nb = (m + CR_EDGES - 1) / CR_EDGES;
     const uint64_t region = nb * CR_CAP1, region_n = 16 * m + (1ull << 20);  // both below 2^32
     const uint64_t cap2 = CR_LISTED + nb, cap3 = m / 4096 + 64;
-    Buf<uint64_t> rec(ctx, m), scratch(ctx, region + region_n), result(ctx, 2 + CR_LAYERS);
-    Buf<uint32_t> off(ctx, m + 1), pos(ctx, m), list(ctx, cap2 + cap3);
-    Buf<uint64_t> z(ctx, (uint64_t)(CR_LAYERS + 1) * CR_BINS + 3);  // zeroed: layers, next, ctl, the scan's total
+    Buf<uint64_t> rec(ctx, m), scratch(ctx, region + region_n), result(ctx, CR_HEAD + CR_LAYERS);
+    Buf<uint32_t> off(ctx, m + 1), pos(ctx, m), list(ctx, cap2 + 2 * cap3);
+    Buf<uint64_t> z(ctx, (uint64_t)(CR_LAYERS + 1) * CR_BINS + 4);  // zeroed: layers, next, ctl, the scan's total
     fill_u64(ctx, z.p, 0ull, z.n);
     CrArgs a;
     a.edge = edge;
@@ -440,11 +457,12 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_
     a.ctl = reinterpret_cast<uint32_t *>(a.next + CR_BINS);
     a.list[0] = list.p;
     a.list[1] = list.p + cap2;
+    a.list[2] = list.p + cap2 + cap3;
     a.list_cap[0] = (uint32_t)cap2;
-    a.list_cap[1] = (uint32_t)cap3;
+    a.list_cap[1] = a.list_cap[2] = (uint32_t)cap3;
     a.region = (uint32_t)region;
     a.region_n = (uint32_t)region_n;
-    unsigned long long *total = a.next + CR_BINS + 2;
+    unsigned long long *total = a.next + CR_BINS + 3;
     const unsigned cus = (unsigned)ctx->num_cus;
     hipLaunchKernelGGL(k_cr_records, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, ctx->stream, a);
     hipLaunchKernelGGL(k_cr_gate, dim3(1), dim3(WAVE), 0, ctx->stream, a);
@@ -463,12 +481,16 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_
     XH_CHECK_HIP(hipGetLastError());
     const uint64_t first = 128;
     ctx->read_scalars(result.p, first);
-    if (ctx->host_scalars[0]) return nullptr;
-    const uint64_t pairs = ctx->host_scalars[1];
-    layers.assign(ctx->host_scalars + 2, ctx->host_scalars + first);
+    const uint64_t *h = ctx->host_scalars;
+    if (trace_on())
+        fprintf(stderr, "[xlog_hip] closure walks: %llu sources listed, %llu for the largest sets, %llu handed back%s\n",
+                (unsigned long long)h[2], (unsigned long long)h[3], (unsigned long long)h[4], h[0] ? ": gave up" : "");
+    const uint64_t pairs = h[1], n_rest = h[4];
+    if (h[0] || pairs == 0) return nullptr;
+    layers.assign(h + CR_HEAD, h + first);
     if (layers.back()) {
         layers.resize(CR_LAYERS);
-        XH_CHECK_HIP(hipMemcpyAsync(layers.data(), result.p + 2, CR_LAYERS * sizeof(uint64_t), hipMemcpyDeviceToHost,
+        XH_CHECK_HIP(hipMemcpyAsync(layers.data(), result.p + CR_HEAD, CR_LAYERS * sizeof(uint64_t), hipMemcpyDeviceToHost,
                                     ctx->stream));
         XH_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     }
@@ -479,6 +501,19 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_
                        pos.p, m, out.p);
     XH_CHECK_HIP(hipGetLastError());
     *n = pairs;
+    *rest_n = 0;
+    if (n_rest) {
+        Buf<uint8_t> flags(ctx, m + 3);
+        Buf<uint64_t> cnt(ctx, 1);
+        rest = Buf<uint64_t>(ctx, m);
+        fill_u32(ctx, reinterpret_cast<uint32_t *>(flags.p), 0u, (m + 3) / 4);
+        hipLaunchKernelGGL(k_cr_rest, dim3((unsigned)std::min<uint64_t>(n_rest, 8 * cus)), dim3(256), 0, ctx->stream, a,
+                           (uint32_t)n_rest, flags.p);
+        XH_CHECK_HIP(hipGetLastError());
+        select_flags(ctx, edge, flags.p, m, rest.p, cnt.p);
+        ctx->read_scalars(cnt.p, 1);
+        *rest_n = ctx->host_scalars[0];
+    }
     return out.release();
 }
 

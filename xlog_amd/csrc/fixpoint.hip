@@ -1623,8 +1623,9 @@ struct Driver {
     }
 
     // The closure of one relation, H(X,Z) :- E(X,Z) beside H(X,Z) :- H(X,Y), E(Y,Z) or E(X,Y), H(Y,Z), with H empty
-    // at the start: a walk from every source instead of run_hash's loop (closure_rows.hip).  false, with nothing
-    // done, for other plans, where its scratch is too large for the device and when it gave up.
+    // at the start: a walk from every source instead of run_hash's loop (closure_rows.hip), and that loop for the few
+    // sources that reach too much for it.  false, with nothing done, for other plans, where its scratch is too large
+    // for the device and when it gave up.
     bool run_rows(uint64_t max_iter, std::vector<uint64_t> &deltas, const std::vector<ChainRule> &chains,
                   uint64_t *iterations) {
         if (chains.size() != 2) return false;
@@ -1637,8 +1638,42 @@ struct Driver {
             return false;
         DRel f;
         std::vector<uint64_t> layers;
-        f.k = closure_rows(ctx, full[e].k, full[e].n, max_iter, &f.n, layers);
-        if (!f.k) return false;
+        Buf<uint64_t> rest;
+        uint64_t rest_n = 0;
+        Owned walked(ctx, closure_rows(ctx, full[e].k, full[e].n, max_iter, &f.n, layers, rest, &rest_n));
+        if (!walked.p) return false;
+        if (rest_n) {
+            // H(X,Z) :- S(X,Z).  H(X,Z) :- H(X,Y), E(Y,Z)  from their edges S: the rows of H that the walks left out
+            static const int32_t plan[] = {2, 1, 0, 1, 1, 2, 0, 1, 1, 0, 2, 2, 1, 0, 1, 0, 1, 2};
+            Driver sub{ctx, parse_plan(plan, 3), 3, std::vector<bool>{false, true, false}, std::vector<DRel>(3),
+                       std::vector<DRel>(3)};
+            sub.digits = digits;
+            sub.domain = domain;
+            sub.full[0] = full[e];
+            sub.full[0].owned = false;
+            sub.full[2].k = rest.release();
+            sub.full[2].n = rest_n;
+            sub.full[2].owned = true;
+            for (DRel &r : sub.full) r.version = sub.version_counter++;
+            const std::vector<ChainRule> paths{ChainRule{1, {ChainAtom{2, false}}},
+                                               ChainRule{1, {ChainAtom{1, false}, ChainAtom{0, false}}}};
+            std::vector<uint64_t> more;
+            try {
+                sub.run_hash(max_iter, more, paths);
+                const DRel &g = sub.full[1];
+                Owned both(ctx, alloc_keys(ctx, f.n + g.n));
+                merge_sorted(ctx, walked.p, f.n, g.k, g.n, both.p);
+                walked.reset(both.release());
+                f.n += g.n;
+            } catch (const Error &err) {
+                if (err.code != XLOG_HIP_ITERATION_LIMIT && err.code != XLOG_HIP_OOM) throw;
+                return false;  // (the whole loop reports it)
+            }
+            if (layers.size() < more.size()) layers.resize(more.size(), 0);
+            for (size_t k = 0; k < more.size(); ++k) layers[k] += more[k];
+            while (!layers.empty() && !layers.back()) layers.pop_back();
+        }
+        f.k = walked.release();
         deltas = layers;
         deltas.push_back(0);
         *iterations = layers.size();

@@ -763,10 +763,12 @@ uint64_t closure_columns(Ctx *ctx, const uint64_t *edge, uint64_t m, const uint6
 // packed pairs (a pool block of the caller's) and the new tuples of each
 // iteration, E's own first, up to the last non-empty one; nullptr (nothing
 // done) when sources reach too much for it or the iterations pass max_iter.
+// The edges of a few sources that reach too much come back in rest (*rest_n of
+// them, sorted): nothing of theirs is in the result and the iterations.
 // closure_rows_takes: the sizes it takes, within the device's room.
 bool closure_rows_takes(Ctx *ctx, uint64_t m);
 uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_iter, uint64_t *n,
-                       std::vector<uint64_t> &layers);
+                       std::vector<uint64_t> &layers, Buf<uint64_t> &rest, uint64_t *rest_n);
 
 // Arrow IPC stream codec for relations of 1..4 UInt32 columns (arrow_ipc.cpp,
 // host code).  decode checks the stream and returns pointers to the column
