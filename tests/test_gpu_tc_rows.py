@@ -132,7 +132,7 @@ def test_layers_of_single_sources(provider, lists, layers):
     assert lists() == (max(0, layers - 128), max(0, layers - 512), 0)
 
 
-@pytest.mark.parametrize("n_back", [1, 3, 20])
+@pytest.mark.parametrize("n_back", [1, 3, 20, 60])
 def test_sources_handed_back(provider, lists, n_back):
     """Sources that outgrow the largest sets, and ones that reach them, go through the loop over hash sets; the others
     stay with the walks.  Cycles and long paths among both, so that either part has the more iterations."""

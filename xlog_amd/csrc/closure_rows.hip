@@ -25,8 +25,8 @@
 // when they are many the attempt ends early and the caller goes on with its loop
 // over hash sets.  A few that outgrow the largest set are handed back instead:
 // the caller's loop then runs from their edges alone (when one of them ended the
-// attempt, a source with 10,000 edges among 2^19 others cost STAR_BEFORE us
-// where the loop alone took 1,300; so STAR_NOW).
+// attempt, a source with 10,000 edges among 2^19 others cost 1,523 us
+// where the loop alone took 1,300; so 688).
 #include "internal.hpp"
 #include "host.hpp"
 
@@ -39,10 +39,13 @@ namespace {
 constexpr int CR_EDGES = 24;  // rows of E whose sources one wave walks together: about 16 sources at 1.5 rows each
 constexpr int CR_ROWS = 32;
 constexpr uint32_t CR_CAP1 = 896, CR_CAP2 = 1792, CR_CAP3 = 7168;  // pairs: 7/8 of the tiers' sets
-// Sources listed up to batch b: at most CR_LISTED + b, one batch in 16 or so.  At 0.9 edges a vertex 1 % of the
-// batches are listed; at 0.95 a fifth would be, and the tiers after the first are then no faster than the hash loop
-// (2^20 vertices and as many edges: 18 ms in the second tier before it gave up, of a call of 83 ms without it).
-constexpr uint32_t CR_LISTED = 512;
+// Sources listed up to batch b: at most CR_LISTED and one a batch (one batch in 16 or so) of b, or of CR_AT_ONCE where
+// that is more.  At 0.9 edges a vertex 1 % of the batches are listed; at 0.95 a fifth would be, and the tiers after the
+// first are then no faster than the hash loop (2^20 vertices and as many edges: 18 ms in the second tier before it gave
+// up, of a call of 83 ms without it).  CR_AT_ONCE is about as many batches as run at a time, and those of the first ones
+// that are still walking when many have begun: with CR_LISTED + b alone, one of these that failed late could end an
+// attempt that lists 2,000 sources in all (2^20 vertices at 0.9 edges: 1.1 or 5.2 ms, as it happened).
+constexpr uint32_t CR_LISTED = 512, CR_AT_ONCE = 4096;
 constexpr int CR_LAYERS = 4096;                                    // layers of the largest tier
 constexpr int CR_BINS = 32;                                        // copies of the layer counters
 constexpr uint64_t CR_EMPTY = ~0ull;                               // no pair is: its row is below CR_ROWS
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
     at = __shfl(at, 0, WAVE) + (uint32_t)row;
     if (!head) return;
     // batches begin about in order, so a graph whose sources reach too much ends the attempt in its first batches
-    if (at < CR_LISTED + (uint32_t)b)
+    if (at < min(CR_LISTED + max((uint32_t)b, CR_AT_ONCE), a.list_cap[0]))
         a.list[0][at] = (uint32_t)e;
     else
         cr_give_up(a);
