@@ -1500,16 +1500,19 @@ struct KeyPack {
 };
 constexpr uint64_t NO_KEY = ~0ull;  // a probe row without a match (keys packed from several columns are below 2^31)
 namespace {
-// A bijection of the 31-bit keys.  Keys packed side by side repeat the columns'
-// patterns, which the table's multiplicative hash keeps: their runs then crowd
-// in the table (2^20 keys of 21 + 6 bits: insert 0.11 ms, count 0.12; mixed 0.06
-// and 0.10).
+// A bijection of the 31-bit keys: two rounds of multiplicative hashing (Knuth,
+// The Art of Computer Programming, vol. 3, 6.4) with the upper half of the bits
+// folded into the lower after each; the odd multipliers are 2^31 times the
+// fractions of the golden ratio and of the square root of two.  Keys packed side
+// by side repeat the columns' patterns, which the table's own multiplicative
+// hash keeps: their runs then crowd in the table (2^20 keys of 21 + 6 bits:
+// insert 0.11 ms, count 0.12; mixed 0.06 and 0.10).
 __device__ __forceinline__ uint32_t mix_key(uint32_t x) {
     constexpr uint32_t M = 0x7FFFFFFFu;
-    x = (x * 0x2C1B3C6Du) & M;
-    x ^= x >> 15;
-    x = (x * 0x297A2D39u) & M;
-    return x ^ (x >> 14);
+    x = (x * 0x4F1BBCDDu) & M;
+    x ^= x >> 16;
+    x = (x * 0x3504F335u) & M;
+    return x ^ (x >> 16);
 }
 // (packed key << 32) | row
 __global__ void k_pack_rows(RelView in, KeyPack kp, uint64_t n, uint64_t *__restrict__ out) {
