@@ -117,9 +117,11 @@ __global__ __launch_bounds__(256) void k_read_back(const uint64_t *__restrict__ 
 }
 }  // namespace
 void Ctx::post_read(const void *dev, size_t count_u64, const uint64_t *also) {
-    XH_REQUIRE(count_u64 + (also ? 1 : 0) <= HOST_STAGE_U64, XLOG_HIP_INVALID_ARG, "read-back: more than the pinned staging holds");
+    XH_REQUIRE(count_u64 + (also ? 1 : 0) <= HOST_STAGE_U64, XLOG_HIP_INVALID_ARG,
+               "read-back: more than the pinned staging holds");
     hipLaunchKernelGGL(k_read_back, dim3(1), dim3(count_u64 > 64 ? 256 : 64), 0, stream,
-                       static_cast<const uint64_t *>(dev), (uint32_t)count_u64, host_scalars, also, host_seq, ++read_seq);
+                       static_cast<const uint64_t *>(dev), (uint32_t)count_u64, host_scalars, also, host_seq,
+                       ++read_seq);
     XH_CHECK_HIP(hipGetLastError());
 }
 void Ctx::wait_read() {
@@ -560,7 +562,8 @@ struct KeyBits {
     int col[MAX_ARITY] = {0}, len[MAX_ARITY] = {0};  // distinct columns, bits they use
     bool known = true;                               // (or may use)
 };
-struct KeyPiece {  // bits [lo, lo + bits) of the number, at the top of 64; the row's number in row_bits from row_shift up
+// bits [lo, lo + bits) of the number, at the top of 64; the row's number in row_bits from row_shift up
+struct KeyPiece {
     int n = 0, bits = 0;
     int col[MAX_ARITY] = {0}, rs[MAX_ARITY] = {0}, ls[MAX_ARITY] = {0};
     uint32_t mask[MAX_ARITY] = {0};
@@ -572,7 +575,8 @@ namespace {
 template <int W>
 __global__ __launch_bounds__(256) void k_key_pieces(RelView in, KeyPiece kp, uint64_t n, uint64_t *__restrict__ out,
                                                     uint64_t *__restrict__ aos, const uint64_t *__restrict__ prev,
-                                                    int prev_shift, const uint32_t *__restrict__ group, int group_bits) {
+                                                    int prev_shift, const uint32_t *__restrict__ group,
+                                                    int group_bits) {
     const uint64_t stride = (uint64_t)gridDim.x * 256;
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
         const uint64_t r = prev ? (prev[i] >> prev_shift) & ((1ull << kp.row_bits) - 1) : i;
@@ -603,8 +607,8 @@ __device__ __forceinline__ int compare_rows(const uint64_t *a, const uint64_t *b
 // run is only a group).  With pos, row i of the order goes to place pos[i].
 template <int W>
 __global__ __launch_bounds__(ROWS_TB) void k_sorted_rows(const uint64_t *__restrict__ sorted, KeyPiece kp, uint64_t n,
-                                                         const uint64_t *__restrict__ aos, KeyBits kb, int arity, int ties,
-                                                         RelOut out, uint8_t *__restrict__ flags, uint64_t *d_long,
+                                                         const uint64_t *__restrict__ aos, KeyBits kb, int arity,
+                                                         int ties, RelOut out, uint8_t *__restrict__ flags, uint64_t *d_long,
                                                          const uint32_t *__restrict__ pos) {
     constexpr int SPAN = ROWS_TILE + RUN_MAX + 1;  // (one past the longest run shows its end)
     __shared__ uint64_t s_key[SPAN];
@@ -684,7 +688,8 @@ __global__ void k_take_rows(const uint64_t *__restrict__ in, const uint32_t *__r
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) out[i] = in[rows[i]];
 }
 // in_long[i] = 1 for the sorted words whose run of equal prefix has more than RUN_MAX (in_long[n] = 0: n + 1 entries)
-__global__ void k_long_runs(const uint64_t *__restrict__ sorted, KeyPiece kp, uint64_t n, uint32_t *__restrict__ in_long) {
+__global__ void k_long_runs(const uint64_t *__restrict__ sorted, KeyPiece kp, uint64_t n,
+                            uint32_t *__restrict__ in_long) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     const int shift = 64 - kp.bits;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i <= n; i += stride) {
@@ -768,7 +773,8 @@ struct LongRuns {
     Buf<uint32_t> pos, group;
     uint64_t n = 0, groups = 0;
 };
-static void long_runs(Ctx *ctx, const uint64_t *sorted, const KeyPiece &kp, uint64_t n, const uint32_t *pos, LongRuns &out) {
+static void long_runs(Ctx *ctx, const uint64_t *sorted, const KeyPiece &kp, uint64_t n, const uint32_t *pos,
+                      LongRuns &out) {
     Buf<uint32_t> in_long(ctx, n + 1);
     Buf<unsigned long long> sum(ctx, 1);
     LAUNCH_1D(k_long_runs, n + 1, sorted, kp, n, in_long.p);
@@ -786,8 +792,9 @@ template <int W>
 static void fetch_rows(Ctx *ctx, const xlog_hip_rel *in, const KeyBits &kb, const uint64_t *w, const KeyPiece &kp,
                        uint64_t n, const uint64_t *aos, bool ties, xlog_hip_rel *out, uint8_t *flags,
                        uint64_t *d_long, const uint32_t *pos) {
-    hipLaunchKernelGGL(k_sorted_rows<W>, dim3((unsigned)((n + ROWS_TILE - 1) / ROWS_TILE)), dim3(ROWS_TB), 0, ctx->stream,
-                       w, kp, n, W > 1 ? aos : in->w[0], kb, (int)in->arity, ties ? 1 : 0, out_of(out), flags, d_long, pos);
+    hipLaunchKernelGGL(k_sorted_rows<W>, dim3((unsigned)((n + ROWS_TILE - 1) / ROWS_TILE)), dim3(ROWS_TB), 0,
+                       ctx->stream, w, kp, n, W > 1 ? aos : in->w[0], kb, (int)in->arity, ties ? 1 : 0, out_of(out),
+                       flags, d_long, pos);
     XH_CHECK_HIP(hipGetLastError());
 }
 // By prefixes; false where pieces of the whole key are the better way on.  The
@@ -1217,8 +1224,8 @@ static int join_values(const xlog_hip_rel *l, uint32_t r_arity, uint32_t rk, con
 // SEMI / ANTI: the rows of l whose key is / is not among the right side's (the
 // key words pcol of l's probe rows and rcol of the right rows).  Only the keys
 // matter, so they go into a hash set as they are: no sort, no runs.
-static xlog_hip_rel *key_set_join(Ctx *ctx, const xlog_hip_rel *l, const uint64_t *probe, int pcol, const uint64_t *rows,
-                                  uint64_t nr, int rcol, int type, bool canonical) {
+static xlog_hip_rel *key_set_join(Ctx *ctx, const xlog_hip_rel *l, const uint64_t *probe, int pcol,
+                                  const uint64_t *rows, uint64_t nr, int rcol, int type, bool canonical) {
     Buf<unsigned long long> set;
     key_set_build(ctx, rows, nr, rcol, set);
     Buf<uint8_t> flags(ctx, l->rows);
@@ -1317,7 +1324,8 @@ struct JoinMap {
     int kind[MAX_ARITY] = {0}, col[MAX_ARITY] = {0};
 };
 // output row r from the pair (left row << 32) | payload
-__global__ void k_join_rows(RelView L, RelView R, JoinMap m, const uint64_t *__restrict__ pairs, uint64_t n, RelOut out) {
+__global__ void k_join_rows(RelView L, RelView R, JoinMap m, const uint64_t *__restrict__ pairs, uint64_t n,
+                            RelOut out) {
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride) {
         const uint64_t pr = pairs[r];
@@ -1480,8 +1488,8 @@ static xlog_hip_rel *direct_join_wide_left(Ctx *ctx, const xlog_hip_rel *l, uint
     if (max_output && n > max_output) n = max_output;
     std::unique_ptr<xlog_hip_rel, void (*)(xlog_hip_rel *)> o(rel_new(ctx, arity, n), rel_free);
     o->rows = n;
-    LAUNCH_1D(k_join_rows, n, view_of(l), view_of(l), join_map(l, r_arity, {(int)lk}, {(int)rk}, r_arity == 2 ? 1 - (int)rk : -1),
-              w, n, out_of(o.get()));
+    LAUNCH_1D(k_join_rows, n, view_of(l), view_of(l),
+              join_map(l, r_arity, {(int)lk}, {(int)rk}, r_arity == 2 ? 1 - (int)rk : -1), w, n, out_of(o.get()));
     return o.release();
 }
 
@@ -1617,14 +1625,16 @@ static void build_row_index(Ctx *ctx, const xlog_hip_rel *r, const KeyPack &kp, 
     J.ix.table = Buf<unsigned long long>(ctx, 2 * slots);
     J.ix.table_mask = slots - 1;
     J.ix.nruns = n;  // (a bound)
-    // (after a sort that did not fit, the runs are of words that repeat anyhow, and inserting those would probe on and on)
+    // (after a sort that did not fit, the runs are of words that repeat anyhow, and inserting those would probe on and
+    // on)
     run_index_insert_dev(ctx, run_key.p, run_start.p, cnt.p, n, cnt.p + 1, J.ix,
                          *over ? reinterpret_cast<const uint32_t *>(*over) : nullptr);
 }
 // One key column: up to 3 * 2^17 rows.  Beyond, the digit passes, few when the keys have few bits, and a table sized by
 // the runs found take less (10^6 rows a side, by buckets and by digit passes: Zipf keys 213 / 157 us, 1,000 keys 162 /
 // 117, ids 208 / 196, hashed 272 / 275; 4 * 10^5 rows: 153 / 138, 108 / 106, 131 / 143, 158 / 187).  Keys packed from
-// several columns have most of 31 bits: buckets as far as they go (10^6 rows on ids and a column of 64 values 294 / 327).
+// several columns have most of 31 bits: buckets as far as they go (10^6 rows on ids and a column of 64 values 294 /
+// 327).
 static bool small_build(uint64_t n, int key_cols) {
     return n <= BLOCK_SORT_KEYS || ((key_cols > 1 || n <= (3ull << 17)) && bucket_sort_takes(n));
 }
@@ -1751,8 +1761,8 @@ static xlog_hip_rel *op_join(Ctx *ctx, const xlog_hip_rel *l, const xlog_hip_rel
         uint64_t n = 0;
         // (its table is sized for as many runs as rows: without room for that, the index below)
         if (fits_memory([&] {
-                n = row_index_join(ctx, l->w[0], l->rows, pcol, r, kp, r->arity == 2 ? 1 - (int)rk : -1, out_arity, oc, o0,
-                                   o1);
+                n = row_index_join(ctx, l->w[0], l->rows, pcol, r, kp, r->arity == 2 ? 1 - (int)rk : -1, out_arity, oc,
+                                   o0, o1);
             })) {
             if (n == 0) return rel_new(ctx, (uint32_t)out_arity, 0);
             return rel_adopt(ctx, (uint32_t)out_arity, n, o0.release(), o1.release(), 0);

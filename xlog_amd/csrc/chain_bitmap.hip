@@ -1175,7 +1175,8 @@ void chain_fixpoint(Ctx *ctx, const std::vector<ChainRule> &rules, uint32_t n_pr
                 *iterations = deltas.size() - 1;
                 XH_REQUIRE(converged, XLOG_HIP_ITERATION_LIMIT,
                            "Recursive SCC iteration limit (" + std::to_string(max_iter) + ") exceeded");
-                out_n[seed_h] = bitmap_emit(ctx, R.p, domain, words, &out[seed_h], XLOG_HIP_KERNEL_CHAIN_EMIT, total, rc.p);
+                out_n[seed_h] = bitmap_emit(ctx, R.p, domain, words, &out[seed_h], XLOG_HIP_KERNEL_CHAIN_EMIT, total,
+                                            rc.p);
                 return;
             }
         }

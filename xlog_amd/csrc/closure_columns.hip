@@ -82,7 +82,8 @@ __device__ __forceinline__ uint32_t bin_take(uint32_t *bins, uint32_t bin, bool 
 }
 
 // Rows per out-degree bin.
-__global__ __launch_bounds__(256) void k_cl_bins(const uint64_t *__restrict__ row_ptr, uint32_t domain, uint32_t *bins) {
+__global__ __launch_bounds__(256) void k_cl_bins(const uint64_t *__restrict__ row_ptr, uint32_t domain,
+                                                 uint32_t *bins) {
     __shared__ uint32_t s_bin[CL_DEG_BINS];
     const int lane = threadIdx.x & (WAVE - 1);
     for (int i = threadIdx.x; i < CL_DEG_BINS; i += 256) s_bin[i] = 0;
@@ -338,7 +339,8 @@ __global__ __launch_bounds__(CL_TB) void k_cl_columns(ClArgs a) {
                 for (int q = 0; q < 4; ++q) {
                     const uint64_t bal = __ballot(t[q] != 0);
                     cnt += (uint32_t)__popc(t[q]);
-                    before += __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+                    before += __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
                     total += (uint32_t)__popcll(bal);
                 }
                 if (!total) return;
@@ -437,7 +439,8 @@ __global__ __launch_bounds__(CL_TB) void k_cl_columns(ClArgs a) {
 #pragma unroll
                     for (int j = 0; j < GRP; ++j) {
                         const uint32_t mj = (uint32_t)__builtin_amdgcn_readlane((int)my_m, i0 + j);
-                        if (mj & CL_HEAVY) acc[j] = heavy_slice(a, s_r, (uint32_t)((i0 + j) * CL_WAVES + wave) * WAVE, ln);
+                        if (mj & CL_HEAVY)
+                            acc[j] = heavy_slice(a, s_r, (uint32_t)((i0 + j) * CL_WAVES + wave) * WAVE, ln);
                         // (its group's light slices, past the depth that CL_HEAVY hides)
                         for (uint32_t k = 1; !(mj & CL_HEAVY) && k < mj; ++k) acc[j] |= read_quad(load_quad(i0 + j, k));
                     }
@@ -547,8 +550,8 @@ __global__ __launch_bounds__(256) void k_cl_transpose(const uint32_t *__restrict
 // 1.16 and 2.4 / 3.7 ms); 500 a row (1,000 x 1,000 complete bipartite) 0.64 / 0.33.
 bool closure_columns_fits(uint32_t domain, uint64_t edges, uint64_t seeds) {
     const uint64_t per_row = domain >= 12288 ? 64 : 32;
-    return domain <= (uint32_t)CL_MAX_RPT * CL_TB && edges <= std::min<uint64_t>(per_row * domain, CLOSURE_COLUMNS_EDGES) &&
-           seeds <= CLOSURE_COLUMNS_EDGES;
+    return domain <= (uint32_t)CL_MAX_RPT * CL_TB &&
+           edges <= std::min<uint64_t>(per_row * domain, CLOSURE_COLUMNS_EDGES) && seeds <= CLOSURE_COLUMNS_EDGES;
 }
 
 uint64_t closure_columns(Ctx *ctx, const uint64_t *edge, uint64_t m, const uint64_t *row_ptr, const uint32_t *adj,
@@ -583,8 +586,8 @@ uint64_t closure_columns(Ctx *ctx, const uint64_t *edge, uint64_t m, const uint6
     hipLaunchKernelGGL(k_cl_bins, dim3(grid_for(domain, 256, 128)), dim3(256), 0, ctx->stream, row_ptr, domain, bins);
     hipLaunchKernelGGL(k_cl_place, dim3((domain + CL_TB - 1) / CL_TB), dim3(CL_TB), 0, ctx->stream, row_ptr, domain,
                        bins, cursor, perm.p, inv.p);
-    hipLaunchKernelGGL(k_cl_in_degrees, dim3(grid_for(std::max(m, n_seed), 256, 1024)), dim3(256), 0, ctx->stream, adj, m,
-                       own_seed ? seed : nullptr, n_seed, inv.p, in_ptr, seed_ptr, rank.p, seed_rank.p);
+    hipLaunchKernelGGL(k_cl_in_degrees, dim3(grid_for(std::max(m, n_seed), 256, 1024)), dim3(256), 0, ctx->stream, adj,
+                       m, own_seed ? seed : nullptr, n_seed, inv.p, in_ptr, seed_ptr, rank.p, seed_rank.p);
     XH_CHECK_HIP(hipGetLastError());
     scan_u32_inplace(ctx, in_ptr, d1, sum.p);
     if (own_seed) scan_u32_inplace(ctx, seed_ptr, d1, sum.p);

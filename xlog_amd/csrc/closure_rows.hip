@@ -42,9 +42,9 @@ constexpr uint32_t CR_CAP1 = 896, CR_CAP2 = 1792, CR_CAP3 = 7168;  // pairs: 7/8
 // Sources listed up to batch b: at most CR_LISTED and one a batch (one batch in 16 or so) of b, or of CR_AT_ONCE where
 // that is more.  At 0.9 edges a vertex 1 % of the batches are listed; at 0.95 a fifth would be, and the tiers after the
 // first are then no faster than the hash loop (2^20 vertices and as many edges: 18 ms in the second tier before it gave
-// up, of a call of 83 ms without it).  CR_AT_ONCE is about as many batches as run at a time, and those of the first ones
-// that are still walking when many have begun: with CR_LISTED + b alone, one of these that failed late could end an
-// attempt that lists 2,000 sources in all (2^20 vertices at 0.9 edges: 1.1 or 5.2 ms, as it happened).
+// up, of a call of 83 ms without it).  CR_AT_ONCE is about as many batches as run at a time: one of the first may fail
+// when many have begun, and with CR_LISTED + b alone it could end an attempt that lists 2,000 sources in all (2^20
+// vertices at 0.9 edges: 1.1 or 5.2 ms, as it happened).
 constexpr uint32_t CR_LISTED = 512, CR_AT_ONCE = 4096;
 constexpr int CR_LAYERS = 4096;                                    // layers of the largest tier
 constexpr int CR_BINS = 32;                                        // copies of the layer counters
@@ -486,15 +486,16 @@ uint64_t *closure_rows(Ctx *ctx, const uint64_t *edge, uint64_t m, uint64_t max_
     ctx->read_scalars(result.p, first);
     const uint64_t *h = ctx->host_scalars;
     if (trace_on())
-        fprintf(stderr, "[xlog_hip] closure walks: %llu sources listed, %llu for the largest sets, %llu handed back%s\n",
+        fprintf(stderr,
+                "[xlog_hip] closure walks: %llu sources listed, %llu for the largest sets, %llu handed back%s\n",
                 (unsigned long long)h[2], (unsigned long long)h[3], (unsigned long long)h[4], h[0] ? ": gave up" : "");
     const uint64_t pairs = h[1], n_rest = h[4];
     if (h[0] || pairs == 0) return nullptr;
     layers.assign(h + CR_HEAD, h + first);
     if (layers.back()) {
         layers.resize(CR_LAYERS);
-        XH_CHECK_HIP(hipMemcpyAsync(layers.data(), result.p + CR_HEAD, CR_LAYERS * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                                    ctx->stream));
+        XH_CHECK_HIP(hipMemcpyAsync(layers.data(), result.p + CR_HEAD, CR_LAYERS * sizeof(uint64_t),
+                                    hipMemcpyDeviceToHost, ctx->stream));
         XH_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     }
     while (!layers.empty() && !layers.back()) layers.pop_back();

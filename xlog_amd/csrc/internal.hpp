@@ -306,17 +306,18 @@ void rel_free(xlog_hip_rel *r);
 // stream-ordered on ctx->stream.
 // ---------------------------------------------------------------------------
 
-// LSD radix sort of u64 keys, stable, over the 8-bit digits [digit_lo, digit_hi) (0..8 = the whole key; 4..8 = the high
-// word only).  On return *keys points at whichever of the two buffers holds
-// the result; the other is scratch.  The pass of the lowest
-// digit always runs (it is queued before the histograms are read back); every
-// higher digit that is constant over the input is skipped.  A keys-only sort
+// LSD radix sort of u64 keys, stable, over the 8-bit digits [digit_lo,
+// digit_hi) (0..8 = the whole key; 4..8 = the high word only).  On return *keys
+// points at whichever of the two buffers holds the result; the other is
+// scratch.  The pass of the lowest digit always runs (it is queued before the
+// histograms are read back); every higher digit that is constant over the input
+// is skipped.  A keys-only sort
 // of the whole key over at least 2^22 keys instead waits for the histograms,
 // and when they predict that the high word leaves runs of a few keys, runs
 // the high word's passes and one sort_short_runs pass (the low word's passes
 // only if some run exceeds 256 keys).  Returns the number of passes executed.
-// With `src` the first pass reads src and both buffers are
-// scratch, so an input that must not be modified is never copied first.
+// With `src` the first pass reads src and both buffers are scratch, so an input
+// that must not be modified is never copied first.
 // With known_digits (a bitmask of digits that may vary, e.g. from the value
 // domain) the passes are exactly those digits of [digit_lo, digit_hi) and the
 // histograms are not read back (a known digit that turns out constant costs a

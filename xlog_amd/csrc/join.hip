@@ -731,7 +731,9 @@ __global__ __launch_bounds__(JB) void k_wcoj_triangle(const uint64_t *__restrict
 
 // A set of u32 keys for semi and anti joins, which need no runs: 8-byte slots
 // (1 << 32) | key, 0 empty, linear probing.
-__device__ __forceinline__ uint32_t key_of_row(uint64_t row, int pcol) { return pcol ? (uint32_t)row : (uint32_t)(row >> 32); }
+__device__ __forceinline__ uint32_t key_of_row(uint64_t row, int pcol) {
+    return pcol ? (uint32_t)row : (uint32_t)(row >> 32);
+}
 // A workgroup inserts a key once, more or less: the last keys that its threads
 // took on are in LDS, and a thread that finds its key there leaves it to the
 // thread that put it there.  Hub keys otherwise send most threads to one line of

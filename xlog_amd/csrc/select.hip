@@ -1794,9 +1794,10 @@ bool diff_by_merge(Ctx *ctx, const uint64_t *k, uint64_t n, const uint64_t *b, u
             flags = Buf<uint8_t>(ctx, n);
         }))
         return false;
-    hipLaunchKernelGGL(k_merge_partition, dim3((unsigned)((tiles + 1 + 255) / 256)), dim3(256), 0, ctx->stream, b, nb, k, n,
-                       tiles, split.p, MergeDev{});
-    hipLaunchKernelGGL(k_merge_absent, dim3((unsigned)tiles), dim3(MRG_BLOCK), 0, ctx->stream, b, nb, k, n, split.p, flags.p);
+    hipLaunchKernelGGL(k_merge_partition, dim3((unsigned)((tiles + 1 + 255) / 256)), dim3(256), 0, ctx->stream, b, nb, k,
+                       n, tiles, split.p, MergeDev{});
+    hipLaunchKernelGGL(k_merge_absent, dim3((unsigned)tiles), dim3(MRG_BLOCK), 0, ctx->stream, b, nb, k, n, split.p,
+                       flags.p);
     XH_CHECK_HIP(hipGetLastError());
     select_flags(ctx, k, flags.p, n, out, d_count);
     return true;

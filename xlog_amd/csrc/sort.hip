@@ -21,9 +21,9 @@
 //      word's digits take passes; k_sort_short_runs then orders every run of
 //      equal high word by its low word in one more pass (4 + 1 passes over
 //      uniform keys instead of 8).
-// Each pass reads and writes every key exactly once (16 B per key).  Tiles go to the XCDs in chunks of consecutive
-// tiles, so that neighbouring tiles share an L2, and a tile only ever waits
-// for tiles of earlier-dispatched blocks.
+// Each pass reads and writes every key exactly once (16 B per key).  Tiles go to
+// the XCDs in chunks of consecutive tiles, so that neighbouring tiles share an
+// L2, and a tile only ever waits for tiles of earlier-dispatched blocks.
 #include "internal.hpp"
 #include "short_runs.hpp"
 
@@ -437,14 +437,17 @@ __global__ __launch_bounds__(BS_TB) void k_block_sort(const uint64_t *in, uint32
 // can fill another bucket, which sets `over`: the caller then takes the digit
 // passes.  The buckets are filled in arrival order (whole keys: it does not show).
 constexpr int BK_TB = 512, BK_ITEMS = 8, BK_KEYS = BK_TB * BK_ITEMS, BK_MAX_BITS = 10;
-constexpr uint32_t BK_SAMPLE = 8 << BK_MAX_BITS;  // eight keys per bucket: the fullest holds about 2.5 times the average
+// eight keys per bucket: the fullest holds about 2.5 times the average
+constexpr uint32_t BK_SAMPLE = 8 << BK_MAX_BITS;
 struct BucketState {
     uint32_t over, pad;
     uint32_t cursor[1 << BK_MAX_BITS], uniq[1 << BK_MAX_BITS];  // keys, unique keys of each bucket
     uint64_t bound[1 << BK_MAX_BITS];  // bucket b holds the keys x with bound[b - 1] <= x < bound[b]
 };
 // bucket b holds one value, bound[b]: its bounds are equal (the last bound is the largest key)
-__device__ __forceinline__ bool bucket_of_one(const uint64_t *bound, uint32_t b) { return b > 0 && bound[b - 1] == bound[b]; }
+__device__ __forceinline__ bool bucket_of_one(const uint64_t *bound, uint32_t b) {
+    return b > 0 && bound[b - 1] == bound[b];
+}
 __global__ __launch_bounds__(BS_TB) void k_bucket_sample(const uint64_t *__restrict__ in, uint64_t n, BucketState *st,
                                                          int bits, uint64_t *__restrict__ sample) {
     __shared__ BsSmem<BS_TB, BK_SAMPLE / BS_TB> sm;
@@ -604,7 +607,8 @@ __global__ __launch_bounds__(BK_TB) void k_bucket_gather(const uint64_t *__restr
     const uint32_t n = st->uniq[t];
     uint64_t k[BK_ITEMS];
 #pragma unroll
-    for (int r = 0; r < BK_ITEMS; ++r) k[r] = r * BK_TB + tid < n ? regions[(uint64_t)t * BK_KEYS + r * BK_TB + tid] : 0ull;
+    for (int r = 0; r < BK_ITEMS; ++r)
+        k[r] = r * BK_TB + tid < n ? regions[(uint64_t)t * BK_KEYS + r * BK_TB + tid] : 0ull;
     uint32_t before = 0;
     for (uint32_t i = tid; i < t; i += BK_TB) before += st->uniq[i];
     before = bucket_block_total(before, s_part);
@@ -659,8 +663,8 @@ __device__ uint32_t tile_digit_count(const uint64_t *__restrict__ kin, uint64_t 
 // of that predecessor, and under in-order dispatch the bound is never reached.
 template <int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) void k_onesweep(
-    const uint64_t *__restrict__ kin, uint64_t *__restrict__ kout, uint64_t n, uint32_t tiles, int shift, const uint32_t *__restrict__ digit_off,
-    uint32_t *status, uint32_t *status_next, uint32_t chunk, unsigned long long *ticket,
+    const uint64_t *__restrict__ kin, uint64_t *__restrict__ kout, uint64_t n, uint32_t tiles, int shift,
+    const uint32_t *__restrict__ digit_off, uint32_t *status, uint32_t *status_next, uint32_t chunk, unsigned long long *ticket,
     unsigned long long ticket_base, const uint64_t *d_n, const uint32_t *stop, uint32_t spin_limit) {
     __shared__ uint32_t s_wcnt[(BLOCK / WAVE)][256];
     __shared__ uint32_t s_ticket;
@@ -1221,8 +1225,8 @@ bool bucket_sort(Ctx *ctx, const uint64_t *in, uint64_t n, uint64_t *out, uint64
     BucketState *st = reinterpret_cast<BucketState *>(state.p);
     // (the sample's keys pass through the regions, which the scatter fills afterwards)
     hipLaunchKernelGGL(k_bucket_sample, dim3(1), dim3(BS_TB), 0, ctx->stream, in, n, st, bits, regions.p);
-    hipLaunchKernelGGL(k_bucket_scatter, dim3((unsigned)((n + BC_TB * BC_ITEMS - 1) / (BC_TB * BC_ITEMS))), dim3(BC_TB), 0,
-                       ctx->stream, in, n, st, bits, regions.p);
+    hipLaunchKernelGGL(k_bucket_scatter, dim3((unsigned)((n + BC_TB * BC_ITEMS - 1) / (BC_TB * BC_ITEMS))),
+                       dim3(BC_TB), 0, ctx->stream, in, n, st, bits, regions.p);
     Prof prof(ctx, XLOG_HIP_KERNEL_SORT_SEGMENTS, 16.0 * (double)n);
     if (d_count) {
         hipLaunchKernelGGL(k_bucket_sort<true>, dim3(1u << bits), dim3(BK_TB), 0, ctx->stream, regions.p, st, out);
