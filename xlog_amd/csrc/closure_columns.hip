@@ -101,17 +101,49 @@ __global__ __launch_bounds__(256) void k_cl_bins(const uint64_t *__restrict__ ro
 
 // Edges per target (in_deg, by internal row) and each edge's rank among its
 // target's (any order), and the same of the seed pairs when they are not the
-// edges.  One atomic per edge, which also spares the lists' fill its own (on
-// hub targets they wait for each other).
+// edges.  One atomic per edge, which also spares the lists' fill its own, or one
+// for the edges of a wave to a hub target: hubs' atomics wait for each other
+// (30,000 vertices, 90,000 edges, 55 % of them to one target: the closure 858 us
+// with an atomic each, 719 so, by row gathers 673).
+__device__ __forceinline__ uint32_t take_rank(uint32_t *count, uint32_t z, bool valid, int lane) {
+    constexpr int TRIES = 4, MANY = 8;  // targets looked at, edges of the wave that make one a hub
+    uint32_t rank = 0;
+    uint64_t todo = __ballot(valid);
+    for (int r = 0; r < TRIES && todo; ++r) {
+        const uint32_t hub = (uint32_t)__builtin_amdgcn_readlane((int)z, __ffsll((unsigned long long)todo) - 1);
+        const uint64_t m = __ballot(valid && z == hub);
+        todo &= ~m;
+        if (__popcll(m) < MANY) continue;  // wave-uniform
+        uint32_t base = 0;
+        const int first = __ffsll((unsigned long long)m) - 1;
+        if (lane == first) base = atomicAdd(&count[hub], (uint32_t)__popcll(m));
+        base = (uint32_t)__builtin_amdgcn_readlane((int)base, first);
+        if ((m >> lane) & 1ull) {
+            rank = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            valid = false;
+        }
+    }
+    if (valid) rank = atomicAdd(&count[z], 1u);
+    return rank;
+}
 __global__ __launch_bounds__(256) void k_cl_in_degrees(const uint32_t *__restrict__ adj, uint64_t m,
                                                        const uint64_t *__restrict__ seed, uint64_t n_seed,
                                                        const uint16_t *__restrict__ inv, uint32_t *in_deg,
                                                        uint32_t *seed_deg, uint32_t *__restrict__ rank,
                                                        uint32_t *__restrict__ seed_rank) {
+    const int lane = threadIdx.x & (WAVE - 1);
     const uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x, stride = (uint64_t)gridDim.x * 256;
-    for (uint64_t e = t; e < m; e += stride) rank[e] = atomicAdd(&in_deg[inv[adj[e]]], 1u);
-    if (seed)
-        for (uint64_t e = t; e < n_seed; e += stride) seed_rank[e] = atomicAdd(&seed_deg[inv[(uint32_t)seed[e]]], 1u);
+    for (uint64_t b = t - lane; b < m; b += stride) {
+        const uint64_t e = b + lane;
+        const uint32_t r = take_rank(in_deg, e < m ? inv[adj[e]] : 0u, e < m, lane);
+        if (e < m) rank[e] = r;
+    }
+    if (!seed) return;
+    for (uint64_t b = t - lane; b < n_seed; b += stride) {
+        const uint64_t e = b + lane;
+        const uint32_t r = take_rank(seed_deg, e < n_seed ? inv[(uint32_t)seed[e]] : 0u, e < n_seed, lane);
+        if (e < n_seed) seed_rank[e] = r;
+    }
 }
 
 // Rows in descending order of degree (perm: internal row -> vertex, inv: its
