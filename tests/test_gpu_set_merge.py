@@ -48,3 +48,20 @@ def test_every_tile_edge(provider):
     for shift in range(5):
         a = b[shift :: 5][:4999]
         _check(provider, a, b)
+
+
+@pytest.mark.parametrize("shared", ["none", "one", "first tile", "half", "all"])
+def test_shared_keys_of_many_tiles(provider, shared):
+    """Hundreds of tiles with shared keys in none, one or all of them."""
+    b = np.arange(0, 2_000_000, dtype=np.uint64) * np.uint64(4)
+    a = b[: 1_000_000] * np.uint64(2) + np.uint64(1)
+    if shared == "one":
+        a[500_000] += np.uint64(3)
+    elif shared == "first tile":
+        a[:10] = b[:20:2]
+    elif shared == "half":
+        a[::2] += np.uint64(3)
+    elif shared == "all":
+        a = b[: 1_000_000].copy()
+    assert len(np.intersect1d(a, b)) == {"none": 0, "one": 1, "first tile": 10, "half": 500_000, "all": 1_000_000}[shared]
+    _check(provider, np.unique(a), b)

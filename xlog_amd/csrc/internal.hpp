@@ -500,10 +500,10 @@ void merge_sorted(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *b, u
 void merge_sorted_dev(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *d_na, const uint64_t *b, uint64_t nb,
                       const uint64_t *d_nb, uint64_t *out, const uint64_t *skip, const uint32_t *stop,
                       unsigned long long *equal = nullptr);
-// The union of two sorted sets: their merge in out, and d_res[0] (device) the
-// number of keys they share.  When that is not zero the merge repeats those
-// keys, and uniq holds the d_res[1] unique ones (na + nb entries each);
-// otherwise the merge is the union and nothing is written to uniq.
+// The union of two sorted sets: their merge in out, and d_res[0] (device) not
+// zero when they share a key.  Then the merge repeats the shared keys, and uniq
+// holds the d_res[1] unique ones (na + nb entries each); otherwise the merge is
+// the union and nothing is written to uniq.
 void merge_unique_sorted(Ctx *ctx, const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb, uint64_t *out,
                          uint64_t *uniq, uint64_t *d_res);
 // The keys of the sorted set k that are not in the sorted set b, in order, by

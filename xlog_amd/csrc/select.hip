@@ -938,7 +938,8 @@ __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict_
     const uint64_t *sa = s, *sb = s + la;
     uint32_t td = tid * MRG_ITEMS;
     uint64_t r[MRG_ITEMS];
-    uint32_t cnt = 0, eq = 0;
+    uint32_t cnt = 0;
+    int eq = 0;
     if (td < len) {
         uint32_t ia = (uint32_t)merge_path(sa, la, sb, lb, td);
         uint32_t ib = td - ia;
@@ -948,14 +949,17 @@ __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict_
                 bool take_a = ib >= lb || (ia < la && sa[ia] <= sb[ib]);
                 r[j] = take_a ? sa[ia] : sb[ib];
                 // a key of b equal to one of a comes right after it
-                if (!take_a && (ia ? sa[ia - 1] == r[j] : (a0 && s_prev == r[j]))) ++eq;
+                eq |= !take_a && (ia ? sa[ia - 1] == r[j] : (a0 && s_prev == r[j])) ? 1 : 0;
                 ia += take_a; ib += !take_a;
                 ++cnt;
             }
         }
     }
-    if (equal && eq) atomicAdd(equal, (unsigned long long)eq);
-    __syncthreads();
+    // (one store, and only until another block's is seen: counts from every thread took as long as the merge and more,
+    // 4 * 10^6 keys against as many with half of them shared 255 us, 92 so)
+    if (__syncthreads_or(eq) && equal && tid == 0 &&
+        !__hip_atomic_load(equal, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        __hip_atomic_store(equal, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
     for (int j = 0; j < MRG_ITEMS; ++j)
         if ((uint32_t)j < cnt) s[td + j] = r[j];
