@@ -179,9 +179,10 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int lane) {
 // the bits that vary (the high word's varying bits above the low word's, so
 // that ids of a small domain fill the bins) with LDS atomics, and each key is
 // ranked in its bin by the whole key; equal keys are indistinguishable, so the
-// bins' order by arrival does not show.  Bins that are long on average
-// (BLOCK_SORT_BIN keys: hub ids) and sorts by a part of the key, which have to
-// be stable, take digit passes in LDS instead, over the digits that vary.
+// bins' order by arrival does not show.  Where a bin is long (more than
+// BLOCK_SORT_BIN keys: hub ids), and in sorts by a part of the key, which have to
+// be stable, digit passes in LDS run instead, over the digits that vary (9,500
+// pairs of Zipf ids whose longest bin has 700: ranked 146 us, by four digit passes 41).
 constexpr int BS_TB = 1024, BS_ITEMS = 16;
 constexpr uint32_t BLOCK_SORT_BIN = 64;
 static_assert(BS_TB * BS_ITEMS == BLOCK_SORT_KEYS, "keys of one workgroup");
@@ -250,22 +251,21 @@ __device__ __forceinline__ void block_sort(const uint64_t *in, uint32_t n, uint6
             slot[r] = (uint32_t)r < rounds && i < n ? atomicAdd(&sm.bin[bin_of(k[r])], 1u) : 0u;
         }
         __syncthreads();
-        uint32_t c[PER], tot = 0, sq = 0;
+        uint32_t c[PER], tot = 0, longest = 0;
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
             c[q] = sm.bin[tid * (PER) + q];
             tot += c[q];
-            sq += c[q] * c[q];  // (at most 2^28 over all bins)
+            longest = max(longest, c[q]);
         }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) sq += (uint32_t)__shfl_xor((int)sq, o, WAVE);
-        if (lane == 0) sm.part2[wave] = sq;
+        for (int o = 32; o > 0; o >>= 1) longest = max(longest, (uint32_t)__shfl_xor((int)longest, o, WAVE));
+        if (lane == 0) sm.part2[wave] = longest;
         uint32_t pre = block_scan(tot);  // (its barrier also publishes sm.part2)
-        uint32_t sum = 0;
-        for (int w = 0; w < WAVES; ++w) sum += sm.part2[w];
+        for (int w = 0; w < WAVES; ++w) longest = max(longest, sm.part2[w]);
         __syncthreads();
         const bool exact = nlo + nhi <= BIN_BITS;  // a bin's keys are equal: nothing to rank
-        sorted = exact || sum <= BLOCK_SORT_BIN * n;  // block-uniform
+        sorted = exact || longest <= BLOCK_SORT_BIN;  // block-uniform
         if (sorted) {
 #pragma unroll
             for (int q = 0; q < PER; ++q) {
