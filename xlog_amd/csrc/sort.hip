@@ -441,6 +441,7 @@ constexpr int BK_TB = 512, BK_ITEMS = 8, BK_KEYS = BK_TB * BK_ITEMS, BK_MAX_BITS
 constexpr uint32_t BK_SAMPLE = 8 << BK_MAX_BITS;
 struct BucketState {
     uint32_t over, pad;
+    uint32_t repeats, pad2;  // some value is two bounds or more
     uint32_t cursor[1 << BK_MAX_BITS], uniq[1 << BK_MAX_BITS];  // keys, unique keys of each bucket
     uint64_t bound[1 << BK_MAX_BITS];  // bucket b holds the keys x with bound[b - 1] <= x < bound[b]
 };
@@ -461,8 +462,14 @@ __global__ __launch_bounds__(BS_TB) void k_bucket_sample(const uint64_t *__restr
     __syncthreads();
     uint64_t k[BK_SAMPLE / BS_TB];
     block_sort<BS_TB, BK_SAMPLE / BS_TB>(sample, ns, ~0ull, false, sm, k);
-    for (uint32_t i = threadIdx.x; i < nb; i += BS_TB)
-        st->bound[i] = i + 1 < nb ? sm.key[(i + 1) * 8] : ~0ull;
+    int repeats = 0;
+    for (uint32_t i = threadIdx.x; i < nb; i += BS_TB) {
+        const uint64_t x = i + 1 < nb ? sm.key[(i + 1) * 8] : ~0ull;
+        st->bound[i] = x;
+        repeats |= i > 0 && sm.key[i * 8] == x ? 1 : 0;
+    }
+    repeats = __syncthreads_or(repeats);
+    if (threadIdx.x == 0) st->repeats = repeats ? 1u : 0u;
 }
 constexpr int BC_TB = 1024, BC_ITEMS = 8;  // a tile of 8,192 keys
 __global__ __launch_bounds__(BC_TB) void k_bucket_scatter(const uint64_t *__restrict__ in, uint64_t n, BucketState *st,
@@ -474,13 +481,12 @@ __global__ __launch_bounds__(BC_TB) void k_bucket_scatter(const uint64_t *__rest
     uint64_t k[BC_ITEMS];
 #pragma unroll
     for (int r = 0; r < BC_ITEMS; ++r) k[r] = base + r * BC_TB < n ? in[base + r * BC_TB] : 0ull;
-    int repeats = 0;  // some value is two bounds
+    const bool repeats = st->repeats != 0;
     for (int i = tid; i < nb; i += BC_TB) {
         s_cnt[i] = 0;
         s_bound[i] = st->bound[i];
-        repeats |= bucket_of_one(st->bound, i) ? 1 : 0;
     }
-    repeats = __syncthreads_or(repeats);
+    __syncthreads();
     // the number of bounds <= the key (the last bound is no bound: every search ends below it)
     uint32_t b[BC_ITEMS], rank[BC_ITEMS];
 #pragma unroll
@@ -551,8 +557,15 @@ __global__ __launch_bounds__(BK_TB) void k_bucket_sort(uint64_t *regions, Bucket
     const uint32_t t = blockIdx.x, n = st->cursor[t];
     uint64_t *region = regions + (uint64_t)t * BK_KEYS;
     uint64_t k[BK_ITEMS];
-    const bool one = bucket_of_one(st->bound, t);  // block-uniform
+    const bool repeats = st->repeats != 0, one = repeats && bucket_of_one(st->bound, t);  // block-uniform
     if (n && !one) block_sort<BK_TB, BK_ITEMS>(region, n, ~0ull, false, sm, k);
+    if (!UNIQUE && !repeats) {
+        uint32_t before = 0;
+        for (uint32_t i = tid; i < t; i += BK_TB) before += st->cursor[i];
+        before = bucket_block_total(before, sm.part);
+        for (uint32_t i = tid; i < n; i += BK_TB) out[before + i] = sm.key[i];
+        return;
+    }
     if (!UNIQUE) {
         // every bucket's place; values with more repeats than one workgroup should write are listed
         constexpr int PER = (1 << BK_MAX_BITS) / BK_TB;
