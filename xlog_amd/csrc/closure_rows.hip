@@ -271,7 +271,7 @@ __global__ __launch_bounds__(WAVE) void k_cr_walk(CrArgs a) {
     const bool mine = lane < CR_EDGES && e < a.m;
     const uint32_t src = e < a.m ? (uint32_t)(a.edge[e] >> 32) : 0u;
     const bool head = mine && (e == 0 || (uint32_t)(a.edge[e - 1] >> 32) != src);
-    if (__builtin_amdgcn_readfirstlane((int)cr_gave_up(a))) return;  // (the workgroup is one wave)
+    if (cr_gave_up(a)) return;  // (the workgroup is one wave, whose lanes read one word in one load)
     const uint64_t heads = __ballot(head);
     const int row = __popcll(heads & ((2ull << min(lane, CR_EDGES - 1)) - 1ull)) - 1;  // -1: an earlier batch's
     const uint32_t last_src = __shfl(src, CR_EDGES - 1, WAVE);

@@ -907,6 +907,7 @@ __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict_
                                                      MergeDev dv, unsigned long long *equal) {
     __shared__ uint64_t s[MRG_TILE];
     __shared__ uint64_t s_split[2], s_prev;
+    __shared__ int s_eq;
     const int tid = threadIdx.x;
     if (dv.off()) return;
     dv.counts(na, nb);
@@ -930,7 +931,10 @@ __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict_
     }
     const uint32_t la = (uint32_t)(a1 - a0), len = (uint32_t)(d1 - d0), lb = len - la;
     const uint64_t b0 = d0 - a0;
-    if (equal && tid == 0) s_prev = a0 ? a[a0 - 1] : 0ull;
+    if (equal && tid == 0) {
+        s_prev = a0 ? a[a0 - 1] : 0ull;
+        s_eq = 0;
+    }
     batched_copy<MRG_BLOCK, MRG_ITEMS>(
         len, tid, [&](uint32_t i) { return i < la ? a[a0 + i] : b[b0 + (i - la)]; },
         [&](uint32_t i, uint64_t v) { s[i] = v; });
@@ -955,10 +959,11 @@ __global__ __launch_bounds__(MRG_BLOCK) void k_merge(const uint64_t *__restrict_
             }
         }
     }
+    if (eq) s_eq = 1;
+    __syncthreads();
     // (one store, and only until another block's is seen: counts from every thread took as long as the merge and more,
     // 4 * 10^6 keys against as many with half of them shared 255 us, 92 so)
-    if (__syncthreads_or(eq) && equal && tid == 0 &&
-        !__hip_atomic_load(equal, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    if (equal && tid == 0 && s_eq && !__hip_atomic_load(equal, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
         __hip_atomic_store(equal, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
     for (int j = 0; j < MRG_ITEMS; ++j)
