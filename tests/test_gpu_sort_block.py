@@ -35,6 +35,21 @@ def test_sort_and_dedup(provider, kind):
         assert np.array_equal(provider.download_packed(R), k), n  # the input is left as it is
 
 
+@pytest.mark.parametrize("digits", [2, 3, 5, 8])
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+def test_longest_bin(provider, digits, extra):
+    """One bin (a value of the top 12 bits that vary) holds as many keys as are ranked, one fewer, one more; the low
+    word of the keys varies whole before the high word does."""
+    rng = np.random.default_rng(digits * 3 + extra)
+    below, long = 8 * digits - 12, 14 * digits + extra
+    top = np.concatenate([np.arange(4096), np.full(long - 1, 77)]).astype(np.uint64)
+    low = rng.integers(0, 1 << below, len(top), dtype=np.uint64)
+    k = rng.permutation((top << np.uint64(below)) | low)
+    R = provider.create_buffer_from_packed(k)
+    assert np.array_equal(provider.download_packed(provider.sort(R, [0, 1])), np.sort(k))
+    assert np.array_equal(provider.download_packed(provider.dedup_full_row(R)), np.unique(k))
+
+
 @pytest.mark.parametrize("kind", ["hashed", "dense", "hub", "few", "equal"])
 @pytest.mark.parametrize("n", [1, 65, 1025, 16384])
 def test_stable_by_column(provider, kind, n):

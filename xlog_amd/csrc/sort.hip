@@ -179,12 +179,15 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int lane) {
 // the bits that vary (the high word's varying bits above the low word's, so
 // that ids of a small domain fill the bins) with LDS atomics, and each key is
 // ranked in its bin by the whole key; equal keys are indistinguishable, so the
-// bins' order by arrival does not show.  Where a bin is long (more than
-// BLOCK_SORT_BIN keys: hub ids), and in sorts by a part of the key, which have to
-// be stable, digit passes in LDS run instead, over the digits that vary (9,500
-// pairs of Zipf ids whose longest bin has 700: ranked 146 us, by four digit passes 41).
+// bins' order by arrival does not show.  Where a bin is long (hub ids: more than
+// BLOCK_SORT_BIN keys for every digit that varies, since a thread reads a key's
+// whole bin and the passes cost by the digit), and in sorts by a part of the key,
+// which have to be stable, digit passes in LDS run instead, over the digits that
+// vary (9,500 pairs of Zipf ids whose longest bin has 700: ranked 146 us, by four
+// digit passes 41; 10^6 pairs of 300, whose bins are up to 100 keys of 8 digits:
+// by passes 112, ranked 85; 64 keys whatever the digits, or 20 for each, is slower).
 constexpr int BS_TB = 1024, BS_ITEMS = 16;
-constexpr uint32_t BLOCK_SORT_BIN = 64;
+constexpr uint32_t BLOCK_SORT_BIN = 14;
 static_assert(BS_TB * BS_ITEMS == BLOCK_SORT_KEYS, "keys of one workgroup");
 template <int TB, int ITEMS>
 struct BsSmem {
@@ -265,7 +268,9 @@ __device__ __forceinline__ void block_sort(const uint64_t *in, uint32_t n, uint6
         for (int w = 0; w < WAVES; ++w) longest = max(longest, sm.part2[w]);
         __syncthreads();
         const bool exact = nlo + nhi <= BIN_BITS;  // a bin's keys are equal: nothing to rank
-        sorted = exact || longest <= BLOCK_SORT_BIN;  // block-uniform
+        uint32_t digits = 0;
+        for (int dgt = 0; dgt < 8; ++dgt) digits += ((vary >> (8 * dgt)) & 255u) ? 1u : 0u;
+        sorted = exact || longest <= BLOCK_SORT_BIN * digits;  // block-uniform
         if (sorted) {
 #pragma unroll
             for (int q = 0; q < PER; ++q) {
